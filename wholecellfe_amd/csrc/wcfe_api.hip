@@ -2847,7 +2847,7 @@ void dense_solve_impl(wcfe_ctx *ctx, int n_sys, const int32_t *n, const double *
                             WorkList{plan.d_prefix + plan.solve_batched.fwd_off, plan.solve_batched.tot},
                             WorkList{plan.d_prefix + plan.solve_batched.bwd_off, plan.solve_batched.tot}, dK, dDinv,
                             dr, dx, dy, dsync, it > 0);
-    launch_dense_residual(s, dcp, dcs, dcells, n_sys, dA, dAoff, db, dx, dr);
+    launch_dense_residual(s, dcp, dcs, dcells, n_sys, max_npad, dA, dAoff, db, dx, dr);
     launch_cell_norm(s, dcp, dcs, dcells, n_sys, dr, 1, 1, ctx->opt.lin_rtol);
   }
   HIPCHECK(hipGetLastError());

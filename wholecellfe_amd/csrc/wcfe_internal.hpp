@@ -232,7 +232,8 @@ void launch_ref_force_fa_subs(hipStream_t s, int n_nodes, const int *ring_start,
                               const int *stris, const double *Sx, int law, double kint, int *hit_tri,
                               double *hit_val, int *n_hits, int *overflow);
 void launch_dense_residual(hipStream_t s, const CellParams *cp, const CellState *cs, const int *cells, int ncell,
-                           const double *A64, const long long *a_off, const double *b, const double *x, double *r);
+                           int max_ndof, const double *A64, const long long *a_off, const double *b, const double *x,
+                           double *r);
 
 // Host-side VTK frame writer (wcfe_vtk.hip): one cell or substrate, the
 // reference's file layout.  Positions and fa_u with 2 (z = 0) or 3 components
