@@ -1432,7 +1432,7 @@ void enqueue_lu(wcfe_ctx *ctx, hipStream_t s, const LuPlan &plan, const std::vec
       }
       case ST_PANEL: {
         PhaseScope ph(ctx, WCFE_PH_LU_PANEL);
-        launch_lu_panel_pp<T>(s, cp, cs, wl, g.k, K, ipiv, Dinv);
+        launch_lu_panel_pp<T>(s, cp, cs, wl, g.k, K, ipiv, Dinv, (plan.max_nblk - g.k) * NB);
         break;
       }
       case ST_SWP: {

@@ -108,7 +108,7 @@ template <class T>
 void launch_lu_diag_inv(hipStream_t s, const CellParams *cp, CellState *cs, const WorkList &wl, int k, T *K, T *Dinv);
 template <class T>
 void launch_lu_panel_pp(hipStream_t s, const CellParams *cp, CellState *cs, const WorkList &wl, int k, T *K,
-                        int *ipiv, T *Dinv);
+                        int *ipiv, T *Dinv, int rows);
 template <class T>
 void launch_lu_laswp(hipStream_t s, const CellParams *cp, const WorkList &wl, int k, T *K, const int *ipiv);
 template <class T>
