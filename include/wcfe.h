@@ -91,31 +91,28 @@ typedef struct wcfe_options {
   int32_t cg_max_iter;   /* PCG iteration cap per refinement sweep */
   int32_t lu_groups;     /* batched dense LU: cells split in this many groups factored on concurrent
                             streams (1..16; 0 = automatic: 1 when every dense band is narrow -- 2 when
-                            the batch has two-chain cells -- else 4) */
+                            the batch has cut cells (twist) -- else 4) */
   int32_t lu_depth;      /* static pivoting: block steps per delayed trailing update (1..8; 0 = automatic:
                             1 when every dense band is narrow, else 4) */
   int32_t band;          /* 1: dense cells under static pivoting are numbered to narrow their band
                             (reverse Cuthill-McKee) and factored inside it (fill stays in the band);
                             0: natural numbering, full matrix */
-  int32_t fused_step;    /* with one panel per round (lu_depth 1) in FP32, one launch per block step:
-                            trailing update, next diagonal inverse and its block solves together.
-                            1: per launch, L items (each inverts the diagonal block itself: shortest
-                            chain) while they are at most 2 per compute unit; else split panel
-                            items while those are (one item inverts and solves the first L block,
-                            the other L blocks are L items, one item takes the cell's trailing
-                            blocks); else one panel item per cell (one inverse, then every L
-                            block: least work) and one item for the trailing blocks;
-                            2: L items only; 3: panel items after the first step; 4: one
-                            launch for the whole factorization, each cell's block steps in
-                            order in one workgroup (no launch between two steps of a cell's
-                            chain); 5: as 1, split panel items wherever 1 takes panel items;
-                            0: separate launches */
-  int32_t twist;         /* with fused block steps and one-workgroup sweeps in FP32 (block bandwidths
-                            up to 4): cells whose chain of block steps is longer than the batch needs
-                            are factored as two chains at once (top down and bottom up, meeting in a
-                            middle window of bw blocks), about half the dependent block steps.
-                            1: when the batch's block steps are latency bound (at most 8 block
-                            products per compute unit and step); 2: always; 0: one chain per cell */
+  int32_t fused_step;    /* with one panel per round (lu_depth 1), one launch per level of the band LU's
+                            elimination: the pending updates, the pivots' inverses and their
+                            block columns together. 1: how a launch's work is dealt out in items
+                            (column blocks per inverse, updated blocks per item) by estimated
+                            time; 2: an item per column block and per updated block (shortest
+                            launch of few cells); 3: one item per pivot and per node (least
+                            work); 4: one launch for the whole factorization, each cell's items
+                            in order in one workgroup (FP32); 5: an item per column block, the
+                            first with the pivot's; 0: separate launches */
+  int32_t twist;         /* with fused block steps and one-workgroup sweeps (block bandwidths up to 8):
+                            a cell's band may be cut by separators of bw blocks into independent
+                            parts that are eliminated at the same time, the separators after
+                            them: fewer dependent block steps, more products per step. 1: as many
+                            cuts as the estimated time of the batch's launches asks for; 2: one
+                            cut in every cell longer than the batch needs (top down and bottom up
+                            at once, meeting in the middle); 0: none */
   int32_t pcg_lanes;     /* block-CSR PCG: lanes per block row in the SpMV, 4, 8 or 16 (0: 4); a
                             workgroup of 1024 threads per chunk of 256 block rows */
 } wcfe_options;
@@ -258,12 +255,13 @@ int wcfe_synchronize(wcfe_ctx *ctx);
  * the fused block step, with split panel items (fused_step 5) and (mixed
  * precision, one group) the whole factorization in one launch (fused_step
  * 4); then, with fused block steps,
- * one chain per cell against two-chain cells (twist 0 / 2); WCFE_TUNE_PCG
+ * uncut cells against one cut per longer cell (twist 0 / 2); WCFE_TUNE_PCG
  * (batches with block-CSR cells): lanes per block row of the PCG's SpMV
  * (pcg_lanes 4, 8, 16).  Every trial starts from the state the cells were
  * added with, and so does the batch afterwards: call it after wcfe_finalize
  * and before any Newton step.  chosen (optional, 6 entries): lu_depth,
- * lu_groups, dense_max_dof, fused_step, the number of two-chain cells and
+ * lu_groups, dense_max_dof, fused_step, the number of cut cells
+ * (wcfe_get_cell_layout) and
  * pcg_lanes in effect; ms_best (optional): ms per step. */
 #define WCFE_TUNE_SOLVER 1
 #define WCFE_TUNE_LU 2
@@ -348,8 +346,10 @@ int wcfe_get_cell_sizes(wcfe_ctx *ctx, int32_t cell, int32_t *n_nodes, int32_t *
 /* How a cell is solved after wcfe_finalize: solver (WCFE_SOLVER_DENSE or
  * WCFE_SOLVER_CSR), 64-row blocks of its dense system, their block bandwidth
  * in the band numbering (nblk - 1: full matrix), symmetric factorization, and
- * for a two-chain factorization (wcfe_options.twist) the top blocks of chain
- * A and the bottom blocks of chain B (0, 0: one chain). */
+ * for a cut cell (wcfe_options.twist) longer than the batch's shortest chain
+ * of halved cells the blocks of its two halves around a separator in the
+ * middle (0, 0: uncut, or cut although a shorter cell; deeper cuts are not
+ * reported). */
 int wcfe_get_cell_layout(wcfe_ctx *ctx, int32_t cell, int32_t *solver, int32_t *nblk, int32_t *bw, int32_t *sym,
                          int32_t *chain_top, int32_t *chain_bottom);
 int wcfe_get_cell_info(wcfe_ctx *ctx, int32_t cell, double *time, int32_t *step, int32_t *newton_iter,

@@ -16,53 +16,55 @@ template <class T> struct Vec16;
 template <> struct Vec16<float> { typedef float4 type; static constexpr int n = 4; };
 template <> struct Vec16<double> { typedef double2 type; static constexpr int n = 2; };
 
+// lower_only: symmetric cells get the blocks (i, j) with j eliminated no later
+// than i (rank) only: the band LU writes the others, U = L^T, before anything
+// reads them
 template <class T>
-// lower_only: symmetric cells get the blocks up to the diagonal only (the
-// fused band LU writes every upper band block, U = L^T, before anything
-// reads it); a symmetric two-chain cell's bottom chain factors the block
-// reversal, whose lower blocks are the real upper ones: block rows of the
-// bottom part get the blocks from the diagonal on, the middle window's rows
-// the whole envelope
 __global__ __launch_bounds__(256) void k_fill_systems(const CellParams *cp, const int *cells, int ncell, T *K,
-                                                      int lower_only) {
+                                                      const int *rank, int lower_only) {
   const int ci = blockIdx.y;
   if (ci >= ncell) return;
   const CellParams p = cp[cells[ci]];
   typedef typename Vec16<T>::type V;
   constexpr int VN = Vec16<T>::n;
-  // blocks within the fill envelope |i - j| <= env only; one wave per row
-  // (a row holds at most (2 env + 1) * 64 / VN vectors)
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  for (int r = 4 * blockIdx.x + wave; r < p.npad; r += 4 * gridDim.x) {
-    const int rb = r / NB;
-    const bool lo = lower_only && p.sym;
-    const bool bottom = lo && p.tw_m > 0 && rb >= p.tw_m + p.bw, top = lo && (p.tw_m == 0 || rb < p.tw_m);
-    const int c0 = (bottom ? rb : max(0, rb - p.env)) * (NB / VN),
-              c1 = min(p.nblk, rb + 1 + (top ? 0 : p.env)) * (NB / VN);
-    V *row = reinterpret_cast<V *>(K + p.k_off + (long long)r * p.npad);
-    for (int c = c0 + lane; c < c1; c += 64) {
+  // blocks within the fill envelope |i - j| <= env only; a wave takes whole
+  // 64-entry row segments, 64 * VN / 64 rows of a block at a time
+  constexpr int LPR = 64 / VN;       // lanes per row segment
+  constexpr int RPW = 64 / LPR;      // rows per wave
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane / LPR, lc = (lane % LPR) * VN;
+  const bool lo = lower_only && p.sym;
+  const int *rk = rank + p.rank_off;
+  for (int r0 = RPW * (4 * (int)blockIdx.x + wave); r0 < p.npad; r0 += RPW * 4 * (int)gridDim.x) {
+    const int rb = r0 / NB, r = r0 + lr;
+    const int mine = lo ? rk[rb] : 0;
+    T *row = K + p.k_off + (long long)r * p.npad;
+    for (int jb = max(0, rb - p.env); jb <= min(p.nblk - 1, rb + p.env); ++jb) {
+      if (lo && rk[jb] > mine) continue;
       T vals[VN];
 #pragma unroll
-      for (int k = 0; k < VN; ++k) vals[k] = (r >= p.ndof && r == c * VN + k) ? T(1) : T(0);
+      for (int k = 0; k < VN; ++k) vals[k] = (r >= p.ndof && r == jb * NB + lc + k) ? T(1) : T(0);
       V w;
       memcpy(&w, vals, sizeof(V));
-      row[c] = w;
+      *reinterpret_cast<V *>(row + jb * NB + lc) = w;
     }
   }
 }
 
 template <class T>
 void launch_fill_systems(hipStream_t s, const CellParams *cp, const int *cells, int ncell, int max_npad, T *K,
-                         int lower_only) {
+                         const int *rank, int lower_only) {
   if (ncell <= 0) return;
-  // 4 rows per block and pass; at most 128 blocks per cell (the largest
-  // cells loop) so that small cells launch few empty blocks
-  int gx = (max_npad + 3) / 4 < 128 ? (max_npad + 3) / 4 : 128;
+  // 16 (FP64: 8) rows per workgroup and pass; at most 64 workgroups per cell
+  // (the largest cells loop) so that small cells launch few empty ones
+  const int rows = 4 * Vec16<T>::n;
+  int gx = (max_npad + rows - 1) / rows < 64 ? (max_npad + rows - 1) / rows : 64;
   if (gx < 1) gx = 1;
-  hipLaunchKernelGGL(k_fill_systems<T>, dim3(gx, ncell), dim3(256), 0, s, cp, cells, ncell, K, lower_only);
+  hipLaunchKernelGGL(k_fill_systems<T>, dim3(gx, ncell), dim3(256), 0, s, cp, cells, ncell, K, rank, lower_only);
 }
-template void launch_fill_systems<float>(hipStream_t, const CellParams *, const int *, int, int, float *, int);
-template void launch_fill_systems<double>(hipStream_t, const CellParams *, const int *, int, int, double *, int);
+template void launch_fill_systems<float>(hipStream_t, const CellParams *, const int *, int, int, float *, const int *,
+                                         int);
+template void launch_fill_systems<double>(hipStream_t, const CellParams *, const int *, int, int, double *,
+                                          const int *, int);
 
 __global__ __launch_bounds__(256) void k_fill(double *p, long long n, double value) {
   for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
@@ -236,12 +238,11 @@ __global__ __launch_bounds__(256) void k_group_gather(View v, const int *node_ce
     G[2 * n + 1] = g1;
   }
   const CellParams &p = v.cp[node_cell[n]];
-  // lower_only: a symmetric cell's blocks above the diagonal block are
-  // written by the fused band LU (U = L^T) before any read; a two-chain
-  // cell's blocks that involve its bottom part: those below the diagonal
+  // lower_only: a symmetric cell's blocks whose column is eliminated after
+  // their row are written by the fused band LU (U = L^T) before any read
   if (lower_only && p.sym && !p.csr) {
-    const int bi = v.kpos[n] >> 5, bj = v.kpos[gp.col[g]] >> 5;
-    if (p.tw_m > 0 && max(bi, bj) >= p.tw_m + p.bw ? bi > bj : bi < bj) return;
+    const int *rk = v.rank + p.rank_off;
+    if (rk[v.kpos[n] >> 5] < rk[v.kpos[gp.col[g]] >> 5]) return;
   }
   T *b0, *b1;
   if (p.csr) {

@@ -11,6 +11,7 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <string>
 #include <thread>
 #include <vector>
@@ -312,37 +313,11 @@ struct LuPlan {
       case ST_GEMM1: return k < nb ? tiles(p, m) : 0;
       case ST_GEMM: return nb - k - np >= 1 ? tiles(p, std::min(nb - k - np, p.bw)) : 0;
       case ST_PANEL: return k < nb ? 1 : 0;
-      case ST_STEP:  // fused block step k (k = -1 .. chain_steps - 2), see k_lu_step; np: the form
-        return cell_step_items(p, k, step_flag(np));
-      case ST_CELL: return nb > 0 ? 1 : 0;  // the whole factorization, one workgroup
       default: return (k < nb && m > 0) ? (m * NB + 255) / 256 : 0;
     }
   }
-  // a block step's form (Stage::np): 1 L items, 2 panel items, 3 split
-  // panel items; the kernel's panel argument: 0, 1, 2
-  static int step_flag(int np) { return np == 2 ? 1 : np == 3 ? 2 : 0; }
-  static long long chain_products(const Chain &v, int k) {
-    const int s0 = k + 1;
-    if (s0 >= v.nblk || s0 > v.elim) return 0;
-    if (s0 == v.elim) return std::max(0, chain_items(v, k, 0) - 1);  // update-only: one product per block
-    const int w = std::min(v.nblk - s0 - 1, v.bw);
-    const long long npl = k >= 0 ? std::max(0, std::min(v.nblk - 1, k + v.bw) - s0) : 0;
-    const long long upd =
-        k >= 0 ? 1 + (v.sym ? 1 : 2) * std::min(w, v.bw - 1) + (v.sym ? npl * (npl + 1) / 2 : npl * npl) : 0;
-    return upd + w + 1;
-  }
   static long long block_products(const CellParams &p, int kind, int k, int np, int pivoting) {
     if (kind == ST_STRIP || kind == ST_GEMM || kind == ST_GEMM1) return (long long)np * items(p, kind, k, np, pivoting);
-    if (kind == ST_STEP) {  // useful 64^3 products: updated blocks, L block solves, the inverse
-      long long tot = chain_products(chain_of(p, 0), k);
-      if (p.tw_m > 0) tot += chain_products(chain_of(p, 1), k);
-      return tot;
-    }
-    if (kind == ST_CELL) {  // every block step: the first in the L-item form, the others in the panel form
-      long long tot = 0;
-      for (int kk = -1; kk < chain_steps(p) - 1; ++kk) tot += block_products(p, ST_STEP, kk, kk >= 0 ? 2 : 1, pivoting);
-      return tot;
-    }
     return 0;
   }
   // static pivoting: LU_DEPTH block steps per round -- panel k, then the
@@ -354,15 +329,11 @@ struct LuPlan {
   // update depth): the trailing matrix is read and written once per `depth`
   // block steps
   int depth = 4;
-  bool fused = false;      // static pivoting, depth 1: one fused launch per block step
-  bool cell_loop = false;  // ... or one launch for every step, one workgroup per cell
+  bool fused = false;      // static pivoting, depth 1: one fused launch per level of the band plans
+  bool cell_loop = false;  // ... or one launch for every level, one workgroup per cell
   std::vector<std::array<int, 3>> schedule(int nblk, int pivoting) const {
     std::vector<std::array<int, 3>> s;
-    if (!pivoting && cell_loop) {
-      if (nblk > 0) s.push_back({ST_CELL, -1, 0});
-    } else if (!pivoting && fused) {
-      for (int k = -1; k < nblk - 1; ++k) s.push_back({ST_STEP, k, 1});
-    } else if (!pivoting) {
+    if (!pivoting) {
       s.push_back({ST_DIAG, 0, 0});
       for (int k = 0; k < nblk; k += depth) {
         const int R = std::min(depth, nblk - k);
@@ -384,90 +355,219 @@ struct LuPlan {
     return s;
   }
 
-  // Fused block step lists: k_lu_step hands item i of a launch to XCD
-  // chunk xcd_item^-1(i) (eight contiguous chunks, dispatched in order within
-  // each); inside every chunk the diagonal and L items (the inverse on their
-  // critical path) go first and the trailing tiles fill in after them.
-  static void step_heavy_first(std::vector<int> &buf, const std::vector<CellParams> &cp, const Stage &g) {
-    if (g.kind != ST_STEP) return;
-    const int q = g.tot >> 3, r = g.tot & 7;
-    for (int x = 0; x < 8; ++x) {
-      const int b0 = g.off + x * q + std::min(x, r), nx = q + (x < r ? 1 : 0);
-      std::stable_partition(buf.begin() + b0, buf.begin() + b0 + nx, [&](int v) {
-        const CellParams &p = cp[v >> 20];
-        int t = v & 0xFFFFF;
-        Chain ch = chain_of(p, 0);
-        if (p.tw_m > 0) {
-          const int na = chain_items(ch, g.k, step_flag(g.np));
-          if (t >= na) {
-            ch = chain_of(p, 1);
-            t -= na;
-          }
-        }
-        if (g.k + 1 >= ch.elim) return false;  // update-only items
-        const int wl = std::min(ch.nblk - g.k - 2, ch.bw);
-        return t <= (g.np == 2 ? 0 : g.np == 3 ? std::max(wl - 1, 0) : wl);
-      });
+  // a fused schedule's items (device), one contiguous range per stage
+  StepItem *d_items = nullptr;
+  int *d_solve = nullptr;  // solve_batched / solve_single of a fused schedule with the spread-out solve
+  int2 *d_ranges = nullptr;  // ST_CELL: each cell's items
+
+  // Fused block steps: one launch per level of the cells' plans.  How a
+  // level's work is dealt out in items (k_band.hip): `cols` column blocks of a
+  // pivot per item, each item inverting the pivot itself (apart: the pivot's
+  // own item, which stores the inverse, takes none), and `tiles` updated
+  // blocks of a node per item, the node's last one with its forward
+  // operations (apart: these too in an item of their own).  Every dealing runs
+  // the same products in the same order.
+  struct Deal {
+    int cols, tiles, apart;
+  };
+  static constexpr int ALL = 1 << 20;
+  static int ceil_div(int a, int b) { return (a + b - 1) / b; }
+  template <class I, class R> static void deal_level(const BandPlan::Level &L, const Deal &d, I inv, R rest) {
+    for (const BandPlan::Pivot &v : L.piv) {
+      if (d.apart) inv(v, 0, 0, true);
+      if (!d.apart && v.nref == 0) inv(v, 0, 0, true);
+      for (int r = 0; r < v.nref; r += d.cols) inv(v, r, std::min(d.cols, v.nref - r), !d.apart && r == 0);
+    }
+    for (const BandPlan::Group &g : L.grp) {
+      int r = 0;
+      const int n = d.apart ? ceil_div(g.nref, d.tiles) : std::max(1, ceil_div(g.nref, d.tiles));
+      for (int i = 0; i < n; ++i) {
+        const int t = ceil_div(g.nref - r, n - i);
+        const bool fwd = !d.apart && i + 1 == n;
+        rest(g.ref0 + r, t, g.fop0, fwd ? g.nfop : 0);
+        r += t;
+      }
+      if (d.apart && g.nfop) rest(g.ref0, 0, g.fop0, g.nfop);
     }
   }
+  // Estimated time of a level dealt out in a way (us): the longest item, or
+  // the items' time over the workgroups that run at once.  An item's time as
+  // measured on an MI355X with few items in a launch: FP32 12 with one column
+  // block, 3.5 for each further one, 2.5 + 2.5 per updated block; FP64 twice.
+  struct Load {
+    double total = 0.0, longest = 0.0;
+    void add(double n, double t) {
+      total += n * t;
+      longest = std::max(longest, t);
+    }
+  };
+  static double inv_time(int cols, int f64) { return (cols ? 12.0 + 3.5 * (cols - 1) : 10.5) * (f64 ? 2.0 : 1.0); }
+  static double tile_time(int tiles, int f64) { return (2.5 + 2.5 * tiles) * (f64 ? 2.0 : 1.0); }
+  static void level_load(const BandPlan::Level &L, const Deal &d, int f64, double n, Load &w) {
+    deal_level(L, d, [&](const BandPlan::Pivot &, int, int c, bool) { w.add(n, inv_time(c, f64)); },
+               [&](int, int t, int, int) { w.add(n, tile_time(t, f64)); });
+  }
+  static double load_time(const Load &w, double slots) { return 1.5 + std::max(w.longest, w.total / slots); }
+  // fuse (the fused_step option): 1 the fastest by the estimate; 2 an item
+  // per column block and updated block; 3 one item per pivot and node; 5 an
+  // item per column block, the pivot's with the first
+  static std::vector<Deal> deals(int fuse) {
+    if (fuse == 2) return {Deal{1, 1, 1}};
+    if (fuse == 3 || fuse == 4) return {Deal{ALL, ALL, 0}};
+    if (fuse == 5) return {Deal{1, 4, 0}};
+    std::vector<Deal> d{Deal{1, 1, 1}};
+    for (int c : {1, 2, 3, 4, 6, ALL})
+      for (int t : {1, 2, 4, 8}) d.push_back(Deal{c, t, 0});
+    return d;
+  }
+  static Deal choose_deal(const std::vector<std::pair<const BandPlan::Level *, double>> &levels, int fuse, int f64,
+                          double slots, double *time = nullptr) {
+    Deal best{1, 1, 1};
+    double bt = 1e300;
+    for (const Deal &d : deals(fuse)) {
+      Load w;
+      for (const auto &l : levels) level_load(*l.first, d, f64, l.second, w);
+      const double t = load_time(w, slots);
+      if (t < bt) {
+        bt = t;
+        best = d;
+      }
+    }
+    if (time) *time = bt;
+    return best;
+  }
+  // One level of the listed cells as a stage.  k_lu_step hands item i to XCD
+  // chunk xcd_item^-1(i) (eight contiguous chunks, dispatched in order within
+  // each): inside every chunk the longest items go first and the others fill
+  // in after them.
+  static Stage step_stage(std::vector<StepItem> &buf, const std::vector<int> &cells,
+                          const std::vector<const BandPlan *> &plans, const std::vector<int2> &base, int level,
+                          int fuse, int f64, double slots) {
+    Stage g{ST_STEP, level, 1, (int)buf.size(), 0, 0};
+    std::map<const BandPlan::Level *, double> count;
+    for (int c : cells) {
+      if (level >= (int)plans[c]->lev.size()) continue;
+      count[&plans[c]->lev[level]] += 1.0;
+      g.work += plans[c]->lev[level].products;
+    }
+    const Deal d = choose_deal({count.begin(), count.end()}, fuse, f64, slots);
+    std::vector<std::pair<int, StepItem>> seq;  // (cost, item)
+    for (int c : cells)
+      if (level < (int)plans[c]->lev.size()) add_items(seq, c, plans[c]->lev[level], base[c].x, base[c].y, d);
+    g.tot = (int)seq.size();
+    const int q = g.tot >> 3, r = g.tot & 7;
+    for (int x = 0, b0 = 0; x < 8; ++x) {
+      const int nx = q + (x < r ? 1 : 0);
+      std::stable_sort(seq.begin() + b0, seq.begin() + b0 + nx,
+                       [](const std::pair<int, StepItem> &a, const std::pair<int, StepItem> &b) { return a.first > b.first; });
+      b0 += nx;
+    }
+    for (const auto &i : seq) buf.push_back(i.second);
+    return g;
+  }
+  static void add_items(std::vector<std::pair<int, StepItem>> &seq, int c, const BandPlan::Level &L, int rbase,
+                        int fbase, const Deal &d) {
+    deal_level(L, d,
+               [&](const BandPlan::Pivot &v, int r, int n, bool store) {
+                 seq.push_back({(int)(10 * inv_time(n, 0)), StepItem{c, STEP_INV | (store ? STEP_STORE : 0), v.s, v.p,
+                                                                     rbase + v.ref0 + r, n, 0, 0}});
+               },
+               [&](int r, int n, int f, int nf) {
+                 seq.push_back({(int)(10 * tile_time(n, 0)), StepItem{c, 0, 0, -1, rbase + r, n, fbase + f, nf}});
+               });
+  }
+  // fuse 4: the whole factorization in one launch (k_lu_cell), every cell's
+  // items in level order in one workgroup, longest cells first
+  void build_fused(const std::vector<CellParams> &cp, const std::vector<const BandPlan *> &plans,
+                   const std::vector<int2> &base, int groups, int fuse, int f64, double slots, bool per_cell) {
+    pivoting = 0;
+    depth = 1;
+    fused = true;
+    cell_loop = fuse == 4;
+    const int n = (int)cp.size();
+    std::vector<int> order(n);
+    for (int c = 0; c < n; ++c) order[c] = c;
+    std::vector<StepItem> buf;
+    std::vector<int> cells_buf;
+    std::vector<int2> ranges;
+    auto stages = [&](const std::vector<int> &cells) {
+      std::vector<Stage> st;
+      int levels = 0;
+      for (int c : cells) levels = std::max(levels, (int)plans[c]->lev.size());
+      if (cell_loop) {
+        Stage g{ST_CELL, 0, 0, (int)ranges.size(), 0, 0};
+        std::vector<int> by_len(cells);
+        std::stable_sort(by_len.begin(), by_len.end(),
+                         [&](int a, int b) { return plans[a]->lev.size() > plans[b]->lev.size(); });
+        for (int c : by_len) {
+          if (plans[c]->lev.empty()) continue;
+          std::vector<std::pair<int, StepItem>> seq;
+          const int i0 = (int)buf.size();
+          for (const BandPlan::Level &L : plans[c]->lev) {
+            add_items(seq, c, L, base[c].x, base[c].y, deals(4)[0]);
+            g.work += L.products;
+          }
+          for (const auto &i : seq) buf.push_back(i.second);
+          ranges.push_back(make_int2(i0, (int)buf.size()));
+          ++g.tot;
+        }
+        if (g.tot > 0) st.push_back(g);
+        return st;
+      }
+      for (int l = 0; l < levels; ++l) {
+        const Stage g = step_stage(buf, cells, plans, base, l, fuse, f64, slots);
+        if (g.tot > 0) st.push_back(g);
+      }
+      return st;
+    };
+    batched = stages(order);
+    single.assign(n, {});
+    if (per_cell)
+      for (int c = 0; c < n; ++c) single[c] = stages({c});
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cp[a].nblk > cp[b].nblk; });
+    grp.clear();
+    grp_cells_off.clear();
+    grp_ncell.clear();
+    const int G = std::min(std::max(groups, 1), n);
+    for (int g = 0; G > 1 && g < G; ++g) {
+      std::vector<int> mine;
+      for (int q = g; q < n; q += G) mine.push_back(order[q]);
+      grp.push_back(stages(mine));
+      grp_cells_off.push_back((int)cells_buf.size());
+      grp_ncell.push_back((int)mine.size());
+      cells_buf.insert(cells_buf.end(), mine.begin(), mine.end());
+    }
+    d_prefix = dupload(cells_buf);
+    d_items = dupload(buf);
+    d_ranges = dupload(ranges);
+  }
 
-  // fused block steps (fuse = the fused_step option): 1 per launch, L items
-  // while they are at most panel_min, else split panel items while those
-  // are, else panel items (one inverse per cell: the least work); 2 L items
-  // only; 3 panel items after the first step; 4 one launch for the whole
-  // factorization (k_lu_cell: every cell's steps in one workgroup, largest
-  // cells first); 5 split panel items (the first L block with the inverse,
-  // the others as L items) in every launch with more than panel_min L items,
-  // L items in the others
-  void build(const std::vector<CellParams> &cp, int piv, int groups, int lu_depth, int fuse = 0, int panel_min = 512) {
+  void build(const std::vector<CellParams> &cp, int piv, int groups, int lu_depth) {
     if (lu_depth < 1 || groups < 1) throw ApiError{WCFE_ERR_ARG, "LU schedule needs depth and groups >= 1"};
     pivoting = piv;
     depth = lu_depth;
-    fused = fuse && !piv && lu_depth == 1;
-    cell_loop = fused && fuse == 4;
-    // the step's form: L items (np 1), one panel item per cell (np 2) or
-    // split panel items (np 3)
-    auto step_form = [&](const std::vector<int> &cells, std::array<int, 3> &st) {
-      if (st[0] != ST_STEP || st[1] < 0 || fuse == 2) return;
-      if (fuse == 3) {
-        st[2] = 2;
-        return;
-      }
-      long long tot = 0, split = 0;
-      for (int c : cells) {
-        tot += items(cp[c], ST_STEP, st[1], 1, pivoting);
-        split += items(cp[c], ST_STEP, st[1], 3, pivoting);
-      }
-      if (tot > panel_min) st[2] = (fuse == 5 || split <= panel_min) ? 3 : 2;
-    };
     std::vector<int> all((size_t)cp.size());
     for (size_t c = 0; c < cp.size(); ++c) all[c] = (int)c;
     const int n = (int)cp.size();
     std::vector<int> buf;
     max_nblk = 0;
-    for (auto &p : cp) max_nblk = std::max(max_nblk, chain_steps(p));
+    for (auto &p : cp) max_nblk = std::max(max_nblk, p.nblk);
     if (n >= (1 << 11)) throw ApiError{WCFE_ERR_ARG, "at most 2047 systems per batch"};
     batched.clear();
-    std::vector<int> by_size(all);  // the cell launch takes the longest chains first
-    std::stable_sort(by_size.begin(), by_size.end(),
-                     [&](int a, int b) { return chain_steps(cp[a]) > chain_steps(cp[b]); });
     for (auto st : schedule(max_nblk, pivoting)) {
-      step_form(all, st);
       Stage g{st[0], st[1], st[2], (int)buf.size(), 0, 0};
-      for (int c : (st[0] == ST_CELL ? by_size : all)) {
+      for (int c : all) {
         const long long t = items(cp[c], st[0], st[1], st[2], pivoting);
         if (t >= (1 << 20)) throw ApiError{WCFE_ERR_ARG, "too many LU work items per cell"};
         for (int i = 0; i < t; ++i) buf.push_back((c << 20) | i);
         g.tot += (int)t;
         g.work += block_products(cp[c], st[0], st[1], st[2], pivoting);
       }
-      step_heavy_first(buf, cp, g);
       if (g.tot > 0) batched.push_back(g);
     }
     single.assign(n, {});
     for (int c = 0; c < n; ++c)
-      for (auto st : schedule(chain_steps(cp[c]), pivoting)) {
-        step_form({c}, st);
+      for (auto st : schedule(cp[c].nblk, pivoting)) {
         const long long t = items(cp[c], st[0], st[1], st[2], pivoting);
         if (t == 0) continue;
         if (t >= (1 << 20)) throw ApiError{WCFE_ERR_ARG, "too many LU work items per cell"};
@@ -503,10 +603,9 @@ struct LuPlan {
         std::vector<int> mine;
         for (int q = g; q < n; q += G) mine.push_back(order[q]);
         int gmax = 0;
-        for (int c : mine) gmax = std::max(gmax, chain_steps(cp[c]));
+        for (int c : mine) gmax = std::max(gmax, cp[c].nblk);
         std::vector<Stage> st;
         for (auto sk : schedule(gmax, pivoting)) {
-          step_form(mine, sk);
           Stage gs{sk[0], sk[1], sk[2], (int)buf.size(), 0, 0};
           for (int c : mine) {
             const long long t = items(cp[c], sk[0], sk[1], sk[2], pivoting);
@@ -514,7 +613,6 @@ struct LuPlan {
             gs.tot += (int)t;
             gs.work += block_products(cp[c], sk[0], sk[1], sk[2], pivoting);
           }
-          step_heavy_first(buf, cp, gs);
           if (gs.tot > 0) st.push_back(gs);
         }
         grp.push_back(st);
@@ -595,9 +693,32 @@ struct Batch {
   // the first solve's forward sweep, run inside the fused block steps: per
   // band row its batch dof (-1: padding) and the forward result
   int *kinv = nullptr;
-  float *yfwd = nullptr;
-  // batches with two-chain cells: the sweeps' forward result (sys elements)
-  void *ysw = nullptr;
+  void *yfwd = nullptr;
+  // the sweeps' vector (sys elements) and the plans' slots
+  void *ysw = nullptr, *slots = nullptr;
+  // band plans of the dense cells (one per distinct size, shared), their
+  // tables on the device and the sweeps' workgroups: the leaves forward, the
+  // separators (all of it, or backward only), the leaves backward; a batch
+  // without separators runs its whole sweeps in one launch
+  std::vector<std::shared_ptr<BandPlan>> plans;
+  std::vector<int> chain_top, chain_bottom;  // reported layout (wcfe_get_cell_layout)
+  int nslot = 0;
+  int *rank = nullptr;
+  BlockRef *refs = nullptr;
+  FwdOp *fops = nullptr;
+  SweepOp *sops = nullptr;
+  SweepLoc *slocs = nullptr;
+  int *saccs = nullptr;
+  SweepWG *swg = nullptr;
+  struct SweepList {
+    int off = 0, n = 0, max_loc = 0;
+  };
+  struct SweepLists {
+    SweepList fwd, top, top_bwd, bwd, whole;
+    bool split = false;
+  };
+  SweepLists sweeps;                    // every cell
+  std::vector<SweepLists> sweeps_cell;  // one cell's (per-cell Newton steps)
   std::vector<std::vector<int>> kpos_h;
   double *rp = nullptr, *dp = nullptr;
   bool solve_wg = false;  // static pivoting: one workgroup per cell walks its band (narrow bands)
@@ -618,7 +739,7 @@ struct Batch {
     void *ptrs[] = {X, x, fau, ea, cC, el_tri, el_cell, el_spr, sp_bary, sp_anchor, sp_state, sp_cell, sp_elem,
                     sp_local, cp, cs, node_cell, adj_start, adj, Ge, g_start, g_col, g_bpos, g_cstart, g_ke, g_node, Ke64, G, r, delta, Rea, MM, K, Dinv, ysol, sync, ipiv, cells,
                     replica, transitions, plan.d_prefix, row_ptr, bcol, diag_pos, el_bpos, csr_cells, chunks, Kb,
-                    cgvec, cg, partials, norm_part, norm_cnt, kpos, kinv, yfwd, ysw, rp, dp, bt_bidx, bt_node, bt_cst, crange, bt_cand, bt_frame, bt_g, bt_J, bt_area,
+                    cgvec, cg, partials, norm_part, norm_cnt, kpos, kinv, yfwd, ysw, slots, rank, refs, fops, sops, slocs, saccs, swg, plan.d_items, plan.d_ranges, plan.d_solve, rp, dp, bt_bidx, bt_node, bt_cst, crange, bt_cand, bt_frame, bt_g, bt_J, bt_area,
                     bt_gd, bt_fext};
     for (void *p : ptrs)
       if (p) (void)hipFree(p);
@@ -755,6 +876,7 @@ View make_view(const wcfe_ctx *ctx, const Batch &b) {
   View v;
   v.X = b.X; v.x = b.x; v.ea = b.ea; v.cC = b.cC; v.fau = b.fau;
   v.el_tri = b.el_tri; v.el_cell = b.el_cell; v.el_spr = b.el_spr; v.el_bpos = b.el_bpos; v.kpos = b.kpos;
+  v.rank = b.rank;
   v.sp_bary = b.sp_bary; v.sp_anchor = b.sp_anchor; v.sp_state = b.sp_state;
   v.cp = b.cp; v.cs = b.cs;
   v.tab_px = ctx->tab_px; v.tab_py = ctx->tab_py; v.tab_k = ctx->tab_k;
@@ -780,6 +902,244 @@ template <class F> void parallel_cells(int ncell, F f) {
       for (int c = next++; c < ncell; c = next++) f(c);
     });
   for (auto &th : pool) th.join();
+}
+
+// Workgroups of a block step that make headway at once: two FP32 ones fit a
+// compute unit but each then takes about twice as long (a launch of 322 items
+// over 256 compute units 24 us, of 850 about 60; alone an item takes 12), and
+// one FP64.
+double step_slots(const wcfe_ctx *ctx, int elem_size) { return (elem_size == 4 ? 1.0 : 0.75) * ctx->n_cu; }
+
+// Which cells' bands are cut, and how deep (band_plan.hpp).  A cut halves a
+// cell's chain of dependent block steps and adds the fill of the separators:
+// about twice the products of that cell.  A batch takes as many launches as
+// its longest cell has levels, so the choice is one number, the batch's
+// levels C: each cell is cut as little as reaches C, and C is the one with
+// the least estimated time: the launches' (LuPlan::choose_deal) and the
+// sweeps' longest stream.
+// twist 0: no cuts; 2: at most one cut per cell, of every cell longer than
+// the batch's shortest chain of half-length cells.
+constexpr int MAX_CUTS = 5;
+void plan_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
+  b.plans.assign(b.ncell, nullptr);
+  b.chain_top.assign(b.ncell, 0);
+  b.chain_bottom.assign(b.ncell, 0);
+  // products of the block steps without cuts: wide matrices keep the
+  // separate launches (their plans would list every block product)
+  double refs = 0.0;
+  for (const CellParams &p : b.cp_h)
+    if (!p.csr) refs += (double)p.nblk * p.bw * p.bw;
+  const bool fused = ctx->opt.fused_step > 0 && ctx->opt.pivoting == WCFE_PIVOT_STATIC && b.lu_depth == 1 &&
+                     (elem_size == 4 || ctx->opt.fused_step != 4) && (b.solve_wg || refs <= 2e6);
+  if (!fused && !b.solve_wg) return;
+  std::map<std::array<int, 4>, std::shared_ptr<BandPlan>> made;
+  auto plan_of = [&](const CellParams &p, int depth) {
+    std::shared_ptr<BandPlan> &q = made[{p.nblk, p.bw, p.sym, depth}];
+    if (!q) q = std::make_shared<BandPlan>(make_band_plan(p.nblk, p.bw, p.sym != 0, depth));
+    return q;
+  };
+  std::vector<int> depth(b.ncell, 0);
+  auto cuts_for = [&](const CellParams &p, int levels, int most) {  // fewest cuts reaching `levels`, else the shortest
+    int best = 0, len = band_steps(p.nblk, p.bw, 0);
+    for (int d = 0; d <= most; ++d) {
+      const int e = band_steps(p.nblk, p.bw, d);
+      if (e < len) { len = e; best = d; }
+      if (e <= levels) return d;
+    }
+    return best;
+  };
+  // the reported two-chain layout: cells longer than the shortest batch of
+  // cells cut once
+  int chain2 = 0;
+  auto halves = [](const CellParams &p, int &m, int &nb) {
+    if (p.csr || p.bw < 1 || p.bw >= p.nblk - 1 || p.nblk - 2 * p.bw < 2) return false;
+    nb = (p.nblk - 2 * p.bw) / 2;
+    m = p.nblk - p.bw - nb;
+    return m + p.bw < p.nblk;
+  };
+  for (const CellParams &p : b.cp_h) {
+    int m, nb;
+    if (!p.csr) chain2 = std::max(chain2, halves(p, m, nb) ? m + p.bw : p.nblk);
+  }
+  if (fused && b.solve_wg && ctx->opt.fused_step >= 1 && ctx->opt.twist) {
+    if (ctx->opt.twist == 2) {
+      for (int c = 0; c < b.ncell; ++c)
+        if (!b.cp_h[c].csr && b.cp_h[c].nblk > chain2) depth[c] = 1;
+    } else {
+      const int f64 = elem_size == 8;
+      const double t_op = f64 ? 0.5 : 0.25, slots = step_slots(ctx, elem_size);
+      // cells of one shape count once
+      std::map<std::array<int, 3>, int> shapes;
+      for (const CellParams &p : b.cp_h)
+        if (!p.csr && p.nblk > 0) ++shapes[{p.nblk, p.bw, p.sym}];
+      std::vector<int> cand;
+      for (auto &sh : shapes)
+        for (int d = 0; d <= MAX_CUTS; ++d) cand.push_back(band_steps(sh.first[0], sh.first[1], d));
+      std::sort(cand.begin(), cand.end());
+      cand.erase(std::unique(cand.begin(), cand.end()), cand.end());
+      double best = 1e300;
+      int best_c = INT_MAX;
+      for (int C : cand) {
+        int levels = 0;
+        double sweep = 0.0;
+        bool split = false;
+        std::vector<std::vector<std::pair<const BandPlan::Level *, double>>> by_level;
+        for (auto &sh : shapes) {
+          CellParams p{};
+          p.nblk = sh.first[0];
+          p.bw = sh.first[1];
+          p.sym = sh.first[2];
+          const std::shared_ptr<BandPlan> P = plan_of(p, cuts_for(p, C, MAX_CUTS));
+          levels = std::max(levels, (int)P->lev.size());
+          by_level.resize(levels);
+          for (size_t l = 0; l < P->lev.size(); ++l) by_level[l].push_back({&P->lev[l], (double)sh.second});
+          int f = 0, w = 0;
+          for (size_t q = 0; q < P->fwd.size(); ++q) {
+            f = std::max(f, P->fwd[q].nop);
+            w = std::max(w, P->bwd[q].nop);
+          }
+          split |= P->top.nop > 0;
+          sweep = std::max(sweep, t_op * (f + 2.0 * w + P->top.nop + P->top_bwd.nop));
+        }
+        double t = sweep + (split ? 30.0 : 0.0);
+        for (int l = 0; l < levels; ++l) {
+          double tl = 0.0;
+          LuPlan::choose_deal(by_level[l], 1, f64, slots, &tl);  // the cuts do not depend on fused_step
+          t += tl;
+        }
+        if (t < best) {
+          best = t;
+          best_c = C;
+        }
+      }
+      for (int c = 0; c < b.ncell; ++c)
+        if (!b.cp_h[c].csr) depth[c] = cuts_for(b.cp_h[c], best_c, MAX_CUTS);
+    }
+  }
+  for (int c = 0; c < b.ncell; ++c) {
+    CellParams &p = b.cp_h[c];
+    if (p.csr || p.nblk == 0) continue;
+    b.plans[c] = plan_of(p, depth[c]);
+    p.slot_off = b.nslot;
+    b.nslot += b.plans[c]->nslot;
+    if (b.plans[c]->leaves > 1) {
+      int m, nb;
+      if (p.nblk > chain2 && halves(p, m, nb)) {
+        b.chain_top[c] = m;
+        b.chain_bottom[c] = nb;
+      }
+      // automatic schedule: two concurrent cell groups, so one group's
+      // latency-bound launches overlap the other's fuller ones
+      if (ctx->opt.lu_groups == 0) b.lu_groups = 2;
+    }
+  }
+}
+
+// The band plans' tables on the device, the LU schedule and the sweeps'
+// workgroup lists.
+void upload_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
+  std::vector<int> rank;
+  for (CellParams &p : b.cp_h) {
+    p.rank_off = (int)rank.size();
+    const std::shared_ptr<BandPlan> &P = b.plans[&p - b.cp_h.data()];
+    for (int i = 0; i < p.nblk; ++i) rank.push_back(P ? P->rank[i] : i);
+  }
+  b.rank = dupload(rank);
+  HIPCHECK(hipMemcpy(b.cp, b.cp_h.data(), sizeof(CellParams) * b.ncell, hipMemcpyHostToDevice));
+  const bool planned = std::any_of(b.plans.begin(), b.plans.end(), [](const std::shared_ptr<BandPlan> &p) { return !!p; });
+  bool fused = ctx->opt.fused_step > 0 && b.lu_depth == 1 && planned &&
+               (elem_size == 4 || ctx->opt.fused_step != 4);
+  std::vector<BlockRef> refs;
+  std::vector<FwdOp> fops;
+  std::vector<SweepOp> ops;
+  std::vector<SweepLoc> locs;
+  std::vector<int> accs;
+  struct At {
+    int ref, fop, op, loc, acc;
+  };
+  std::map<const BandPlan *, At> at;
+  std::vector<const BandPlan *> plans(b.ncell, nullptr);
+  std::vector<int2> base(b.ncell, make_int2(0, 0));
+  static const BandPlan empty;
+  for (int c = 0; c < b.ncell; ++c) {
+    const BandPlan *P = b.plans[c] ? b.plans[c].get() : &empty;
+    plans[c] = P;
+    auto it = at.find(P);
+    if (it == at.end()) {
+      it = at.insert({P, At{(int)refs.size(), (int)fops.size(), (int)ops.size(), (int)locs.size(), (int)accs.size()}}).first;
+      refs.insert(refs.end(), P->refs.begin(), P->refs.end());
+      fops.insert(fops.end(), P->fops.begin(), P->fops.end());
+      ops.insert(ops.end(), P->ops.begin(), P->ops.end());
+      for (SweepLoc l : P->locs) {
+        l.acc0 += it->second.acc;
+        locs.push_back(l);
+      }
+      accs.insert(accs.end(), P->accs.begin(), P->accs.end());
+    }
+    base[c] = make_int2(it->second.ref, it->second.fop);
+  }
+  b.refs = dupload(refs);
+  b.fops = dupload(fops);
+  if (fused)
+    b.plan.build_fused(b.cp_h, plans, base, b.lu_groups, ctx->opt.fused_step, elem_size == 8,
+                       step_slots(ctx, elem_size), !ctx->opt.batched);
+  if (!fused || !b.solve_wg) {
+    LuPlan lists;
+    lists.build(b.cp_h, ctx->opt.pivoting, b.lu_groups, b.lu_depth);
+    if (!fused) {
+      b.plan = lists;
+    } else {  // the spread-out solve's lists beside the fused schedule
+      b.plan.solve_batched = lists.solve_batched;
+      b.plan.solve_single = lists.solve_single;
+      (void)hipFree(b.plan.d_solve);
+      b.plan.d_solve = lists.d_prefix;
+    }
+  }
+  if (!b.solve_wg) return;
+  b.sops = dupload(ops);
+  b.slocs = dupload(locs);
+  b.saccs = dupload(accs);
+  std::vector<SweepWG> wg;
+  auto lists_of = [&](const std::vector<int> &cells) {
+    Batch::SweepLists S;
+    for (int c : cells) S.split |= plans[c]->top.nop > 0;
+    auto list = [&](Batch::SweepList &L, auto parts) {
+      L.off = (int)wg.size();
+      for (int c : cells) {
+        const At &o = at[plans[c]];
+        for (const SweepPart *q : parts(*plans[c])) {
+          if (q->nloc == 0) continue;
+          wg.push_back(SweepWG{c, SweepPart{q->op0 + o.op, q->nop, q->loc0 + o.loc, q->nloc}});
+          L.max_loc = std::max(L.max_loc, q->nloc);
+        }
+      }
+      L.n = (int)wg.size() - L.off;
+    };
+    auto each = [](const std::vector<SweepPart> &v) {
+      std::vector<const SweepPart *> r;
+      for (const SweepPart &p : v) r.push_back(&p);
+      return r;
+    };
+    typedef std::vector<const SweepPart *> Parts;
+    if (S.split) {
+      list(S.fwd, [&](const BandPlan &P) { return each(P.fwd); });
+      list(S.top, [&](const BandPlan &P) { return Parts{&P.top}; });
+      list(S.top_bwd, [&](const BandPlan &P) { return Parts{&P.top_bwd}; });
+    } else {
+      list(S.whole, [&](const BandPlan &P) { return Parts{&P.whole}; });
+    }
+    list(S.bwd, [&](const BandPlan &P) { return each(P.bwd); });
+    return S;
+  };
+  // longest streams first
+  std::vector<int> order(b.ncell);
+  for (int c = 0; c < b.ncell; ++c) order[c] = c;
+  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return b.cp_h[x].nblk > b.cp_h[y].nblk; });
+  b.sweeps = lists_of(order);
+  b.sweeps_cell.clear();
+  if (!ctx->opt.batched)
+    for (int c = 0; c < b.ncell; ++c) b.sweeps_cell.push_back(lists_of({c}));
+  b.swg = dupload(wg);
 }
 
 void build_batch(wcfe_ctx *ctx, Batch &b, const std::vector<HostCell> &hc, int elem_size) {
@@ -907,44 +1267,7 @@ void build_batch(wcfe_ctx *ctx, Batch &b, const std::vector<HostCell> &hc, int e
     p.env = std::min(full, p.bw + std::max(b.lu_depth - 1, b.solve_wg ? 0 : 1));
     if (!p.csr) b.max_bw = std::max(b.max_bw, p.bw);
   }
-  // two-chain band LU: the batch's chain of block steps is its longest cell's;
-  // a cell of n blocks and block bandwidth bw factored as two chains takes
-  // m + bw steps (m = n - bw - nb top blocks, nb = (n - 2 bw) / 2 bottom
-  // blocks: nb <= m - bw, so the chains never update the middle window in the
-  // same step).  Only cells longer than the shortest achievable batch chain
-  // are split (the others keep their factorization bit for bit).
-  if (elem_size == 4 && ctx->opt.twist && ctx->opt.pivoting == WCFE_PIVOT_STATIC && b.lu_depth == 1 &&
-      b.solve_wg && ctx->opt.fused_step >= 1 && b.max_bw <= 4) {
-    auto split = [](const CellParams &p, int &m, int &nb) {
-      if (p.csr || p.bw < 1 || p.bw >= p.nblk - 1 || p.nblk - 2 * p.bw < 2) return false;
-      nb = (p.nblk - 2 * p.bw) / 2;
-      m = p.nblk - p.bw - nb;
-      return m + p.bw < p.nblk;
-    };
-    int chain = 0;
-    double work = 0.0;  // block products of the whole factorization, about nblk (bw+1)(bw+2)/2 per cell
-    for (const CellParams &p : b.cp_h) {
-      if (p.csr) continue;
-      int m, nb;
-      chain = std::max(chain, split(p, m, nb) ? m + p.bw : p.nblk);
-      work += (double)p.nblk * (p.bw + 1) * (p.sym ? (p.bw + 2) * 0.5 : (p.bw + 1));
-    }
-    // automatic (twist 1): only when the shorter chain's launches stay
-    // latency bound -- at most 8 block products per compute unit and step;
-    // a batch whose launches are throughput bound gains nothing from fewer,
-    // fuller launches
-    if (ctx->opt.twist == 1 && work > 8.0 * ctx->n_cu * chain) chain = INT_MAX;
-    for (CellParams &p : b.cp_h) {
-      int m, nb;
-      if (p.nblk > chain && split(p, m, nb)) {
-        p.tw_m = m;
-        p.tw_nb = nb;
-        // automatic schedule: two concurrent cell groups, so one group's
-        // latency-bound launches overlap the other's fuller ones
-        if (ctx->opt.lu_groups == 0) b.lu_groups = 2;
-      }
-    }
-  }
+  plan_bands(ctx, b, elem_size);
   // colour-major element order
   b.color_start.assign(b.ncolor + 1, 0);
   b.cell_color.assign(b.ncell, std::vector<int>(b.ncolor + 1, 0));
@@ -1157,10 +1480,9 @@ void build_batch(wcfe_ctx *ctx, Batch &b, const std::vector<HostCell> &hc, int e
         for (int d = 0; d < 2; ++d) kinv[p.sys_off + 2 * b.kpos_h[c][i] + d] = 2 * (p.node_off + i) + d;
     }
     b.kinv = dupload(kinv);
-    b.yfwd = dalloc<float>(std::max(sys, 1));
-    bool twist = false;
-    for (const CellParams &p : b.cp_h) twist |= p.tw_m > 0;
-    if (twist) b.ysw = (void *)dalloc<unsigned char>((size_t)std::max(sys, 1) * elem_size);
+    b.yfwd = (void *)dalloc<unsigned char>((size_t)std::max(sys, 1) * elem_size);
+    b.ysw = (void *)dalloc<unsigned char>((size_t)std::max(sys, 1) * elem_size);
+    b.slots = (void *)dalloc<unsigned char>((size_t)std::max(b.nslot, 1) * NB * elem_size);
   }
   const size_t yb = lu_solve_exchange_bytes(std::max(sys, 1), elem_size);
   b.ysol = (void *)dalloc<unsigned char>(yb);
@@ -1316,8 +1638,7 @@ void build_batch(wcfe_ctx *ctx, Batch &b, const std::vector<HostCell> &hc, int e
     b.g_node = dupload(gnode);
     b.g_start_h = gs;
   }
-  b.plan.build(b.cp_h, ctx->opt.pivoting, b.lu_groups, b.lu_depth, elem_size == 4 ? ctx->opt.fused_step : 0,
-               2 * ctx->n_cu);
+  upload_bands(ctx, b, elem_size);
   if (ctx->opt.pivoting == WCFE_PIVOT_PARTIAL &&
       lu_solve_lds_bytes(b.max_npad, elem_size) > lu_solve_max_dynamic(ctx->max_lds))
     fail(WCFE_ERR_ARG, "system of %d unknowns exceeds the LDS-resident triangular solve (%zu bytes max)", b.max_npad,
@@ -1413,10 +1734,50 @@ template <class T> void enqueue_assemble(wcfe_ctx *ctx, Batch &b, const Scope &s
                        static_cast<T *>(b.Kb), b.row_ptr, b.bcol, b.diag_pos, b.G);
 }
 
+// The first solve's forward substitution beside the fused block steps (its
+// result is only read by the one-workgroup sweeps).
+template <class T> StepFwd<T> step_fwd(const Batch &b) {
+  StepFwd<T> f;
+  if (b.solve_wg) f.y = static_cast<T *>(b.yfwd);
+  else f.store_id = 1;
+  f.slot = static_cast<T *>(b.slots);
+  f.kinv = b.kinv;
+  f.G = b.G;
+  return f;
+}
+
+// One refinement solve of the band plans' sweeps: forward over the leaves,
+// the separators, backward over the leaves (first: the forward part already
+// ran beside the block steps).
+template <class T>
+void enqueue_sweeps(hipStream_t s, const Batch &b, const Batch::SweepLists &L, bool first, int accumulate) {
+  SweepVec<T> v;
+  v.rhs = b.r;
+  v.x = static_cast<T *>(b.ysw);
+  v.y = first ? static_cast<const T *>(b.yfwd) : v.x;
+  v.slot = static_cast<T *>(b.slots);
+  v.delta = b.delta;
+  v.from_y = first ? 1 : 0;
+  auto go = [&](const Batch::SweepList &l) {
+    launch_band_sweep<T>(s, b.cp, b.cs, b.swg + l.off, l.n, l.max_loc, b.sops, b.slocs, b.saccs,
+                         static_cast<const T *>(b.K), static_cast<const T *>(b.Dinv), b.kinv, v, accumulate);
+  };
+  if (first) {
+    go(L.top_bwd);
+    go(L.bwd);
+  } else if (L.split) {
+    go(L.fwd);
+    go(L.top);
+    go(L.bwd);
+  } else {
+    go(L.whole);
+  }
+}
+
 // Launch the LU stages of a plan for a list of cells.
 template <class T>
 void enqueue_lu(wcfe_ctx *ctx, hipStream_t s, const LuPlan &plan, const std::vector<Stage> &stages, const int *cells,
-                int ncell, const CellParams *cp, CellState *cs, T *K, T *Dinv, int *ipiv, StepFwd fwd = StepFwd{}) {
+                int ncell, const CellParams *cp, CellState *cs, T *K, T *Dinv, int *ipiv, const Batch *b = nullptr) {
   const bool piv = plan.pivoting != 0;
   {
     PhaseScope ph(ctx, WCFE_PH_LU_PANEL);
@@ -1461,15 +1822,19 @@ void enqueue_lu(wcfe_ctx *ctx, hipStream_t s, const LuPlan &plan, const std::vec
         break;
       }
       case ST_STEP: {
-        if (sizeof(T) != 4) fail(WCFE_ERR_STATE, "the fused block step is built for FP32 factors only");
         KernelTimer kt(ctx, WCFE_PH_LU_GEMM, g.work);
-        launch_lu_step<T>(s, cp, cs, wl, g.k, K, Dinv, LuPlan::step_flag(g.np), fwd, kt.a, kt.b);
+        launch_lu_step<T>(s, cp, cs, plan.d_items + g.off, g.tot, b->refs, b->fops, K, Dinv, step_fwd<T>(*b), kt.a,
+                          kt.b);
         break;
       }
       case ST_CELL: {
-        if (sizeof(T) != 4) fail(WCFE_ERR_STATE, "the fused block step is built for FP32 factors only");
-        KernelTimer kt(ctx, WCFE_PH_LU_GEMM, g.work);
-        launch_lu_cell<T>(s, cp, cs, wl, K, Dinv, fwd, kt.a, kt.b);
+        if constexpr (sizeof(T) == 4) {
+          KernelTimer kt(ctx, WCFE_PH_LU_GEMM, g.work);
+          launch_lu_cell(s, cp, cs, plan.d_ranges + g.off, g.tot, plan.d_items, b->refs, b->fops, K, Dinv,
+                         step_fwd<T>(*b), kt.a, kt.b);
+        } else {
+          fail(WCFE_ERR_STATE, "one workgroup per cell is built for FP32 factors only");
+        }
         break;
       }
     }
@@ -1487,14 +1852,13 @@ template <class T> void enqueue_factor(wcfe_ctx *ctx, Batch &b, const Scope &sc)
       hipStream_t gs = ctx->side[g];
       HIPCHECK(hipStreamWaitEvent(gs, ctx->fork_ev, 0));
       enqueue_lu<T>(ctx, gs, b.plan, b.plan.grp[g], b.plan.d_prefix + b.plan.grp_cells_off[g], b.plan.grp_ncell[g],
-                    b.cp, b.cs, static_cast<T *>(b.K), static_cast<T *>(b.Dinv), b.ipiv,
-                    StepFwd{b.yfwd, b.kinv, b.G});
+                    b.cp, b.cs, static_cast<T *>(b.K), static_cast<T *>(b.Dinv), b.ipiv, &b);
       HIPCHECK(hipEventRecord(ctx->join_ev[g], gs));
       HIPCHECK(hipStreamWaitEvent(ctx->stream, ctx->join_ev[g], 0));
     }
   } else {
     enqueue_lu<T>(ctx, ctx->stream, b.plan, stages, sc.cells, sc.ncell, b.cp, b.cs, static_cast<T *>(b.K),
-                  static_cast<T *>(b.Dinv), b.ipiv, StepFwd{b.yfwd, b.kinv, b.G});
+                  static_cast<T *>(b.Dinv), b.ipiv, &b);
   }
   const int *cl;
   int cb, nch, ncl;
@@ -1571,6 +1935,8 @@ template <class T> void enqueue_pcg(wcfe_ctx *ctx, Batch &b, const Scope &sc, in
   if (hint) *hint = most;
 }
 
+const int *solve_lists(const LuPlan &p) { return p.d_solve ? p.d_solve : p.d_prefix; }
+
 // The refinement residual for a mesh batch: r = -G - K d from the FP64
 // element matrices.
 template <class T> void enqueue_solve_refine(wcfe_ctx *ctx, Batch &b, const Scope &sc) {
@@ -1594,15 +1960,13 @@ template <class T> void enqueue_solve_refine(wcfe_ctx *ctx, Batch &b, const Scop
       } else if (npad > 0) {
         // in each dense cell's own numbering: rp = P r, solve, delta (+)= P^T dp
         const LuPlan::SolveLists &L = sc.cell < 0 ? b.plan.solve_batched : b.plan.solve_single[sc.cell];
-        if (b.solve_wg) {  // the sweep kernel reads r and writes delta through the numbering itself
+        if (b.solve_wg) {  // the sweeps read r and write delta through the numbering themselves
           // first solve after a fused factorization: its forward sweep ran in the block steps (r = -G)
-          const float *yf = (it == 0 && b.plan.fused) ? b.yfwd : nullptr;
-          launch_lu_solve_band<T>(s, b.cp, b.cs, sc.cells, sc.ncell, K, static_cast<const T *>(b.Dinv), b.kpos, b.r,
-                                  b.delta, it > 0, npad, b.max_bw, yf, static_cast<T *>(b.ysw));
+          enqueue_sweeps<T>(s, b, sc.cell < 0 ? b.sweeps : b.sweeps_cell[sc.cell], it == 0 && b.plan.fused, it > 0);
         } else {
           launch_perm_gather(s, b.node_cell, b.cp, b.kpos, b.r, b.rp, sc.node_begin, sc.node_end);
-          launch_lu_solve_mw<T>(s, b.cp, b.cs, sc.cells, sc.ncell, WorkList{b.plan.d_prefix + L.fwd_off, L.tot},
-                                WorkList{b.plan.d_prefix + L.bwd_off, L.tot}, K, static_cast<const T *>(b.Dinv), b.rp,
+          launch_lu_solve_mw<T>(s, b.cp, b.cs, sc.cells, sc.ncell, WorkList{solve_lists(b.plan) + L.fwd_off, L.tot},
+                                WorkList{solve_lists(b.plan) + L.bwd_off, L.tot}, K, static_cast<const T *>(b.Dinv), b.rp,
                                 b.dp, b.ysol, b.sync, 0);
           launch_perm_scatter(s, b.node_cell, b.cp, b.cs, b.kpos, b.dp, b.delta, sc.node_begin, sc.node_end, it > 0);
         }
@@ -1640,7 +2004,7 @@ template <class T> void enqueue_newton(wcfe_ctx *ctx, Batch &b, const Scope &sc)
     PhaseScope ph(ctx, WCFE_PH_FILL);
     // fused band LU with the one-workgroup sweeps: the upper band blocks of
     // symmetric cells are written by the factorization before any read
-    launch_fill_systems<T>(s, b.cp, sc.cells, sc.ncell, npad, K, b.plan.fused && b.solve_wg ? 1 : 0);
+    launch_fill_systems<T>(s, b.cp, sc.cells, sc.ncell, npad, K, b.rank, b.plan.fused && b.solve_wg ? 1 : 0);
     if (b.any_csr) {
       const long long bb = sc.cell < 0 ? 0 : b.blk_begin_h[sc.cell], be = sc.cell < 0 ? b.nnzb : b.blk_end_h[sc.cell];
       launch_zero<T>(s, static_cast<T *>(b.Kb) + 4 * bb, 4 * (be - bb));
@@ -2255,7 +2619,7 @@ int wcfe_autotune(wcfe_ctx *ctx, int32_t flags, int32_t steps, int32_t *chosen, 
       chosen[2] = ctx->opt.dense_max_dof;
       chosen[3] = ctx->b.plan.cell_loop ? 4 : ctx->b.plan.fused ? ctx->opt.fused_step : 0;
       int ntw = 0;
-      for (const CellParams &p : ctx->b.cp_h) ntw += p.tw_m > 0;
+      for (int m : ctx->b.chain_top) ntw += m > 0;
       chosen[4] = ntw;
       chosen[5] = ctx->opt.pcg_lanes > 0 ? ctx->opt.pcg_lanes : 4;
     }
@@ -2597,8 +2961,8 @@ int wcfe_get_cell_layout(wcfe_ctx *ctx, int32_t cell, int32_t *solver, int32_t *
     if (nblk) *nblk = p.nblk;
     if (bw) *bw = p.bw;
     if (sym) *sym = p.sym;
-    if (chain_top) *chain_top = p.tw_m;
-    if (chain_bottom) *chain_bottom = p.tw_nb;
+    if (chain_top) *chain_top = ctx->b.chain_top[cell];
+    if (chain_bottom) *chain_bottom = ctx->b.chain_bottom[cell];
   });
 }
 
@@ -2682,11 +3046,11 @@ int wcfe_assembled_system(wcfe_ctx *ctx, int32_t cell, double *K, double *G) {
     const size_t es = mixed(ctx) ? 4 : 8;
     const long long b0 = p.csr ? b.blk_begin_h[cell] : 0, b1 = p.csr ? b.blk_end_h[cell] : 0;
     if (mixed(ctx)) {
-      launch_fill_systems<float>(ctx->stream, b.cp, sc.cells, 1, p.npad, static_cast<float *>(b.K));
+      launch_fill_systems<float>(ctx->stream, b.cp, sc.cells, 1, p.npad, static_cast<float *>(b.K), b.rank);
       if (p.csr) launch_zero<float>(ctx->stream, static_cast<float *>(b.Kb) + 4 * b0, 4 * (b1 - b0));
       enqueue_assemble<float>(ctx, b, sc, ASM_FULL);
     } else {
-      launch_fill_systems<double>(ctx->stream, b.cp, sc.cells, 1, p.npad, static_cast<double *>(b.K));
+      launch_fill_systems<double>(ctx->stream, b.cp, sc.cells, 1, p.npad, static_cast<double *>(b.K), b.rank);
       if (p.csr) launch_zero<double>(ctx->stream, static_cast<double *>(b.Kb) + 4 * b0, 4 * (b1 - b0));
       enqueue_assemble<double>(ctx, b, sc, ASM_FULL);
     }

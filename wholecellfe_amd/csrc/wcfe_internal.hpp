@@ -4,6 +4,7 @@
 
 #include <string>
 
+#include "band_plan.hpp"
 #include "wcfe_device.hpp"
 
 namespace wcfe {
@@ -20,7 +21,7 @@ enum AsmMode : int { ASM_FULL = 0, ASM_RESIDUAL = 1, ASM_STRAIN = 2 };
 
 template <class T>
 void launch_fill_systems(hipStream_t s, const CellParams *cp, const int *cells, int ncell, int max_npad, T *K,
-                         int lower_only = 0);
+                         const int *rank, int lower_only = 0);
 void launch_fill(hipStream_t s, double *p, long long n, double value);
 void launch_copy(hipStream_t s, const void *src, void *dst, long long bytes);
 // K: dense systems; Kb: block-CSR values of sparse cells (View::el_bpos)
@@ -117,23 +118,6 @@ void launch_lu_trsm(hipStream_t s, const CellParams *cp, CellState *cs, const Wo
 template <class T>
 void launch_lu_gemm(hipStream_t s, const CellParams *cp, CellState *cs, const WorkList &wl, int k, T *K, T *Dinv,
                     int next_diag, int npanel, int strip, hipEvent_t ev_start = nullptr, hipEvent_t ev_stop = nullptr);
-// fused block step k (narrow bands, static pivoting): trailing update of
-// panel k, factor of diagonal block k + 1 and the block solves of panel k + 1
-// the forward substitution of the first solve inside the fused block steps:
-// y (band numbering, per cell at sys_off) = L^-1 P (-G); kinv: per band row
-// its batch dof (-1: padding); y null: no forward items work
-struct StepFwd {
-  float *y = nullptr;
-  const int *kinv = nullptr;
-  const double *G = nullptr;
-};
-template <class T>
-void launch_lu_step(hipStream_t s, const CellParams *cp, CellState *cs, const WorkList &wl, int k, T *K, T *Dinv,
-                    int panel, StepFwd fwd, hipEvent_t ev_start = nullptr, hipEvent_t ev_stop = nullptr);
-// every block step of every listed cell in one launch, one workgroup per cell
-template <class T>
-void launch_lu_cell(hipStream_t s, const CellParams *cp, CellState *cs, const WorkList &wl, T *K, T *Dinv,
-                    StepFwd fwd, hipEvent_t ev_start = nullptr, hipEvent_t ev_stop = nullptr);
 template <class T>
 void launch_lu_solve(hipStream_t s, const CellParams *cp, const CellState *cs, const int *cells, int ncell,
                      const T *K, const T *Dinv, const int *ipiv, int pivoting, const double *r, double *delta,
@@ -151,19 +135,52 @@ void launch_lu_solve_mw(hipStream_t s, const CellParams *cp, CellState *cs, cons
 size_t lu_solve_exchange_bytes(long long rows, int elem_size);
 size_t lu_solve_lds_bytes(int npad, int elem_size);
 size_t lu_solve_max_dynamic(size_t max_lds);
-// one workgroup per cell, band-limited left-looking sweeps with the next
-// block's data prefetched (static pivoting, max_bw <= SOLVE_WG_MAX_BW); ysw
-// (batches with two-chain cells): a forward and a backward launch with one
-// workgroup per chain, the forward result kept there (sys elements)
-template <class T>
-void launch_lu_solve_band(hipStream_t s, const CellParams *cp, const CellState *cs, const int *cells, int ncell,
-                          const T *K, const T *Dinv, const int *kpos, const double *r, double *delta, int accumulate,
-                          int max_npad, int max_bw, const float *yfwd = nullptr, T *ysw = nullptr);
 // block bandwidth up to which one workgroup per cell runs the triangular sweeps
 constexpr int SOLVE_WG_MAX_BW = 8;
 // concurrent cell groups of the dense LU chosen automatically for wide bands
 constexpr int AUTO_GROUPS_MAX = 4;
 hipError_t lu_prepare_attributes(size_t max_lds);
+
+// ---- band LU over the plans of band_plan.hpp (k_band.hip) ----
+// the forward substitution of the first solve inside the fused block steps:
+// y (band numbering, per cell at sys_off) = L^-1 P (-G); kinv: per band row
+// its batch dof (-1: padding); slot: the plans' slots; y null: none
+template <class T> struct StepFwd {
+  T *y = nullptr, *slot = nullptr;
+  const int *kinv = nullptr;
+  const double *G = nullptr;
+  int store_id = 0;  // also store the identity half of each diagonal pair (the spread-out solve reads it)
+};
+// one launch of n items (one level of the cells' plans)
+template <class T>
+void launch_lu_step(hipStream_t s, const CellParams *cp, CellState *cs, const StepItem *items, int n,
+                    const BlockRef *refs, const FwdOp *fops, T *K, T *Dinv, StepFwd<T> fwd,
+                    hipEvent_t ev_start = nullptr, hipEvent_t ev_stop = nullptr);
+// every level of every listed cell in one launch, one workgroup per cell
+void launch_lu_cell(hipStream_t s, const CellParams *cp, CellState *cs, const int2 *ranges, int ncell,
+                    const StepItem *items, const BlockRef *refs, const FwdOp *fops, float *K, float *Dinv,
+                    StepFwd<float> fwd, hipEvent_t ev_start = nullptr, hipEvent_t ev_stop = nullptr);
+// one workgroup of a triangular sweep
+struct SweepWG {
+  int cell;
+  SweepPart part;
+};
+// its vectors (band numbering, per cell at sys_off, but rhs and delta): SL_RHS
+// blocks from rhs (from_y: from y), SL_Y from y, SL_X from x; SL_OUT_Y to x,
+// SL_OUT_D to delta
+template <class T> struct SweepVec {
+  const double *rhs;
+  const T *y;
+  T *x, *slot;
+  double *delta;
+  int from_y;
+};
+// max_loc: the most LDS vector blocks of a workgroup in the launch
+template <class T>
+void launch_band_sweep(hipStream_t s, const CellParams *cp, const CellState *cs, const SweepWG *wgs, int nwg,
+                       int max_loc, const SweepOp *ops, const SweepLoc *locs, const int *accs, const T *K,
+                       const T *Dinv, const int *kinv, const SweepVec<T> &sv, int accumulate);
+hipError_t band_prepare_attributes(size_t max_lds);
 
 // ---- sparse path: block-CSR systems and batched PCG (k_csr.hip) ----
 constexpr int CG_ROWS = 1024;  // nodes per chunk (one thread per node)
