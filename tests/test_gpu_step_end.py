@@ -1,0 +1,45 @@
+"""A cell's Newton steps do not depend on the batch it is in: alone, one
+workgroup runs its refinement and ends its step; beside enough other cells the
+same phases run as batch-wide launches, with one workgroup per cell only for
+the sweeps after the second."""
+import numpy as np
+import pytest
+
+import cells
+
+pytestmark = pytest.mark.gpu
+
+W = pytest.importorskip("wholecellfe_amd")
+
+
+def states(ds, prec, lin_rtol, kinetics, n):
+    with W.Context(precision=prec, t0=1.0, lin_rtol=lin_rtol, max_refine=5) as c:
+        for d in ds:
+            cells.add_to_context(c, d, kinetics=kinetics)
+        c.finalize()
+        for _ in range(4):
+            c.newton_step(stats=False)
+        c.synchronize()
+        return [(c.positions(i),) + tuple(c.ul_state(i)) for i in range(n)]
+
+
+# lin_rtol 0: all five sweeps run
+@pytest.mark.parametrize("prec", [W.PREC_MIXED, W.PREC_FP64])
+@pytest.mark.parametrize("lin_rtol", [1e-12, 0.0])
+@pytest.mark.parametrize("kind", ["spring", "ul"])
+def test_cell_alone_equals_cell_in_a_large_batch(kind, lin_rtol, prec):
+    print("case", kind, lin_rtol, prec, flush=True)
+    make = (lambda K: cells.cst_cell(K=K, n_spr=10 * K, seed=K, time=1.0)) if kind == "spring" else \
+        (lambda K: cells.ul_cell(K=K, seed=K))
+    kin = 0 if kind == "spring" else W.KIN_MEANFIELD
+    few = [make(K) for K in (1, 2, 5)]
+    # 10 disks of 6936 triangles: above 65536 elements, and too long for one workgroup's whole refinement
+    filler = [make(34) for _ in range(10)]
+    lone = [states([d], prec, lin_rtol, kin, 1)[0] for d in few]
+    many = states(few + filler, prec, lin_rtol, kin, len(few))
+    for d, a, b in zip(few, lone, many):
+        move = np.linalg.norm(b[0] - np.asarray(d["x"]).ravel())
+        # relative residual 1e-12 at a condition number below 1e6
+        assert np.linalg.norm(a[0] - b[0]) <= 1e-6 * move
+        for p, q in zip(a[1:], b[1:]):
+            assert np.abs(p - q).max() <= 1e-6 * max(1.0, np.abs(q).max())

@@ -23,7 +23,7 @@ ARCH = "gfx950"
 
 SOURCES = ["k_assemble.hip", "k_lu.hip", "k_band.hip", "k_csr.hip", "k_reference.hip", "k_boundary.hip", "wcfe_vtk.hip",
            "wcfe_api.hip", "wcfe_noalloc.hip"]
-HEADERS = ["wcfe_device.hpp", "wcfe_internal.hpp", "band_plan.hpp", "lu_tiles.hpp", "wcfe_exp.hpp"]
+HEADERS = ["wcfe_device.hpp", "wcfe_internal.hpp", "band_plan.hpp", "cell_steps.hpp", "lu_tiles.hpp", "wcfe_exp.hpp"]
 
 FLAGS = [
     "--offload-arch=" + ARCH, "-O3", "-fPIC", "-std=c++17",

@@ -84,10 +84,10 @@ struct BandPlan {
   std::vector<BlockRef> refs;
   std::vector<FwdOp> fops;
   // sweeps: per leaf its forward and backward part; the separators' part
-  // (forward and backward, or backward only); a one-leaf plan has the whole
-  // sweep (forward and backward) in `whole`
+  // (forward and backward, or backward only); the whole sweep by one
+  // workgroup (likewise)
   std::vector<SweepPart> fwd, bwd;
-  SweepPart top, top_bwd, whole;
+  SweepPart top, top_bwd, whole, whole_bwd;
   std::vector<SweepOp> ops;
   std::vector<SweepLoc> locs;
   std::vector<int> accs;
@@ -339,14 +339,15 @@ inline BandPlan make_band_plan(int n, int bw, bool sym, int depth) {
     bwd_rows(mine[v]);
     part(b, o0, l0);
     P.bwd.push_back(b);
-    if (nn == 1) {
-      o0 = (int)P.ops.size();
-      l0 = (int)P.locs.size();
-      for (int t : mine[v]) add_loc(t, SL_RHS, SL_OUT_D, l0);
-      fwd_rows(mine[v]);
-      bwd_rows(mine[v]);
-      part(P.whole, o0, l0);
-    }
+  }
+  {
+    const int o0 = (int)P.ops.size(), l0 = (int)P.locs.size();
+    for (int b : order) add_loc(b, SL_RHS, SL_OUT_D, l0);
+    for (int s : order) row(s, pre[s], SW_FWD, local[s]);
+    const int o1 = (int)P.ops.size();
+    bwd_rows(order);
+    part(P.whole, o0, l0);
+    part(P.whole_bwd, o1, l0);
   }
   if (!top.empty()) {
     const int l0 = (int)P.locs.size();

@@ -5,7 +5,7 @@
 // elements share a node, so every += into the dense system and the residual
 // has a single writer and the summation order per entry is fixed by the
 // colour sequence (run-to-run bitwise deterministic, no atomics).
-#include "wcfe_internal.hpp"
+#include "cell_steps.hpp"
 
 namespace wcfe {
 
@@ -204,7 +204,7 @@ __global__ __launch_bounds__(256) void k_node_gather(const int *adj_start, const
                                                      const double *Ge, double *G) {
   const int n = n0 + blockIdx.x * blockDim.x + threadIdx.x;
   if (n >= n1) return;
-  double g0 = G[2 * n], g1 = G[2 * n + 1];
+  double g0 = 0.0, g1 = 0.0;
   for (int k = adj_start[n]; k < adj_start[n + 1]; ++k) {
     const int pk = adj[k];
     const int e = pk >> 2, a = pk & 3;
@@ -227,7 +227,7 @@ __global__ __launch_bounds__(256) void k_group_gather(View v, const int *node_ce
   if (g >= gp.g1) return;
   const int n = gp.node[g];
   if (g == gp.start[n]) {
-    double g0 = G[2 * n], g1 = G[2 * n + 1];
+    double g0 = 0.0, g1 = 0.0;
     for (int k = adj_start[n]; k < adj_start[n + 1]; ++k) {
       const int pk = adj[k];
       const int e = pk >> 2, a = pk & 3;
@@ -237,7 +237,8 @@ __global__ __launch_bounds__(256) void k_group_gather(View v, const int *node_ce
     G[2 * n] = g0;
     G[2 * n + 1] = g1;
   }
-  const CellParams &p = v.cp[node_cell[n]];
+  const int c = node_cell[n];
+  const CellParams &p = v.cp[c];
   // lower_only: a symmetric cell's blocks whose column is eliminated after
   // their row are written by the fused band LU (U = L^T) before any read
   if (lower_only && p.sym && !p.csr) {
@@ -246,6 +247,7 @@ __global__ __launch_bounds__(256) void k_group_gather(View v, const int *node_ce
   }
   T *b0, *b1;
   if (p.csr) {
+    if (gp.bpos[g] < 0) return;  // a node of no element
     b0 = Kb + 4LL * gp.bpos[g];
     b1 = b0 + 2;
   } else {
@@ -334,77 +336,91 @@ void launch_element_dump(hipStream_t s, const View &v, int e_begin, int e_end, d
 //        iterate), 1 = refinement residual (rnorm), 2 = residual after the
 //        update (gnorm)
 // ---------------------------------------------------------------------------
-__device__ void norm_finish(CellState &s, int which, double nrm, double lin_rtol) {
-  if (which == 0) {
-    s.gnorm = nrm;
-    s.bnorm = nrm;
-    if (s.newton_it == 0) s.g0 = nrm;
-  } else if (which == 1) {
-    s.rnorm = nrm;
-    if (lin_rtol >= 0.0 && !s.ir_done) {  // refinement control (k_ir_control) for this cell
-      s.ir_iters += 1;
-      s.lin_relres = s.bnorm > 0.0 ? s.rnorm / s.bnorm : 0.0;
-      if (s.rnorm <= lin_rtol * s.bnorm) s.ir_done = 1;
-    }
-  } else {
-    s.gnorm = nrm;
-  }
-}
-
 // One workgroup per cell (blockIdx.x) and chunk of NORM_CHUNK entries
 // (blockIdx.y).  A cell of one chunk is summed by its one workgroup; a larger
 // cell's chunks write partial sums and the last chunk to arrive adds them in
 // chunk order (fixed order: bitwise reproducible).
-__global__ __launch_bounds__(256) void k_cell_norm(const CellParams *cp, CellState *cs, const int *cells,
-                                                   const double *vec, int which, int only_active, double lin_rtol,
-                                                   NormWork nw) {
+// K (which 0, dense cells): also the factorization's pivot threshold from the
+// diagonal.  Bound by latency: 16 waves, four entries of both in flight each
+// (10300 nodes: 10 + 28 us as a norm and a threshold kernel of 4 waves).
+constexpr int NORM_THREADS = 1024;
+template <class T>
+__global__ __launch_bounds__(NORM_THREADS) void k_cell_norm(const CellParams *cp, CellState *cs, const int *cells,
+                                                            const double *vec, int which, int only_active,
+                                                            double lin_rtol, NormWork nw, const T *K) {
   const int c = cells[blockIdx.x];
-  if (only_active && cs[c].ir_done) return;
   const CellParams &p = cp[c];
+  if (only_active && (cs[c].ir_done || p.refine)) return;
   const int nch = nw.part ? (p.ndof + NORM_CHUNK - 1) / NORM_CHUNK : 1;
   const int chunk = blockIdx.y;
   if (chunk >= nch) return;
   const double *v = vec + (long long)p.vec_off;
   const int lo = nch > 1 ? chunk * NORM_CHUNK : 0;
   const int hi = nch > 1 ? min(p.ndof, lo + NORM_CHUNK) : p.ndof;
-  // four partial sums per thread: four loads in flight
-  double acc[4] = {0.0, 0.0, 0.0, 0.0};
-  for (int i0 = lo + threadIdx.x; i0 < hi; i0 += 4 * 256) {
+  const bool tau = K && !p.csr;
+  const T *A = K + p.k_off;
+  double acc[4] = {0.0, 0.0, 0.0, 0.0}, m = 0.0;
+  for (int i0 = lo + threadIdx.x; i0 < hi; i0 += 4 * NORM_THREADS) {
+    T d[4] = {T(0), T(0), T(0), T(0)};
+    if (tau) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const long long i = min(i0 + NORM_THREADS * u, hi - 1);
+        d[u] = A[i * p.npad + i];
+      }
+    }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const int i = i0 + 256 * u;
+      const int i = i0 + NORM_THREADS * u;
       const double x = i < hi ? v[i] : 0.0;
       acc[u] += x * x;
     }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) m = fmax(m, fabs((double)d[u]));  // fmax: a NaN is left out
   }
-  __shared__ double red[256];
+  __shared__ double red[NORM_THREADS], redm[NORM_THREADS];
   red[threadIdx.x] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+  redm[threadIdx.x] = m;
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+  for (int w = NORM_THREADS / 2; w > 0; w >>= 1) {
+    if (threadIdx.x < w) {
+      red[threadIdx.x] += red[threadIdx.x + w];
+      redm[threadIdx.x] = fmax(redm[threadIdx.x], redm[threadIdx.x + w]);
+    }
     __syncthreads();
   }
   if (threadIdx.x != 0) return;
-  if (nch == 1) {
-    norm_finish(cs[c], which, sqrt(red[0]), lin_rtol);
-    return;
+  const double eps = sizeof(T) == 4 ? 5.9604644775390625e-08 : 1.1102230246251565e-16;
+  double sum = red[0];
+  m = redm[0];
+  if (nch > 1) {
+    double *part = nw.part + 2LL * c * nw.stride;
+    part[2 * chunk] = sum;
+    part[2 * chunk + 1] = m;
+    const unsigned prev = __hip_atomic_fetch_add(nw.cnt + c, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+    if (prev != (unsigned)(nch - 1)) return;  // not the last chunk of the cell to arrive
+    __hip_atomic_store(nw.cnt + c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    sum = m = 0.0;
+    for (int k = 0; k < nch; ++k) {
+      sum += __hip_atomic_load(part + 2 * k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      m = fmax(m, __hip_atomic_load(part + 2 * k + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    }
   }
-  double *part = nw.part + (long long)c * nw.stride;
-  part[chunk] = red[0];
-  const unsigned prev = __hip_atomic_fetch_add(nw.cnt + c, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-  if (prev != (unsigned)(nch - 1)) return;  // not the last chunk of the cell to arrive
-  __hip_atomic_store(nw.cnt + c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  double sum = 0.0;
-  for (int k = 0; k < nch; ++k) sum += __hip_atomic_load(part + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   norm_finish(cs[c], which, sqrt(sum), lin_rtol);
+  if (tau) tau_finish(cs[c], m, eps);
 }
+template <class T>
 void launch_cell_norm(hipStream_t s, const CellParams *cp, CellState *cs, const int *cells, int ncell,
-                      const double *vec, int which, int only_active, double lin_rtol, const NormWork &nw) {
+                      const double *vec, int which, int only_active, double lin_rtol, const NormWork &nw, const T *K) {
   if (ncell <= 0) return;
   const int nx = nw.part ? std::max(1, nw.stride) : 1;
-  hipLaunchKernelGGL(k_cell_norm, dim3(ncell, nx), dim3(256), 0, s, cp, cs, cells, vec, which, only_active, lin_rtol,
-                     nw);
+  hipLaunchKernelGGL(k_cell_norm<T>, dim3(ncell, nx), dim3(NORM_THREADS), 0, s, cp, cs, cells, vec, which, only_active,
+                     lin_rtol, nw, K);
 }
+template void launch_cell_norm<float>(hipStream_t, const CellParams *, CellState *, const int *, int, const double *,
+                                      int, int, double, const NormWork &, const float *);
+template void launch_cell_norm<double>(hipStream_t, const CellParams *, CellState *, const int *, int, const double *,
+                                       int, int, double, const NormWork &, const double *);
 
 // ---------------------------------------------------------------------------
 // FP64 refinement residual r = -G - K d, element by element from the stored
@@ -418,48 +434,10 @@ __global__ __launch_bounds__(256) void k_matvec_ir(const int *el_tri, const int 
   const int i = node_begin + blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= node_end) return;
   const int c = node_cell[i];
-  if (cs[c].ir_done) return;
-  const double2 *d2 = reinterpret_cast<const double2 *>(delta);
-  double y0 = 0.0, y1 = 0.0;
-  for (int k = adj_start[i]; k < adj_start[i + 1]; ++k) {
-    const int pk = adj[k];
-    const int e = pk >> 2, a = pk & 3;
-    const double *Ke = Ke64 + 36 * (long long)e + 12 * a;
-#pragma unroll
-    for (int b = 0; b < 3; ++b) {
-      const double2 d = d2[el_tri[3 * e + b]];
-      y0 += Ke[2 * b] * d.x + Ke[2 * b + 1] * d.y;
-      y1 += Ke[6 + 2 * b] * d.x + Ke[6 + 2 * b + 1] * d.y;
-    }
-  }
-  if (bv.bidx && cp[c].bterm) {
-    // node terms: drag diagonal, the boundary vertex's 2 x 6 block and the
-    // area term's rank-one part k g_i (sum_m g_m . d_m)
-    const CellParams &p = cp[c];
-    const double2 di = d2[i];
-    if (p.bterm & BT_DRAG) {
-      const double cd = p.drag / bv.dt;
-      y0 += cd * di.x;
-      y1 += cd * di.y;
-    }
-    const int b = bv.bidx[i];
-    if (b >= 0 && (p.bterm & (BT_BEND | BT_AREA))) {
-      const int2 fr = bv.frame[b];
-      if (fr.x >= 0) {
-        const double *J = bv.J + 12LL * b;
-        const double2 d1 = d2[fr.x], dd2 = d2[fr.y];
-        y0 += J[0] * di.x + J[1] * di.y + J[2] * d1.x + J[3] * d1.y + J[4] * dd2.x + J[5] * dd2.y;
-        y1 += J[6] * di.x + J[7] * di.y + J[8] * d1.x + J[9] * d1.y + J[10] * dd2.x + J[11] * dd2.y;
-        if (p.bterm & BT_AREA) {
-          const double2 g = bv.g[b];
-          y0 += p.k_area * g.x * bv.gd[c];
-          y1 += p.k_area * g.y * bv.gd[c];
-        }
-      }
-    }
-  }
-  r[2 * i] = -G[2 * i] - y0;
-  r[2 * i + 1] = -G[2 * i + 1] - y1;
+  if (cs[c].ir_done || cp[c].refine) return;
+  const double2 ri = residual_node(i, c, el_tri, adj_start, adj, Ke64, G, delta, cp[c], bv, bv.gd ? bv.gd[c] : 0.0);
+  r[2 * i] = ri.x;
+  r[2 * i + 1] = ri.y;
 }
 void launch_matvec_ir(hipStream_t s, const View &v, const int *node_cell, const int *adj_start, const int *adj,
                       const double *Ke64, const double *G, const double *delta, double *r, int node_begin,
@@ -507,26 +485,6 @@ void launch_perm_scatter(hipStream_t s, const int *node_cell, const CellParams *
                      n0, n1, accumulate);
 }
 
-__global__ void k_ir_control(CellState *cs, const int *cells, int ncell, double lin_rtol, int reset) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= ncell) return;
-  CellState &s = cs[cells[i]];
-  if (reset) {
-    s.ir_done = 0;
-    s.ir_iters = 0;
-    s.lin_relres = 0.0;
-    return;
-  }
-  if (s.ir_done) return;
-  s.ir_iters += 1;
-  s.lin_relres = s.bnorm > 0.0 ? s.rnorm / s.bnorm : 0.0;
-  if (s.rnorm <= lin_rtol * s.bnorm) s.ir_done = 1;
-}
-void launch_ir_control(hipStream_t s, CellState *cs, const int *cells, int ncell, double lin_rtol, int reset) {
-  if (ncell <= 0) return;
-  hipLaunchKernelGGL(k_ir_control, dim3((ncell + 63) / 64), dim3(64), 0, s, cs, cells, ncell, lin_rtol, reset);
-}
-
 __global__ __launch_bounds__(256) void k_update_x(double2 *x, const double *delta, int node_begin, int node_end) {
   const int i = node_begin + blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= node_end) return;
@@ -543,11 +501,7 @@ void launch_update_x(hipStream_t s, double2 *x, const double *delta, int node_be
 
 __global__ void k_newton_control(CellState *cs, const int *cells, int ncell, double rtol, double atol) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= ncell) return;
-  CellState &s = cs[cells[i]];
-  s.newton_it += 1;
-  s.converged = (s.gnorm <= rtol * s.g0 || s.gnorm <= atol) ? 1 : 0;
-  if (!s.ir_done) s.lin_failed = 1;
+  if (i < ncell) newton_finish(cs[cells[i]], rtol, atol);
 }
 void launch_newton_control(hipStream_t s, CellState *cs, const int *cells, int ncell, double rtol, double atol) {
   if (ncell <= 0) return;
@@ -557,9 +511,6 @@ void launch_newton_control(hipStream_t s, CellState *cs, const int *cells, int n
 // ---------------------------------------------------------------------------
 // commit of a converged load step
 // ---------------------------------------------------------------------------
-// UL:607-612 strain update; UL:2046-2171 mean-field bond kinetics with a rigid
-// substrate (subs_u = 0): fa_u += x - X, catch-slip k_off, forward Euler c_C,
-// dissipative rescale; the new reference configuration is the converged x.
 __global__ __launch_bounds__(256) void k_commit_nodes(View v, const int *node_cell, double2 *X, double2 *x, double *ea,
                                                       double *cC, double2 *fau, const double *Rea, const double *MM,
                                                       int node_begin, int node_end, double dt) {
@@ -567,44 +518,7 @@ __global__ __launch_bounds__(256) void k_commit_nodes(View v, const int *node_ce
   if (i >= node_end) return;
   const int c = node_cell[i];
   if (!v.cs[c].converged) return;
-  const CellParams &p = v.cp[c];
-  if (p.law == LAW_UL) {
-    const double m = MM[i];
-    for (int q = 0; q < 3; ++q) ea[3 * i + q] += Rea[3 * i + q] / m;
-  }
-  const double2 xi = x[i], Xi = X[i];
-  if (p.node_springs) {
-    double2 u = fau[i];
-    u.x = u.x + (xi.x - Xi.x);
-    u.y = u.y + (xi.y - Xi.y);
-    if (p.kinetics == KIN_MEANFIELD) {
-#pragma clang fp contract(off)
-      double force;
-      if (p.spring_law == SPRING_LINEAR) {
-        force = p.k_lin * sqrt(u.x * u.x + u.y * u.y);  // 2D norm, UL1:2077
-      } else {
-        double f[2], J[4];
-        spring_force(v, p, u.x, u.y, f, J);
-        force = sqrt(f[0] * f[0] + f[1] * f[1]);  // UL:2137
-      }
-      const double k_on = 1.0, ka = 0.004, kb = 10.0, Fa = 15.0, Fb = 15.0;  // UL:2139-2143
-      const double k_off = ka * shared_exp(force / Fa) + kb * shared_exp(-force / Fb);
-      const double cold = cC[i];
-      double cnew = cold + dt * k_on * (1.0 - cold) - dt * k_off * cold;
-      if (cnew < 0.0) cnew = 0.0;
-      cC[i] = cnew;
-      const double keep = cold - dt * k_off * cold;
-      if (keep > 0.0 && cnew > 0.0) {
-        u.x = u.x * keep / cnew;
-        u.y = u.y * keep / cnew;
-      } else {
-        u.x = 0.0 * u.x;
-        u.y = 0.0 * u.y;
-      }
-    }
-    fau[i] = u;
-  }
-  if (p.law == LAW_UL) X[i] = xi;
+  commit_node(v, v.cp[c], i, X, x, ea, cC, fau, Rea, MM, dt);
 }
 void launch_commit_nodes(hipStream_t s, const View &v, const int *node_cell, double2 *X, double2 *x, double *ea,
                          double *cC, double2 *fau, const double *Rea, const double *MM, int node_begin, int node_end,
@@ -615,16 +529,9 @@ void launch_commit_nodes(hipStream_t s, const View &v, const int *node_cell, dou
                      node_begin, node_end, dt);
 }
 
-// Bell kinetics per barycentric spring after a converged load step:
-// bound -> unbound with p = 1 - exp(-k_off0 e^{|F(D)|/f_b} dt), D = |u|,
-// unbound -> bound
-// with p = 1 - exp(-k_on dt), re-anchored at the current attachment point.
-// Uniform u = (w + 0.5) 2^-32, w = Philox(ctr = (replica, spring, step, 0)).
 __global__ __launch_bounds__(256) void k_commit_springs(View v, const int *sp_cell, const int *sp_elem,
                                                         const int *sp_local, double *state, double *anchor,
-                                                        int s_begin, int s_end, double dt, double k_on,
-                                                        double k_off0, double f_b, unsigned key_lo, unsigned key_hi,
-                                                        const int *replica_of_cell, int *transitions) {
+                                                        int s_begin, int s_end, BellArgs bell) {
   const int s = s_begin + blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= s_end) return;
   const int c = sp_cell[s];
@@ -632,54 +539,14 @@ __global__ __launch_bounds__(256) void k_commit_springs(View v, const int *sp_ce
   if (!cst.converged) return;
   const CellParams &p = v.cp[c];
   if (p.kinetics != KIN_BELL) return;
-  const int e = sp_elem[s];
-  const double *bb = v.sp_bary + 3 * s;
-  // attachment point (b0 x0 + b1 x1) + b2 x2, rounded term by term without
-  // contraction so a re-anchored bond lands on the same bits as a plain FP64
-  // evaluation of the same expression
-  const double2 x0 = v.x[v.el_tri[3 * e]], x1 = v.x[v.el_tri[3 * e + 1]], x2 = v.x[v.el_tri[3 * e + 2]];
-  double px, py;
-  {
-#pragma clang fp contract(off)
-    px = bb[0] * x0.x + bb[1] * x1.x + bb[2] * x2.x;
-    py = bb[0] * x0.y + bb[1] * x1.y + bb[2] * x2.y;
-  }
-  unsigned ctr[4] = {(unsigned)replica_of_cell[c], (unsigned)sp_local[s], (unsigned)cst.step, 0u};
-  philox4x32_10(ctr, key_lo, key_hi);
-  const double u = ((double)ctr[0] + 0.5) * (1.0 / 4294967296.0);
-  // the force and both probabilities rounded as written, with the shared exp
-  if (state[s] != 0.0) {
-    double ux, uy;
-    {
-#pragma clang fp contract(off)
-      ux = px - anchor[2 * s];
-      uy = py - anchor[2 * s + 1];
-    }
-    const double F = spring_magnitude(v, p, ux, uy);
-    const double koff = k_off0 * shared_exp(F / f_b);
-    const double prob = 1.0 - shared_exp(-koff * dt);
-    if (u < prob) {
-      state[s] = 0.0;
-      atomicAdd(transitions, 1);
-    }
-  } else {
-    const double prob = 1.0 - shared_exp(-k_on * dt);
-    if (u < prob) {
-      state[s] = 1.0;
-      anchor[2 * s] = px;
-      anchor[2 * s + 1] = py;
-      atomicAdd(transitions, 1);
-    }
-  }
+  commit_spring(v, p, c, (unsigned)cst.step, s, sp_elem, sp_local, state, anchor, bell);
 }
 void launch_commit_springs(hipStream_t s, const View &v, const int *sp_cell, const int *sp_elem, const int *sp_local,
-                           double *state, double *anchor, int s_begin, int s_end, double dt, double k_on,
-                           double k_off0, double f_b, unsigned key_lo, unsigned key_hi, const int *replica_of_cell,
-                           int *transitions) {
+                           double *state, double *anchor, int s_begin, int s_end, const BellArgs &bell) {
   const int n = s_end - s_begin;
   if (n <= 0) return;
   hipLaunchKernelGGL(k_commit_springs, dim3((n + 255) / 256), dim3(256), 0, s, v, sp_cell, sp_elem, sp_local, state,
-                     anchor, s_begin, s_end, dt, k_on, k_off0, f_b, key_lo, key_hi, replica_of_cell, transitions);
+                     anchor, s_begin, s_end, bell);
 }
 
 // A remeshed cell's nodes from its old nodes (the host's remeshing maps): new
@@ -725,41 +592,6 @@ void launch_commit_cells(hipStream_t s, CellState *cs, const int *cells, int nce
   if (ncell <= 0) return;
   hipLaunchKernelGGL(k_commit_cells, dim3((ncell + 63) / 64), dim3(64), 0, s, cs, cells, ncell, dt);
 }
-
-// ---------------------------------------------------------------------------
-// static-pivot threshold: tau = 64 eps max_i |K_ii| per cell (the stiffness
-// matrices are SPD in the configurations, so only a nearly singular system
-// has pivots that small)
-// ---------------------------------------------------------------------------
-template <class T>
-__global__ __launch_bounds__(256) void k_diag_tau(const CellParams *cp, CellState *cs, const int *cells, const T *K) {
-  const int c = cells[blockIdx.x];
-  const CellParams &p = cp[c];
-  if (p.npad == 0) return;  // sparse cell: no dense system
-  const T *A = K + p.k_off;
-  double m = 0.0;
-  for (int i = threadIdx.x; i < p.ndof; i += 256) m = fmax(m, fabs((double)A[(long long)i * p.npad + i]));
-  __shared__ double red[256];
-  red[threadIdx.x] = m;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (threadIdx.x < w) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + w]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    const double eps = sizeof(T) == 4 ? 5.9604644775390625e-08 : 1.1102230246251565e-16;
-    cs[c].tau = 64.0 * eps * (red[0] > 0.0 ? red[0] : 1.0);
-    cs[c].n_static = 0;
-    cs[c].zero_pivot = 0;
-  }
-}
-template <class T>
-void launch_diag_tau(hipStream_t s, const CellParams *cp, CellState *cs, const int *cells, int ncell, const T *K) {
-  if (ncell <= 0) return;
-  hipLaunchKernelGGL(k_diag_tau<T>, dim3(ncell), dim3(256), 0, s, cp, cs, cells, K);
-}
-template void launch_diag_tau<float>(hipStream_t, const CellParams *, CellState *, const int *, int, const float *);
-template void launch_diag_tau<double>(hipStream_t, const CellParams *, CellState *, const int *, int, const double *);
 
 // plain device copy, 16 bytes per thread per iteration (bandwidth probe and
 // the known-size reference for the FETCH_SIZE / WRITE_SIZE counters)

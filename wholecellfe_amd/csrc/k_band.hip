@@ -3,6 +3,7 @@
 // FP32 (v_mfma_f32_16x16x4f32) and FP64 (v_mfma_f64_16x16x4f64).
 #include <hip/hip_ext.h>
 
+#include "cell_steps.hpp"
 #include "lu_tiles.hpp"
 
 namespace wcfe {
@@ -560,25 +561,18 @@ template <class T> __device__ __forceinline__ T sum8(T v) {
   }
 }
 
+// One part by the workgroup; y: its LDS vector, rowb: 64 entries of LDS.
 template <class T>
-__global__ __launch_bounds__(SWEEP_THREADS) void k_band_sweep(const CellParams *cp, const CellState *cs,
-                                                              const SweepWG *wgs, const SweepOp *ops,
-                                                              const SweepLoc *locs, const int *accs, const T *K,
-                                                              const T *Dinv, const int *kinv, SweepVec<T> sv,
-                                                              int accumulate) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  __shared__ __attribute__((aligned(16))) T rowb[64];
+__device__ __forceinline__ void sweep_part(const CellParams &p, const SweepPart &pt, const SweepOp *ops,
+                                           const SweepLoc *locs, const int *accs, const T *K, const T *Dinv,
+                                           const int *kinv, const SweepVec<T> &sv, int accumulate, T *y, T *rowb) {
   constexpr int RING = SweepRing<T>::v;
-  T *y = reinterpret_cast<T *>(smem);
-  const SweepWG wg = wgs[blockIdx.x];
-  if (cs[wg.cell].ir_done) return;
-  const CellParams &p = cp[wg.cell];
   const long long ld = p.npad;
-  const int r = threadIdx.x >> 3, q = threadIdx.x & 7, nop = wg.part.nop;
+  const int r = threadIdx.x >> 3, q = threadIdx.x & 7, nop = pt.nop;
   const T *A = K + p.k_off + (long long)r * ld;
   const T *D = Dinv + dinv_off(p, 0) + 4096 + r * 64;
-  const int4 *op = reinterpret_cast<const int4 *>(ops + wg.part.op0);
-  const SweepLoc *loc = locs + wg.part.loc0;
+  const int4 *op = reinterpret_cast<const int4 *>(ops + pt.op0);
+  const SweepLoc *loc = locs + pt.loc0;
   T *slots = sv.slot + (long long)p.slot_off * NB;
   // The operations themselves: lane l of every wave holds operation l of the
   // current chunk and of the next, and the one needed is broadcast by lane
@@ -602,18 +596,16 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_band_sweep(const CellParams *
   };
 #pragma unroll
   for (int i = 0; i < RING; ++i) fetch(R[i], i);
-  for (int i = threadIdx.x; i < wg.part.nloc * 64; i += SWEEP_THREADS) {
+  for (int i = threadIdx.x; i < pt.nloc * 64; i += SWEEP_THREADS) {
     const SweepLoc l = loc[i >> 6];
     const int row = p.sys_off + l.b * NB + (i & 63);
     T v;
-    if (l.init == SL_X) {
-      v = sv.x[row];
-    } else if (l.init == SL_Y || sv.from_y) {
-      v = sv.y[row];
-    } else {
+    if (l.init == SL_RHS && !sv.from_y) {
       const int dof = kinv[row];
       v = dof >= 0 ? (T)sv.rhs[dof] : T(0);
       for (int a = 0; a < l.nacc; ++a) v -= slots[(long long)accs[l.acc0 + a] * NB + (i & 63)];
+    } else {
+      v = (l.init == SL_X ? sv.x : sv.y)[row];
     }
     y[i] = v;
   }
@@ -654,7 +646,7 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_band_sweep(const CellParams *
     nxt = op_load(c0 + 2 * CHUNK);
   }
   lds_barrier();
-  for (int i = threadIdx.x; i < wg.part.nloc * 64; i += SWEEP_THREADS) {
+  for (int i = threadIdx.x; i < pt.nloc * 64; i += SWEEP_THREADS) {
     const SweepLoc l = loc[i >> 6];
     const int row = p.sys_off + l.b * NB + (i & 63);
     if (l.out & SL_OUT_Y) sv.x[row] = y[i];
@@ -663,6 +655,120 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_band_sweep(const CellParams *
       if (dof >= 0) sv.delta[dof] = accumulate ? sv.delta[dof] + (double)y[i] : (double)y[i];
     }
   }
+}
+template <class T>
+__global__ __launch_bounds__(SWEEP_THREADS) void k_band_sweep(const CellParams *cp, const CellState *cs,
+                                                              const SweepWG *wgs, const SweepOp *ops,
+                                                              const SweepLoc *locs, const int *accs, const T *K,
+                                                              const T *Dinv, const int *kinv, SweepVec<T> sv,
+                                                              int accumulate) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  __shared__ __attribute__((aligned(16))) T rowb[64];
+  const SweepWG wg = wgs[blockIdx.x];
+  if (cs[wg.cell].ir_done) return;
+  sweep_part<T>(cp[wg.cell], wg.part, ops, locs, accs, K, Dinv, kinv, sv, accumulate, reinterpret_cast<T *>(smem),
+                rowb);
+}
+
+// The whole refinement of one cell: sweep, FP64 residual, norm and control,
+// again until lin_rtol is met.  Small cells: a sweep streams few blocks, so
+// five launches per refinement sweep (also of the sweeps that have nothing
+// left to do: 4.5 us each in a captured graph) cost more than the work.
+// Cells with smw: the system in the band is B = K - k g g^T (the area term's
+// rank one left out, g = dA/dx on the boundary), and K d = r is solved as
+// d = y - z (g.y) / (1 + g.z) with y = B^-1 r, z = B^-1 k g (Sherman and
+// Morrison 1950), the dots in FP64; the residual is the full K's.  The full
+// matrix is dense (the boundary couples to itself): n^3 instead of n bw^2.
+template <class T>
+__global__ __launch_bounds__(SWEEP_THREADS) void k_band_refine(const CellParams *cp, CellState *cs,
+                                                               const RefineWG *wgs, const SweepOp *ops,
+                                                               const SweepLoc *locs, const int *accs, const T *K,
+                                                               const T *Dinv, const int *kinv, SweepVec<T> sv,
+                                                               RefineArgs ra) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  __shared__ __attribute__((aligned(16))) T rowb[64];
+  __shared__ double red[SWEEP_THREADS];
+  __shared__ int done;
+  T *y = reinterpret_cast<T *>(smem);
+  const RefineWG wg = wgs[blockIdx.x];
+  const int c = wg.cell;
+  if (cs[c].ir_done) return;
+  const CellParams &p = cp[c];
+  const int n0 = p.node_off, n1 = n0 + p.n_nodes;
+  // sum over the boundary vertices of g . v
+  auto gdot = [&](const double *v) {
+    double a = 0.0;
+    for (int b = p.bnd_off + threadIdx.x; b < p.bnd_off + p.n_bnd; b += SWEEP_THREADS) {
+      if (ra.bv.frame[b].x < 0) continue;
+      const double2 g = ra.bv.g[b], d = reinterpret_cast<const double2 *>(v)[ra.bv.node[b]];
+      a += g.x * d.x + g.y * d.y;
+    }
+    return block_sum<SWEEP_THREADS>(a, red);
+  };
+  double den = 1.0;
+  if (p.smw) {
+    for (int i = n0 + threadIdx.x; i < n1; i += SWEEP_THREADS) {
+      const int b = ra.bv.bidx[i];
+      const bool on = b >= 0 && ra.bv.frame[b].x >= 0;
+      const double2 g = on ? ra.bv.g[b] : make_double2(0.0, 0.0);
+      ra.inc[2 * i] = p.k_area * g.x;
+      ra.inc[2 * i + 1] = p.k_area * g.y;
+    }
+    __syncthreads();
+    SweepVec<T> v = sv;
+    v.rhs = ra.inc;
+    v.delta = ra.z;
+    v.from_y = 0;
+    sweep_part<T>(p, wg.whole, ops, locs, accs, K, Dinv, kinv, v, 0, y, rowb);
+    __syncthreads();
+    den = 1.0 + gdot(ra.z);
+  }
+  if (ra.it0 == 0 && !ra.fwd_done) {
+    for (int i = 2 * n0 + threadIdx.x; i < 2 * n1; i += SWEEP_THREADS) ra.r[i] = -ra.G[i];
+    __syncthreads();
+  }
+  for (int it = ra.it0; it < ra.max_refine; ++it) {
+    SweepVec<T> v = sv;
+    v.rhs = ra.r;
+    v.from_y = it == 0 && ra.fwd_done ? 1 : 0;
+    v.delta = p.smw ? ra.inc : ra.delta;
+    sweep_part<T>(p, v.from_y ? wg.bwd : wg.whole, ops, locs, accs, K, Dinv, kinv, v, p.smw ? 0 : it > 0, y, rowb);
+    __syncthreads();
+    if (p.smw) {
+      const double t = gdot(ra.inc) / den;
+      for (int i = 2 * n0 + threadIdx.x; i < 2 * n1; i += SWEEP_THREADS) {
+        const double d = ra.inc[i] - ra.z[i] * t;
+        ra.delta[i] = it > 0 ? ra.delta[i] + d : d;
+      }
+      __syncthreads();
+    }
+    const double gd = p.bterm & BT_AREA ? gdot(ra.delta) : 0.0;
+    double rr = 0.0;
+    for (int i = n0 + threadIdx.x; i < n1; i += SWEEP_THREADS) {
+      const double2 ri =
+          residual_node(i, c, ra.el_tri, ra.adj_start, ra.adj, ra.Ke64, ra.G, ra.delta, p, ra.bv, gd);
+      ra.r[2 * i] = ri.x;
+      ra.r[2 * i + 1] = ri.y;
+      rr += ri.x * ri.x + ri.y * ri.y;
+    }
+    rr = block_sum<SWEEP_THREADS>(rr, red);
+    if (threadIdx.x == 0) {
+      CellState &s = cs[c];
+      norm_finish(s, 1, sqrt(rr), ra.lin_rtol);
+      done = s.ir_done;
+    }
+    __syncthreads();
+    if (done) return;
+  }
+}
+size_t refine_max_dynamic(size_t max_lds) { return max_lds > 8192 ? max_lds - 8192 : 0; }
+template <class T>
+void launch_band_refine(hipStream_t s, const CellParams *cp, CellState *cs, const RefineWG *wgs, int nwg, int max_loc,
+                        const SweepOp *ops, const SweepLoc *locs, const int *accs, const T *K, const T *Dinv,
+                        const int *kinv, const SweepVec<T> &sv, const RefineArgs &ra) {
+  if (nwg <= 0) return;
+  hipLaunchKernelGGL(k_band_refine<T>, dim3(nwg), dim3(SWEEP_THREADS), (size_t)max_loc * NB * sizeof(T), s, cp, cs,
+                     wgs, ops, locs, accs, K, Dinv, kinv, sv, ra);
 }
 template <class T>
 void launch_band_sweep(hipStream_t s, const CellParams *cp, const CellState *cs, const SweepWG *wgs, int nwg,
@@ -675,7 +781,10 @@ void launch_band_sweep(hipStream_t s, const CellParams *cp, const CellState *cs,
 
 hipError_t band_prepare_attributes(size_t max_lds) {
   const int dyn = (int)lu_solve_max_dynamic(max_lds);
-  const std::pair<const void *, int> fns[] = {{reinterpret_cast<const void *>(&k_band_sweep<float>), dyn},
+  const int ref = (int)refine_max_dynamic(max_lds);
+  const std::pair<const void *, int> fns[] = {{reinterpret_cast<const void *>(&k_band_refine<float>), ref},
+                                              {reinterpret_cast<const void *>(&k_band_refine<double>), ref},
+                                              {reinterpret_cast<const void *>(&k_band_sweep<float>), dyn},
                                               {reinterpret_cast<const void *>(&k_band_sweep<double>), dyn},
                                               {reinterpret_cast<const void *>(&k_lu_step_f64), step_lds<double>()}};
   for (const auto &f : fns) {
@@ -690,7 +799,10 @@ hipError_t band_prepare_attributes(size_t max_lds) {
                                   const BlockRef *, const FwdOp *, T *, T *, StepFwd<T>, hipEvent_t, hipEvent_t);    \
   template void launch_band_sweep<T>(hipStream_t, const CellParams *, const CellState *, const SweepWG *, int, int,  \
                                      const SweepOp *, const SweepLoc *, const int *, const T *, const T *,          \
-                                     const int *, const SweepVec<T> &, int);
+                                     const int *, const SweepVec<T> &, int);                                        \
+  template void launch_band_refine<T>(hipStream_t, const CellParams *, CellState *, const RefineWG *, int, int,      \
+                                      const SweepOp *, const SweepLoc *, const int *, const T *, const T *,         \
+                                      const int *, const SweepVec<T> &, const RefineArgs &);
 WCFE_INST(float)
 WCFE_INST(double)
 

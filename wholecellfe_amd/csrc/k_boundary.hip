@@ -17,7 +17,7 @@
 //  * node terms of the implicit Newton residual G(x) (planar, batched): one
 //    thread per node writes only its own rows of G and K, after the element
 //    assembly, so the scatter needs no colouring and no atomics.
-#include "wcfe_internal.hpp"
+#include "cell_steps.hpp"
 
 namespace wcfe {
 
@@ -280,17 +280,12 @@ void launch_cell_gdot(hipStream_t s, const CellParams *cp, const int *cells, int
 // dense cell with the area term, the rank-one coupling k g_n g_m^T to every
 // boundary vertex m of the cell) and keeps the 2 x 6 block for the FP64
 // refinement matvec.
-template <class T, bool FULL>
-__global__ __launch_bounds__(256) void k_node_terms(View v, BndView bv, const int *node_cell, int n0, int n1, T *K,
-                                                    T *Kb, const int *row_ptr, const int *bcol, const int *diag_pos,
-                                                    double *G) {
-  const int n = n0 + blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= n1) return;
-  const int c = node_cell[n];
-  const CellParams &p = v.cp[c];
-  if (!p.bterm) return;
+template <bool FULL>
+__device__ __forceinline__ double2 node_terms(const View &v, const BndView &bv, const CellParams &p, int c, int n,
+                                              double area, double (&J)[12], int2 &fr, double &cd) {
   const double2 xn = v.x[n];
-  double gx = 0.0, gy = 0.0, cd = 0.0;
+  double gx = 0.0, gy = 0.0;
+  cd = 0.0;
   if (p.bterm & BT_EXT) {  // constant load: the cell's integrin forces on a substrate (UL:467-470)
     gx -= bv.fext[2LL * n];
     gy -= bv.fext[2LL * n + 1];
@@ -302,8 +297,9 @@ __global__ __launch_bounds__(256) void k_node_terms(View v, BndView bv, const in
     gy += cd * (xn.y - Xn.y);
   }
   const int b = bv.bidx[n];
-  double J[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};  // -dF/d(x_n, x_j1, x_j2)
-  int2 fr = make_int2(-1, -1);
+#pragma unroll
+  for (int k = 0; k < 12; ++k) J[k] = 0.0;
+  fr = make_int2(-1, -1);
   if (b >= 0) {
     fr = bv.frame[b];
     if (fr.x >= 0 && (p.bterm & (BT_BEND | BT_AREA))) {
@@ -311,7 +307,7 @@ __global__ __launch_bounds__(256) void k_node_terms(View v, BndView bv, const in
       const CurveGeom g = curve_geom(P(n), P(fr.x), P(fr.y));
       double s = 0.0;
       if (p.bterm & BT_BEND) s += bend_scale(g, p.k_bend);
-      if (p.bterm & BT_AREA) s += area_scale(g, bv.area[c], p.k_area, p.area_0);
+      if (p.bterm & BT_AREA) s += area_scale(g, area, p.k_area, p.area_0);
       gx -= s * g.n[0];
       gy -= s * g.n[1];
       if (FULL) {
@@ -343,7 +339,7 @@ __global__ __launch_bounds__(256) void k_node_terms(View v, BndView bv, const in
                                      t * iL2 * dsm[m] * R[r][q]);
         }
         if (p.bterm & BT_AREA) {
-          const double h = -0.5 * p.k_area * (bv.area[c] - p.area_0);
+          const double h = -0.5 * p.k_area * (area - p.area_0);
 #pragma unroll
           for (int m = 0; m < 3; ++m)
 #pragma unroll
@@ -372,6 +368,23 @@ __global__ __launch_bounds__(256) void k_node_terms(View v, BndView bv, const in
       }
     }
   }
+  return make_double2(gx, gy);
+}
+
+template <class T, bool FULL>
+__global__ __launch_bounds__(256) void k_node_terms(View v, BndView bv, const int *node_cell, int n0, int n1, T *K,
+                                                    T *Kb, const int *row_ptr, const int *bcol, const int *diag_pos,
+                                                    double *G) {
+  const int n = n0 + blockIdx.x * blockDim.x + threadIdx.x;
+  if (n >= n1) return;
+  const int c = node_cell[n];
+  const CellParams &p = v.cp[c];
+  if (!p.bterm) return;
+  double J[12], cd;  // -dF/d(x_n, x_j1, x_j2) and the drag diagonal
+  int2 fr;
+  const double2 g = node_terms<FULL>(v, bv, p, c, n, bv.area ? bv.area[c] : 0.0, J, fr, cd);
+  const double gx = g.x, gy = g.y;
+  const int b = bv.bidx[n];
   G[2 * n] += gx;
   G[2 * n + 1] += gy;
   if (!FULL) return;
@@ -404,7 +417,7 @@ __global__ __launch_bounds__(256) void k_node_terms(View v, BndView bv, const in
       A[(r0 + r) * p.npad + cc + 1] += T(J[6 * r + 2 * m + 1]);
     }
   }
-  if (has_bnd && (p.bterm & BT_AREA)) {
+  if (has_bnd && (p.bterm & BT_AREA) && !p.smw) {
     // rank one: dG_n/dx_m += k g_n g_m^T over the cell's boundary vertices
     const double2 gn = bv.g[b];
     for (int bb = p.bnd_off; bb < p.bnd_off + p.n_bnd; ++bb) {
@@ -435,5 +448,119 @@ template void launch_node_terms<float>(hipStream_t, bool, const View &, const Bn
                                        float *, const int *, const int *, const int *, double *);
 template void launch_node_terms<double>(hipStream_t, bool, const View &, const BndView &, const int *, int, int,
                                         double *, double *, const int *, const int *, const int *, double *);
+
+// The end of a Newton step, one workgroup per cell: x += delta, the FP64
+// residual at the new positions and its norm, the Newton test, and the commit
+// of the load step if it passed.  The batch-wide kernels take eight launches
+// for it (thirteen with UL cells, two or three more with boundary forces), at
+// 4.5 us each in a captured graph whatever they do; a cell's phases need only
+// its own nodes, so a workgroup barrier stands between them.  Every sum has
+// the batch-wide kernels' order but the norm's and the area's.
+constexpr int FINISH_THREADS = 1024;
+__global__ __launch_bounds__(FINISH_THREADS) void k_cell_finish(View v, FinishArgs f, CellState *cs, const int *cells) {
+  __shared__ double red[FINISH_THREADS];
+  __shared__ int conv;
+  const int c = cells[blockIdx.x], tid = threadIdx.x;
+  const CellParams &p = v.cp[c];
+  const int n0 = p.node_off, n1 = n0 + p.n_nodes;
+  const int *elem = f.celem + p.elem_off;
+  const double2 *d2 = reinterpret_cast<const double2 *>(f.delta);
+  for (int i = n0 + tid; i < n1; i += FINISH_THREADS) {
+    double2 q = f.x[i];
+    q.x += d2[i].x;
+    q.y += d2[i].y;
+    f.x[i] = q;
+  }
+  __syncthreads();
+  for (int k = tid; k < p.n_elems; k += FINISH_THREADS) {
+    const int e = elem[k];
+    double Ge[6], Ke[36];
+    if (!element_system<false>(v, e, Ge, Ke)) cs[c].degenerate = 1;
+    double2 *g = reinterpret_cast<double2 *>(f.Ge + 6LL * e);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) g[q] = make_double2(Ge[2 * q], Ge[2 * q + 1]);
+  }
+  double area = 0.0;
+  if (p.bterm) {
+    for (int b = p.bnd_off + tid; b < p.bnd_off + p.n_bnd; b += FINISH_THREADS) {
+      int j1 = -1, j2 = -1;
+      const bool ok = curve_neighbours(Pos2{f.x}, f.bv.node[b], f.bv.cst[b], f.bv.cst[b + 1], f.bv.cand, j1, j2);
+      f.bv.frame[b] = ok ? make_int2(j1, j2) : make_int2(-1, -1);
+      f.bv.g[b] = ok ? make_double2(0.5 * (f.x[j2].y - f.x[j1].y), -0.5 * (f.x[j2].x - f.x[j1].x))
+                     : make_double2(0.0, 0.0);
+    }
+    if (p.bterm & BT_AREA) {
+      double a = 0.0;
+      for (int k = tid; k < p.n_elems; k += FINISH_THREADS) {
+        const int *t = v.el_tri + 3LL * elem[k];
+        const double2 p0 = f.x[t[0]], p1 = f.x[t[1]], p2 = f.x[t[2]];
+        a += 0.5 * fabs((p1.x - p0.x) * (p2.y - p0.y) - (p1.y - p0.y) * (p2.x - p0.x));
+      }
+      area = block_sum<FINISH_THREADS>(a, red);
+      if (tid == 0) f.bv.area[c] = area;
+    }
+  }
+  __syncthreads();
+  double gg = 0.0;
+  for (int i = n0 + tid; i < n1; i += FINISH_THREADS) {
+    double g0 = 0.0, g1 = 0.0;
+    for (int k = f.adj_start[i]; k < f.adj_start[i + 1]; ++k) {
+      const int e = f.adj[k] >> 2, a = f.adj[k] & 3;
+      g0 += f.Ge[6LL * e + 2 * a];
+      g1 += f.Ge[6LL * e + 2 * a + 1];
+    }
+    if (p.bterm) {
+      double J[12], cd;
+      int2 fr;
+      const double2 t = node_terms<false>(v, f.bv, p, c, i, area, J, fr, cd);
+      g0 += t.x;
+      g1 += t.y;
+    }
+    f.G[2 * i] = g0;
+    f.G[2 * i + 1] = g1;
+    gg += g0 * g0 + g1 * g1;
+  }
+  gg = block_sum<FINISH_THREADS>(gg, red);
+  if (tid == 0) {
+    norm_finish(cs[c], 2, sqrt(gg), -1.0);
+    newton_finish(cs[c], f.rtol, f.atol);
+    conv = cs[c].converged;
+  }
+  __syncthreads();
+  if (!conv) return;
+  if (p.law == LAW_UL) {  // strain increments and lumped masses, every node over its elements in element order
+    for (int i = n0 + tid; i < n1; i += FINISH_THREADS) {
+      double re[3] = {0.0, 0.0, 0.0}, m = 0.0;
+      for (int k = f.adj_start[i]; k < f.adj_start[i + 1]; ++k) {
+        const int e = f.adj[k] >> 2, a = f.adj[k] & 3;
+        double rea[9], mm[3];
+        element_strain(v, e, rea, mm);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) re[q] += a == 0 ? rea[q] : a == 1 ? rea[3 + q] : rea[6 + q];
+        m += a == 0 ? mm[0] : a == 1 ? mm[1] : mm[2];
+      }
+#pragma unroll
+      for (int q = 0; q < 3; ++q) f.Rea[3 * i + q] = re[q];
+      f.MM[i] = m;
+    }
+    __syncthreads();
+  }
+  const unsigned step = (unsigned)cs[c].step;
+  if (p.kinetics == KIN_BELL)
+    for (int s = p.spr_off + tid; s < p.spr_off + p.n_spr; s += FINISH_THREADS)
+      commit_spring(v, p, c, step, s, f.sp_elem, f.sp_local, f.sp_state, f.sp_anchor, f.bell);
+  for (int i = n0 + tid; i < n1; i += FINISH_THREADS)
+    commit_node(v, p, i, f.X, f.x, f.ea, f.cC, f.fau, f.Rea, f.MM, f.dt);
+  __syncthreads();  // everybody has read the step
+  if (tid == 0) {
+    cs[c].time += f.dt;
+    cs[c].step += 1;
+    cs[c].newton_it = 0;
+  }
+}
+void launch_cell_finish(hipStream_t s, const View &v, const FinishArgs &f, const int *cells, int ncell) {
+  if (ncell <= 0) return;
+  hipLaunchKernelGGL(k_cell_finish, dim3(ncell), dim3(FINISH_THREADS), 0, s, v, f, const_cast<CellState *>(v.cs), cells);
+}
 
 }  // namespace wcfe

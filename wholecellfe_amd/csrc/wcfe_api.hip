@@ -293,7 +293,6 @@ struct LuPlan {
   // dealt out by decreasing size so that every group holds big and small
   // ones); each group runs the same schedule over its own cells
   std::vector<std::vector<Stage>> grp;
-  std::vector<int> grp_cells_off, grp_ncell;  // each group's cell list in d_prefix
 
   // trailing tiles of an mt x mt block matrix: all, or the lower triangle
   static long long tiles(const CellParams &p, long long mt) { return p.sym ? mt * (mt + 1) / 2 : mt * mt; }
@@ -488,7 +487,6 @@ struct LuPlan {
     std::vector<int> order(n);
     for (int c = 0; c < n; ++c) order[c] = c;
     std::vector<StepItem> buf;
-    std::vector<int> cells_buf;
     std::vector<int2> ranges;
     auto stages = [&](const std::vector<int> &cells) {
       std::vector<Stage> st;
@@ -526,18 +524,12 @@ struct LuPlan {
       for (int c = 0; c < n; ++c) single[c] = stages({c});
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cp[a].nblk > cp[b].nblk; });
     grp.clear();
-    grp_cells_off.clear();
-    grp_ncell.clear();
     const int G = std::min(std::max(groups, 1), n);
     for (int g = 0; G > 1 && g < G; ++g) {
       std::vector<int> mine;
       for (int q = g; q < n; q += G) mine.push_back(order[q]);
       grp.push_back(stages(mine));
-      grp_cells_off.push_back((int)cells_buf.size());
-      grp_ncell.push_back((int)mine.size());
-      cells_buf.insert(cells_buf.end(), mine.begin(), mine.end());
     }
-    d_prefix = dupload(cells_buf);
     d_items = dupload(buf);
     d_ranges = dupload(ranges);
   }
@@ -595,8 +587,6 @@ struct LuPlan {
     solve_batched = add_lists(order);
     // concurrent groups
     grp.clear();
-    grp_cells_off.clear();
-    grp_ncell.clear();
     const int G = std::min(std::max(groups, 1), n);
     if (G > 1) {
       for (int g = 0; g < G; ++g) {
@@ -616,9 +606,6 @@ struct LuPlan {
           if (gs.tot > 0) st.push_back(gs);
         }
         grp.push_back(st);
-        grp_cells_off.push_back((int)buf.size());
-        grp_ncell.push_back((int)mine.size());
-        buf.insert(buf.end(), mine.begin(), mine.end());
       }
     }
     solve_single.assign(n, SolveLists{});
@@ -660,6 +647,7 @@ struct Batch {
   int nsync = 0;
   int *ipiv = nullptr;
   int *cells = nullptr;
+  int *celem = nullptr;                // per cell: its elements, in element order
   int *replica = nullptr;
   int *transitions = nullptr;
   LuPlan plan;
@@ -719,6 +707,13 @@ struct Batch {
   };
   SweepLists sweeps;                    // every cell
   std::vector<SweepLists> sweeps_cell;  // one cell's (per-cell Newton steps)
+  // cells whose refinement one workgroup runs: whole (CellParams::refine), or
+  // (tail) from the third sweep on, which few need
+  RefineWG *rwg = nullptr;
+  int nrefine = 0, refine_loc = 0;
+  std::vector<int> refine_at;  // per cell: its place in rwg, or -1
+  bool tail = false;
+  bool finish = false;  // every cell's step ends in one workgroup (k_cell_finish)
   std::vector<std::vector<int>> kpos_h;
   double *rp = nullptr, *dp = nullptr;
   bool solve_wg = false;  // static pivoting: one workgroup per cell walks its band (narrow bands)
@@ -737,7 +732,7 @@ struct Batch {
 
   void release() {
     void *ptrs[] = {X, x, fau, ea, cC, el_tri, el_cell, el_spr, sp_bary, sp_anchor, sp_state, sp_cell, sp_elem,
-                    sp_local, cp, cs, node_cell, adj_start, adj, Ge, g_start, g_col, g_bpos, g_cstart, g_ke, g_node, Ke64, G, r, delta, Rea, MM, K, Dinv, ysol, sync, ipiv, cells,
+                    sp_local, cp, cs, node_cell, adj_start, adj, Ge, g_start, g_col, g_bpos, g_cstart, g_ke, g_node, Ke64, G, r, delta, Rea, MM, K, Dinv, ysol, sync, ipiv, cells, celem, rwg,
                     replica, transitions, plan.d_prefix, row_ptr, bcol, diag_pos, el_bpos, csr_cells, chunks, Kb,
                     cgvec, cg, partials, norm_part, norm_cnt, kpos, kinv, yfwd, ysw, slots, rank, refs, fops, sops, slocs, saccs, swg, plan.d_items, plan.d_ranges, plan.d_solve, rp, dp, bt_bidx, bt_node, bt_cst, crange, bt_cand, bt_frame, bt_g, bt_J, bt_area,
                     bt_gd, bt_fext};
@@ -1035,6 +1030,36 @@ void plan_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
   }
 }
 
+// Which cells' refinement one workgroup runs whole from its first sweep
+// (k_band_refine), which from the third on, and whether one workgroup per cell
+// ends the step (k_cell_finish).
+// REFINE_OPS: the block products of the longest whole sweep up to which the
+// whole refinement in one workgroup is the faster (us per Newton step, whole
+// / spread over launches: 12 products 92 / 107, 43 FP64 206 / 222, but about
+// 240: 32 cells 629 / 541, 256 cells 1641 / 1450, where the launches' other
+// workgroups work on the same cell).
+// FINISH_BATCH: likewise elements of the batch (85 elements 92 / 97, 905
+// 206 / 211, 32 UL cells 541 / 584, but 375000: 1450 / 1412, 1.07 million
+// 4555 / 4520).
+constexpr int REFINE_OPS = 96, FINISH_BATCH = 65536;
+void choose_refine(const wcfe_ctx *ctx, Batch &b, int elem_size) {
+  for (CellParams &p : b.cp_h) p.refine = 0;
+  b.tail = false;
+  b.finish = b.T <= FINISH_BATCH;
+  for (const CellParams &p : b.cp_h) b.finish = b.finish && p.n_elems <= FINISH_ELEMS;
+  if (!b.solve_wg) return;
+  int ops = 0;
+  for (int c = 0; c < b.ncell; ++c) {
+    if (b.cp_h[c].csr) continue;
+    const SweepPart &w = b.plans[c]->whole;
+    if ((size_t)w.nloc * NB * elem_size > refine_max_dynamic(ctx->max_lds)) return;
+    ops = std::max(ops, w.nop);
+  }
+  const bool all = ops <= REFINE_OPS;
+  b.tail = !all;
+  for (CellParams &p : b.cp_h) p.refine = all && !p.csr;
+}
+
 // The band plans' tables on the device, the LU schedule and the sweeps'
 // workgroup lists.
 void upload_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
@@ -1045,6 +1070,7 @@ void upload_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
     for (int i = 0; i < p.nblk; ++i) rank.push_back(P ? P->rank[i] : i);
   }
   b.rank = dupload(rank);
+  choose_refine(ctx, b, elem_size);
   HIPCHECK(hipMemcpy(b.cp, b.cp_h.data(), sizeof(CellParams) * b.ncell, hipMemcpyHostToDevice));
   const bool planned = std::any_of(b.plans.begin(), b.plans.end(), [](const std::shared_ptr<BandPlan> &p) { return !!p; });
   bool fused = ctx->opt.fused_step > 0 && b.lu_depth == 1 && planned &&
@@ -1132,10 +1158,24 @@ void upload_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
     return S;
   };
   // longest streams first
-  std::vector<int> order(b.ncell);
+  std::vector<int> order(b.ncell), spread;
   for (int c = 0; c < b.ncell; ++c) order[c] = c;
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return b.cp_h[x].nblk > b.cp_h[y].nblk; });
-  b.sweeps = lists_of(order);
+  std::vector<RefineWG> rwg;
+  b.refine_at.assign(b.ncell, -1);
+  for (int c : order) {
+    if (b.cp_h[c].csr) continue;
+    if (!b.cp_h[c].refine) spread.push_back(c);
+    if (!b.cp_h[c].refine && !b.tail) continue;
+    const At &o = at[plans[c]];
+    auto put = [&](const SweepPart &q) { return SweepPart{q.op0 + o.op, q.nop, q.loc0 + o.loc, q.nloc}; };
+    b.refine_at[c] = (int)rwg.size();
+    rwg.push_back(RefineWG{c, put(plans[c]->whole), put(plans[c]->whole_bwd)});
+    b.refine_loc = std::max(b.refine_loc, plans[c]->whole.nloc);
+  }
+  b.nrefine = (int)rwg.size();
+  b.rwg = dupload(rwg);
+  b.sweeps = lists_of(spread);
   b.sweeps_cell.clear();
   if (!ctx->opt.batched)
     for (int c = 0; c < b.ncell; ++c) b.sweeps_cell.push_back(lists_of({c}));
@@ -1309,6 +1349,13 @@ void build_batch(wcfe_ctx *ctx, Batch &b, const std::vector<HostCell> &hc, int e
     }
   }
   b.cell_color = ranges;  // 2 entries (begin, end) per colour
+  std::vector<int> celem;
+  celem.reserve(T);
+  for (int c = 0; c < b.ncell; ++c) {
+    b.cp_h[c].elem_off = (int)celem.size();
+    for (int k = 0; k < b.ncolor; ++k)
+      for (int e = ranges[c][2 * k]; e < ranges[c][2 * k + 1]; ++e) celem.push_back(e);
+  }
   // springs: per cell, ordered by host element global id, then original index
   std::vector<int> el_spr(2 * (size_t)T, 0), sp_cell(S), sp_elem(S), sp_local(S);
   std::vector<double> sp_bary(3 * (size_t)S), sp_anchor(2 * (size_t)S), sp_state(S);
@@ -1421,6 +1468,7 @@ void build_batch(wcfe_ctx *ctx, Batch &b, const std::vector<HostCell> &hc, int e
   b.adj_start = dupload(adj_start);
   b.adj = dupload(adj);
   b.cells = dupload(ident);
+  b.celem = dupload(celem);
   b.replica = dupload(replica);
   {
     std::vector<int> kpos(N);
@@ -1495,7 +1543,7 @@ void build_batch(wcfe_ctx *ctx, Batch &b, const std::vector<HostCell> &hc, int e
     for (int c = 0; c < b.ncell; ++c) max_ndof = std::max(max_ndof, b.cp_h[c].ndof);
     if (max_ndof > NORM_CHUNK) {
       b.norm_stride = (max_ndof + NORM_CHUNK - 1) / NORM_CHUNK;
-      b.norm_part = dalloc<double>((size_t)b.ncell * b.norm_stride);
+      b.norm_part = dalloc<double>(2 * (size_t)b.ncell * b.norm_stride);
       b.norm_cnt = dalloc<unsigned>(b.ncell);
       HIPCHECK(hipMemset(b.norm_cnt, 0, sizeof(unsigned) * b.ncell));
     }
@@ -1602,6 +1650,11 @@ void build_batch(wcfe_ctx *ctx, Batch &b, const std::vector<HostCell> &hc, int e
             }
             lists[g].push_back(36 * e + 12 * a + 2 * q);
           }
+        }
+        if (cols.empty()) {  // a node of no element: its own (zero) block and residual rows
+          cols.push_back(n);
+          bps.push_back(-1);
+          if (lists.empty()) lists.emplace_back();
         }
         for (size_t g = 0; g < cols.size(); ++g) {
           P.gcol.push_back(cols[g]);
@@ -1746,11 +1799,8 @@ template <class T> StepFwd<T> step_fwd(const Batch &b) {
   return f;
 }
 
-// One refinement solve of the band plans' sweeps: forward over the leaves,
-// the separators, backward over the leaves (first: the forward part already
-// ran beside the block steps).
-template <class T>
-void enqueue_sweeps(hipStream_t s, const Batch &b, const Batch::SweepLists &L, bool first, int accumulate) {
+// The sweeps' vectors (first: the forward part's result is in yfwd).
+template <class T> SweepVec<T> sweep_vec(const Batch &b, bool first) {
   SweepVec<T> v;
   v.rhs = b.r;
   v.x = static_cast<T *>(b.ysw);
@@ -1758,6 +1808,15 @@ void enqueue_sweeps(hipStream_t s, const Batch &b, const Batch::SweepLists &L, b
   v.slot = static_cast<T *>(b.slots);
   v.delta = b.delta;
   v.from_y = first ? 1 : 0;
+  return v;
+}
+
+// One refinement solve of the band plans' sweeps: forward over the leaves,
+// the separators, backward over the leaves (first: the forward part already
+// ran beside the block steps).
+template <class T>
+void enqueue_sweeps(hipStream_t s, const Batch &b, const Batch::SweepLists &L, bool first, int accumulate) {
+  const SweepVec<T> v = sweep_vec<T>(b, first);
   auto go = [&](const Batch::SweepList &l) {
     launch_band_sweep<T>(s, b.cp, b.cs, b.swg + l.off, l.n, l.max_loc, b.sops, b.slocs, b.saccs,
                          static_cast<const T *>(b.K), static_cast<const T *>(b.Dinv), b.kinv, v, accumulate);
@@ -1774,15 +1833,12 @@ void enqueue_sweeps(hipStream_t s, const Batch &b, const Batch::SweepLists &L, b
   }
 }
 
-// Launch the LU stages of a plan for a list of cells.
+// Launch the LU stages of a plan for a list of cells (static pivoting: their
+// pivot thresholds are set).
 template <class T>
-void enqueue_lu(wcfe_ctx *ctx, hipStream_t s, const LuPlan &plan, const std::vector<Stage> &stages, const int *cells,
-                int ncell, const CellParams *cp, CellState *cs, T *K, T *Dinv, int *ipiv, const Batch *b = nullptr) {
+void enqueue_lu(wcfe_ctx *ctx, hipStream_t s, const LuPlan &plan, const std::vector<Stage> &stages,
+                const CellParams *cp, CellState *cs, T *K, T *Dinv, int *ipiv, const Batch *b = nullptr) {
   const bool piv = plan.pivoting != 0;
-  {
-    PhaseScope ph(ctx, WCFE_PH_LU_PANEL);
-    if (!piv) launch_diag_tau<T>(s, cp, cs, cells, ncell, K);
-  }
   for (const Stage &g : stages) {
     const WorkList wl{plan.d_prefix + g.off, g.tot};
     switch (g.kind) {
@@ -1851,14 +1907,13 @@ template <class T> void enqueue_factor(wcfe_ctx *ctx, Batch &b, const Scope &sc)
     for (size_t g = 0; g < b.plan.grp.size(); ++g) {
       hipStream_t gs = ctx->side[g];
       HIPCHECK(hipStreamWaitEvent(gs, ctx->fork_ev, 0));
-      enqueue_lu<T>(ctx, gs, b.plan, b.plan.grp[g], b.plan.d_prefix + b.plan.grp_cells_off[g], b.plan.grp_ncell[g],
-                    b.cp, b.cs, static_cast<T *>(b.K), static_cast<T *>(b.Dinv), b.ipiv, &b);
+      enqueue_lu<T>(ctx, gs, b.plan, b.plan.grp[g], b.cp, b.cs, static_cast<T *>(b.K), static_cast<T *>(b.Dinv), b.ipiv, &b);
       HIPCHECK(hipEventRecord(ctx->join_ev[g], gs));
       HIPCHECK(hipStreamWaitEvent(ctx->stream, ctx->join_ev[g], 0));
     }
   } else {
-    enqueue_lu<T>(ctx, ctx->stream, b.plan, stages, sc.cells, sc.ncell, b.cp, b.cs, static_cast<T *>(b.K),
-                  static_cast<T *>(b.Dinv), b.ipiv, &b);
+    enqueue_lu<T>(ctx, ctx->stream, b.plan, stages, b.cp, b.cs, static_cast<T *>(b.K), static_cast<T *>(b.Dinv),
+                  b.ipiv, &b);
   }
   const int *cl;
   int cb, nch, ncl;
@@ -1945,13 +2000,31 @@ template <class T> void enqueue_solve_refine(wcfe_ctx *ctx, Batch &b, const Scop
   View v = make_view(ctx, b);
   const int piv = ctx->opt.pivoting == WCFE_PIVOT_PARTIAL;
   const long long v0 = 2LL * sc.node_begin, vn = 2LL * (sc.node_end - sc.node_begin);
+  const bool one_wg = sc.cell < 0 ? b.nrefine > 0 : b.solve_wg && b.refine_at[sc.cell] >= 0;
   {
     PhaseScope ph(ctx, WCFE_PH_REFINE);
-    launch_ir_control(s, b.cs, sc.cells, sc.ncell, ctx->opt.lin_rtol, 1);
-    launch_neg_copy(s, b.G + v0, b.r + v0, vn);
+    // the fused block steps and the one-workgroup refinement read G themselves
+    if (b.any_csr || !(b.solve_wg && (b.plan.fused || (one_wg && !b.tail)))) launch_neg_copy(s, b.G + v0, b.r + v0, vn);
+  }
+  const int max_refine = std::max(1, ctx->opt.max_refine);
+  auto refine = [&](int it0) {
+    PhaseScope ph(ctx, WCFE_PH_SOLVE);
+    launch_band_refine<T>(s, b.cp, b.cs, b.rwg + (sc.cell < 0 ? 0 : b.refine_at[sc.cell]),
+                          sc.cell < 0 ? b.nrefine : 1, b.refine_loc, b.sops, b.slocs, b.saccs, K,
+                          static_cast<const T *>(b.Dinv), b.kinv, sweep_vec<T>(b, b.plan.fused),
+                          RefineArgs{b.el_tri, b.adj_start, b.adj, b.Ke64, b.G, b.r, b.delta, b.rp, b.dp,
+                                     bnd_view(ctx, b), ctx->opt.lin_rtol, it0, max_refine, b.plan.fused ? 1 : 0});
+  };
+  if (one_wg && !b.tail) {
+    refine(0);
+    if (!b.any_csr) return;
   }
   const int npad = sc.cell < 0 ? b.max_npad : b.cp_h[sc.cell].npad;
-  for (int it = 0; it < std::max(1, ctx->opt.max_refine); ++it) {
+  for (int it = 0; it < max_refine; ++it) {
+    if (one_wg && b.tail && it == 2 && !b.any_csr) {
+      refine(2);
+      break;
+    }
     {
       PhaseScope ph(ctx, WCFE_PH_SOLVE);
       if (piv) {
@@ -1978,12 +2051,12 @@ template <class T> void enqueue_solve_refine(wcfe_ctx *ctx, Batch &b, const Scop
     if (b.any_area) launch_cell_gdot(s, b.cp, sc.cells, sc.ncell, bv, b.delta);
     launch_matvec_ir(s, v, b.node_cell, b.adj_start, b.adj, b.Ke64, b.G, b.delta, b.r, sc.node_begin, sc.node_end,
                      b.cs, bv);
-    launch_cell_norm(s, b.cp, b.cs, sc.cells, sc.ncell, b.r, 1, 1, ctx->opt.lin_rtol, b.norm_work());
+    launch_cell_norm<T>(s, b.cp, b.cs, sc.cells, sc.ncell, b.r, 1, 1, ctx->opt.lin_rtol, b.norm_work());
     // a batch with sparse cells is not captured (its solves check their
     // convergence on the host): from the second sweep on, stop once every
     // cell of the scope has met lin_rtol -- the sweeps left would launch
     // only idle kernels (and a solve's probing iteration)
-    if (b.any_csr && it >= 1 && it + 1 < std::max(1, ctx->opt.max_refine)) {
+    if (b.any_csr && it >= 1 && it + 1 < max_refine) {
       std::vector<CellState> h(b.ncell);
       HIPCHECK(hipMemcpyAsync(h.data(), b.cs, sizeof(CellState) * b.ncell, hipMemcpyDeviceToHost, s));
       HIPCHECK(hipStreamSynchronize(s));
@@ -2009,24 +2082,36 @@ template <class T> void enqueue_newton(wcfe_ctx *ctx, Batch &b, const Scope &sc)
       const long long bb = sc.cell < 0 ? 0 : b.blk_begin_h[sc.cell], be = sc.cell < 0 ? b.nnzb : b.blk_end_h[sc.cell];
       launch_zero<T>(s, static_cast<T *>(b.Kb) + 4 * bb, 4 * (be - bb));
     }
-    launch_fill(s, b.G + v0, vn, 0.0);
+    if (sc.cell >= 0) launch_fill(s, b.G + v0, vn, 0.0);  // the whole-batch gather writes every entry
   }
   {
     PhaseScope ph(ctx, WCFE_PH_ASSEMBLE, sc.cell < 0 ? b.T : b.cp_h[sc.cell].n_elems);
     enqueue_assemble<T>(ctx, b, sc, ASM_FULL);
-    launch_cell_norm(s, b.cp, b.cs, sc.cells, sc.ncell, b.G, 0, 0, -1.0, b.norm_work());
+    launch_cell_norm<T>(s, b.cp, b.cs, sc.cells, sc.ncell, b.G, 0, 0, -1.0, b.norm_work(),
+                        ctx->opt.pivoting == WCFE_PIVOT_STATIC ? K : nullptr);
   }
   // 2. factor
   enqueue_factor<T>(ctx, b, sc);
   // 3. solve K d = -G with FP64 refinement
   enqueue_solve_refine<T>(ctx, b, sc);
+  const BellArgs bell{ctx->opt.dt,      ctx->opt.k_on,    ctx->opt.k_off0, ctx->opt.f_bell,
+                      ctx->opt.seed_lo, ctx->opt.seed_hi, b.replica,       b.transitions};
+  if (b.finish) {
+    PhaseScope ph(ctx, WCFE_PH_RESIDUAL);
+    launch_cell_finish(s, make_view(ctx, b),
+                       FinishArgs{b.X, b.x, b.fau, b.ea, b.cC, b.Ge, b.G, b.Rea, b.MM, b.sp_state, b.sp_anchor,
+                                  b.delta, b.celem, b.adj_start, b.adj, b.sp_elem, b.sp_local, bnd_view(ctx, b), bell,
+                                  ctx->opt.newton_rtol, ctx->opt.newton_atol, ctx->opt.dt},
+                       sc.cells, sc.ncell);
+    return;
+  }
   // 4. x += d, FP64 residual at the new x, convergence test
   {
     PhaseScope ph(ctx, WCFE_PH_RESIDUAL);
     launch_update_x(s, b.x, b.delta, sc.node_begin, sc.node_end);
-    launch_fill(s, b.G + v0, vn, 0.0);
+    if (sc.cell >= 0) launch_fill(s, b.G + v0, vn, 0.0);
     enqueue_assemble<T>(ctx, b, sc, ASM_RESIDUAL);
-    launch_cell_norm(s, b.cp, b.cs, sc.cells, sc.ncell, b.G, 2, 0, -1.0, b.norm_work());
+    launch_cell_norm<T>(s, b.cp, b.cs, sc.cells, sc.ncell, b.G, 2, 0, -1.0, b.norm_work());
     launch_newton_control(s, b.cs, sc.cells, sc.ncell, ctx->opt.newton_rtol, ctx->opt.newton_atol);
   }
   // 5. commit converged cells
@@ -2043,8 +2128,7 @@ template <class T> void enqueue_newton(wcfe_ctx *ctx, Batch &b, const Scope &sc)
   const bool any_bell = sc.cell < 0 ? b.any_bell : (b.cp_h[sc.cell].kinetics == KIN_BELL);
   if (any_bell)
     launch_commit_springs(s, v, b.sp_cell, b.sp_elem, b.sp_local, b.sp_state, b.sp_anchor, sc.spr_begin, sc.spr_end,
-                          ctx->opt.dt, ctx->opt.k_on, ctx->opt.k_off0, ctx->opt.f_bell, ctx->opt.seed_lo,
-                          ctx->opt.seed_hi, b.replica, b.transitions);
+                          bell);
   launch_commit_cells(s, b.cs, sc.cells, sc.ncell, ctx->opt.dt);
 }
 
@@ -3196,10 +3280,9 @@ void dense_solve_impl(wcfe_ctx *ctx, int n_sys, const int32_t *n, const double *
   plan.build(cp, ctx->opt.pivoting, 1, ctx->opt.lu_depth > 0 ? ctx->opt.lu_depth : 4);  // full matrices
   sc.ptrs.push_back(plan.d_prefix);
   const bool piv = ctx->opt.pivoting == WCFE_PIVOT_PARTIAL;
-  enqueue_lu<T>(ctx, ctx->stream, plan, plan.batched, dcells, n_sys, dcp, dcs, dK, dDinv, dipiv);
   // refinement: r = b; repeat { d = LU^-1 r; x += d; r = b - A x (FP64) }
-  launch_cell_norm(s, dcp, dcs, dcells, n_sys, db, 0, 0);
-  launch_ir_control(s, dcs, dcells, n_sys, ctx->opt.lin_rtol, 1);
+  launch_cell_norm<T>(s, dcp, dcs, dcells, n_sys, db, 0, 0, -1.0, NormWork(), piv ? nullptr : dK);
+  enqueue_lu<T>(ctx, ctx->stream, plan, plan.batched, dcp, dcs, dK, dDinv, dipiv);
   HIPCHECK(hipMemcpyAsync(dr, db, sizeof(double) * vo, hipMemcpyDeviceToDevice, s));
   unsigned char *dy = sc.zeros<unsigned char>(lu_solve_exchange_bytes(std::max(sys, 1), sizeof(T)));
   int *dsync = sc.zeros<int>((size_t)SOLVE_SYNC_INTS);
@@ -3212,7 +3295,7 @@ void dense_solve_impl(wcfe_ctx *ctx, int n_sys, const int32_t *n, const double *
                             WorkList{plan.d_prefix + plan.solve_batched.bwd_off, plan.solve_batched.tot}, dK, dDinv,
                             dr, dx, dy, dsync, it > 0);
     launch_dense_residual(s, dcp, dcs, dcells, n_sys, max_npad, dA, dAoff, db, dx, dr);
-    launch_cell_norm(s, dcp, dcs, dcells, n_sys, dr, 1, 1, ctx->opt.lin_rtol);
+    launch_cell_norm<T>(s, dcp, dcs, dcells, n_sys, dr, 1, 1, ctx->opt.lin_rtol);
   }
   HIPCHECK(hipGetLastError());
   HIPCHECK(hipStreamSynchronize(s));
@@ -3395,7 +3478,6 @@ int wcfe_calculate_res(wcfe_ctx *ctx, int32_t n_nodes, int32_t n_tris, const int
       cs.converged = 1;
       HIPCHECK(hipMemcpy(tb.cs, &cs, sizeof cs, hipMemcpyHostToDevice));
       Scope sc = scope_all(tb);
-      launch_fill(ctx->stream, tb.G, 2LL * n_nodes, 0.0);
       enqueue_assemble<double>(ctx, tb, sc, ASM_RESIDUAL);
       launch_fill(ctx->stream, tb.Rea, 3LL * n_nodes, 0.0);
       launch_fill(ctx->stream, tb.MM, n_nodes, 0.0);

@@ -37,6 +37,9 @@ struct CellParams {
   int env;                        // blocks |i - j| <= env are zeroed before assembly (bw + delayed
                                   // panels - 1: the trailing update reads that far off the band)
   int passive;                    // 1: no active stress (the reference's substrate, mat = 2)
+  int refine;                     // 1: one workgroup runs the cell's whole refinement (k_band_refine)
+  int smw;                        // 1: the area term's rank-one part is left out of the (band) system and
+                                  //    comes back in the solves (Sherman-Morrison)
   int slot_off;                   // band plan: the cell's 64-entry slots of the forward sweeps
   int rank_off;                   // band plan: its blocks' places in the elimination order
   long long k_off;                // offset of the dense matrix (elements)

@@ -42,7 +42,7 @@ struct GatherPlan {
 template <class T>
 void launch_assemble_gather(hipStream_t s, const View &v, int e_begin, int e_end, int mode, const int *node_cell,
                             const int *adj_start, const int *adj, const GatherPlan &gp, int n0, int n1, double *Ge,
-                            double *Ke64, double *G, T *K, T *Kb, int lower_only = 0);
+                            double *Ke64, double *G, T *K, T *Kb, int lower_only);
 void launch_element_dump(hipStream_t s, const View &v, int e_begin, int e_end, double *Ge, double *Ke);
 // per-cell norms of cells above NORM_CHUNK entries: partial sums per chunk
 // (stride per cell = the batch's largest chunk count) and an arrival counter
@@ -53,16 +53,18 @@ struct NormWork {
   unsigned *cnt = nullptr;
   int stride = 1;
 };
-// which 1 with lin_rtol >= 0 also applies the refinement control to each
-// refining cell (as launch_ir_control with reset 0)
+// which 0 also starts a new linear solve (the refinement state), and with K
+// takes the dense cells' pivot thresholds from its diagonal (64 units of
+// roundoff of T times the largest entry); which 1 with lin_rtol >= 0 applies
+// the refinement control to each refining cell
+template <class T>
 void launch_cell_norm(hipStream_t s, const CellParams *cp, CellState *cs, const int *cells, int ncell,
                       const double *vec, int which, int only_active, double lin_rtol = -1.0,
-                      const NormWork &nw = NormWork());
+                      const NormWork &nw = NormWork(), const T *K = nullptr);
 void launch_neg_copy(hipStream_t s, const double *src, double *dst, long long n);
 void launch_matvec_ir(hipStream_t s, const View &v, const int *node_cell, const int *adj_start, const int *adj,
                       const double *Ke64, const double *G, const double *delta, double *r, int node_begin,
                       int node_end, const CellState *cs, const BndView &bv);
-void launch_ir_control(hipStream_t s, CellState *cs, const int *cells, int ncell, double lin_rtol, int reset);
 void launch_perm_gather(hipStream_t s, const int *node_cell, const CellParams *cp, const int *kpos, const double *r,
                         double *rp, int n0, int n1);
 void launch_perm_scatter(hipStream_t s, const int *node_cell, const CellParams *cp, const CellState *cs,
@@ -72,16 +74,19 @@ void launch_newton_control(hipStream_t s, CellState *cs, const int *cells, int n
 void launch_commit_nodes(hipStream_t s, const View &v, const int *node_cell, double2 *X, double2 *x, double *ea,
                          double *cC, double2 *fau, const double *Rea, const double *MM, int node_begin, int node_end,
                          double dt);
+// Bell kinetics of the springs (k_commit_springs)
+struct BellArgs {
+  double dt, k_on, k_off0, f_b;
+  unsigned key_lo, key_hi;
+  const int *replica;  // per cell: its Philox stream
+  int *transitions;
+};
 void launch_commit_springs(hipStream_t s, const View &v, const int *sp_cell, const int *sp_elem, const int *sp_local,
-                           double *state, double *anchor, int s_begin, int s_end, double dt, double k_on,
-                           double k_off0, double f_b, unsigned key_lo, unsigned key_hi, const int *replica_of_cell,
-                           int *transitions);
+                           double *state, double *anchor, int s_begin, int s_end, const BellArgs &bell);
 void launch_commit_cells(hipStream_t s, CellState *cs, const int *cells, int ncell, double dt);
 void launch_remap_nodes(hipStream_t s, int n_new, const int *src0, const int *src1, const double *w, int old_off,
                         const double2 *X, const double2 *x, const double *ea, const double *cC, const double2 *fau,
                         double2 *Xn, double2 *xn, double *ean, double *cCn, double2 *faun);
-template <class T>
-void launch_diag_tau(hipStream_t s, const CellParams *cp, CellState *cs, const int *cells, int ncell, const T *K);
 
 // ---- boundary and body forces (k_boundary.hip) ----
 enum : int { REF_BEND = 0, REF_AREA = 1, REF_AP = 2 };
@@ -101,6 +106,20 @@ void launch_cell_gdot(hipStream_t s, const CellParams *cp, const int *cells, int
 template <class T>
 void launch_node_terms(hipStream_t s, bool full, const View &v, const BndView &bv, const int *node_cell, int n0, int n1,
                        T *K, T *Kb, const int *row_ptr, const int *bcol, const int *diag_pos, double *G);
+// the end of a Newton step with one workgroup per cell: x += delta, the FP64
+// residual and its norm, the Newton test and the commit of a converged cell
+constexpr int FINISH_ELEMS = 12000;  // most elements of a cell (larger ones run the batch-wide kernels)
+struct FinishArgs {
+  double2 *X, *x, *fau;
+  double *ea, *cC, *Ge, *G, *Rea, *MM, *sp_state, *sp_anchor;
+  const double *delta;
+  const int *celem;  // every cell's elements (elem_off), in element order
+  const int *adj_start, *adj, *sp_elem, *sp_local;
+  BndView bv;
+  BellArgs bell;
+  double rtol, atol, dt;
+};
+void launch_cell_finish(hipStream_t s, const View &v, const FinishArgs &f, const int *cells, int ncell);
 
 // ---- dense LU and triangular solves (k_lu.hip) ----
 // Dinv holds, per cell and diagonal block, the inverses of the block's unit
@@ -180,6 +199,27 @@ template <class T>
 void launch_band_sweep(hipStream_t s, const CellParams *cp, const CellState *cs, const SweepWG *wgs, int nwg,
                        int max_loc, const SweepOp *ops, const SweepLoc *locs, const int *accs, const T *K,
                        const T *Dinv, const int *kinv, const SweepVec<T> &sv, int accumulate);
+// refinement sweeps it0 .. max_refine - 1 of a cell by one workgroup (solve,
+// FP64 residual, norm and control); parts: the cell's whole sweep and its
+// backward half (the first solve after the fused block steps); z, inc: batch
+// vectors for cells with smw
+struct RefineWG {
+  int cell;
+  SweepPart whole, bwd;
+};
+struct RefineArgs {
+  const int *el_tri, *adj_start, *adj;
+  const double *Ke64, *G;
+  double *r, *delta, *z, *inc;
+  BndView bv;
+  double lin_rtol;
+  int it0, max_refine, fwd_done;
+};
+size_t refine_max_dynamic(size_t max_lds);
+template <class T>
+void launch_band_refine(hipStream_t s, const CellParams *cp, CellState *cs, const RefineWG *wgs, int nwg, int max_loc,
+                        const SweepOp *ops, const SweepLoc *locs, const int *accs, const T *K, const T *Dinv,
+                        const int *kinv, const SweepVec<T> &sv, const RefineArgs &ra);
 hipError_t band_prepare_attributes(size_t max_lds);
 
 // ---- sparse path: block-CSR systems and batched PCG (k_csr.hip) ----
