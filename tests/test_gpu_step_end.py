@@ -43,3 +43,29 @@ def test_cell_alone_equals_cell_in_a_large_batch(kind, lin_rtol, prec):
         assert np.linalg.norm(a[0] - b[0]) <= 1e-6 * move
         for p, q in zip(a[1:], b[1:]):
             assert np.abs(p - q).max() <= 1e-6 * max(1.0, np.abs(q).max())
+
+
+# K = 1: one block (no band); 2 and more: the band with the area term's rank
+# one added by Sherman-Morrison, against the full matrix with row pivoting
+@pytest.mark.parametrize("prec", [W.PREC_MIXED, W.PREC_FP64])
+@pytest.mark.parametrize("K", [1, 2, 5, 11])
+def test_area_term_in_the_band_equals_the_full_matrix(K, prec):
+    print("case area", K, prec, flush=True)
+    d = cells.ul_cell(K=K, seed=K)
+    out = []
+    for piv in (W.PIVOT_STATIC, W.PIVOT_PARTIAL):
+        with W.Context(precision=prec, t0=1.0, lin_rtol=1e-12, max_refine=8, pivoting=piv) as c:
+            c.set_table(0, d["tab_px"], d["tab_py"], d["tab_k"])
+            c.add_cell(X=d["X"], x=d["x"], tris=d["tris"], law=d["law"], mu=d["mu"], thick=d["thick"], ea=d["ea"],
+                       node_springs=1, cC=d["cC"], fau=d["fau0"], rho_max=d["rho_max"], spring_law=1,
+                       kinetics=W.KIN_MEANFIELD, k_bend=W.K_BEND_REF, k_area=W.K_AREA_REF, drag=W.DRAG_REF)
+            c.finalize()
+            Kmat = c.assembled_system(0)[0]
+            for _ in range(3):
+                c.newton_step(stats=False)
+            c.synchronize()
+            out.append((c.positions(0), Kmat))
+    (xs, Ks), (xf, Kf) = out
+    assert np.abs(Ks - Kf).max() <= 1e-12 * np.abs(Kf).max()  # the same sums, rounded alike
+    # relative residual 1e-12 at a condition number below 1e6
+    assert np.linalg.norm(xs - xf) <= 1e-6 * np.linalg.norm(xf - np.asarray(d["x"]).ravel())

@@ -678,7 +678,8 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_band_sweep(const CellParams *
 // rank one left out, g = dA/dx on the boundary), and K d = r is solved as
 // d = y - z (g.y) / (1 + g.z) with y = B^-1 r, z = B^-1 k g (Sherman and
 // Morrison 1950), the dots in FP64; the residual is the full K's.  The full
-// matrix is dense (the boundary couples to itself): n^3 instead of n bw^2.
+// matrix is dense (the boundary couples to itself): n^3 instead of n bw^2
+// (905 elements, load step of two to three Newton steps: 1600 -> 610 us).
 template <class T>
 __global__ __launch_bounds__(SWEEP_THREADS) void k_band_refine(const CellParams *cp, CellState *cs,
                                                                const RefineWG *wgs, const SweepOp *ops,
@@ -707,21 +708,35 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_band_refine(const CellParams 
   };
   double den = 1.0;
   if (p.smw) {
-    for (int i = n0 + threadIdx.x; i < n1; i += SWEEP_THREADS) {
-      const int b = ra.bv.bidx[i];
-      const bool on = b >= 0 && ra.bv.frame[b].x >= 0;
-      const double2 g = on ? ra.bv.g[b] : make_double2(0.0, 0.0);
-      ra.inc[2 * i] = p.k_area * g.x;
-      ra.inc[2 * i + 1] = p.k_area * g.y;
+    // z from the factors of B, and while k g.B^-1 g is large again from its
+    // FP64 residual k g - B z: an error e of z leaves K e (g.y) / (1 + g.z) in
+    // the residual, and the area term makes K e large
+    double gz = 0.0;
+    for (int t = 0; t < 3; ++t) {
+      for (int i = n0 + threadIdx.x; i < n1; i += SWEEP_THREADS) {
+        const int b = ra.bv.bidx[i];
+        const bool on = b >= 0 && ra.bv.frame[b].x >= 0;
+        const double2 g = on ? ra.bv.g[b] : make_double2(0.0, 0.0);
+        double2 q = make_double2(p.k_area * g.x, p.k_area * g.y);
+        if (t > 0) {
+          const double2 ri = residual_node(i, c, ra.el_tri, ra.adj_start, ra.adj, ra.Ke64, ra.G, ra.z, p, ra.bv, 0.0);
+          q.x += ri.x + ra.G[2 * i];
+          q.y += ri.y + ra.G[2 * i + 1];
+        }
+        ra.inc[2 * i] = q.x;
+        ra.inc[2 * i + 1] = q.y;
+      }
+      __syncthreads();
+      SweepVec<T> v = sv;
+      v.rhs = ra.inc;
+      v.delta = ra.z;
+      v.from_y = 0;
+      sweep_part<T>(p, wg.whole, ops, locs, accs, K, Dinv, kinv, v, t > 0, y, rowb);
+      __syncthreads();
+      gz = gdot(ra.z);
+      if (!(fabs(gz) > 16.0)) break;
     }
-    __syncthreads();
-    SweepVec<T> v = sv;
-    v.rhs = ra.inc;
-    v.delta = ra.z;
-    v.from_y = 0;
-    sweep_part<T>(p, wg.whole, ops, locs, accs, K, Dinv, kinv, v, 0, y, rowb);
-    __syncthreads();
-    den = 1.0 + gdot(ra.z);
+    den = 1.0 + gz;
   }
   if (ra.it0 == 0 && !ra.fwd_done) {
     for (int i = 2 * n0 + threadIdx.x; i < 2 * n1; i += SWEEP_THREADS) ra.r[i] = -ra.G[i];

@@ -707,10 +707,10 @@ struct Batch {
   };
   SweepLists sweeps;                    // every cell
   std::vector<SweepLists> sweeps_cell;  // one cell's (per-cell Newton steps)
-  // cells whose refinement one workgroup runs: whole (CellParams::refine), or
-  // (tail) from the third sweep on, which few need
+  // cells whose refinement one workgroup runs: whole (CellParams::refine), then
+  // (tail) those of which it runs the sweeps after the second, which few need
   RefineWG *rwg = nullptr;
-  int nrefine = 0, refine_loc = 0;
+  int nrefine = 0, ntail = 0, refine_loc = 0;
   std::vector<int> refine_at;  // per cell: its place in rwg, or -1
   bool tail = false;
   bool finish = false;  // every cell's step ends in one workgroup (k_cell_finish)
@@ -724,7 +724,7 @@ struct Batch {
   int lu_depth = 4, lu_groups = 4;  // the LU schedule in effect (options, or their automatic choice)
   int max_bw = 0;                    // widest block band of the dense cells
   // boundary and body forces (cells with bterm != 0)
-  int any_bterm = 0, any_area = 0, nbnd = 0;
+  int any_bterm = 0, any_area = 0, any_gdot = 0, nbnd = 0;  // any_gdot: area cells without smw
   int *bt_bidx = nullptr, *bt_node = nullptr, *bt_cst = nullptr, *crange = nullptr;
   int2 *bt_cand = nullptr, *bt_frame = nullptr;
   double2 *bt_g = nullptr;
@@ -1043,21 +1043,19 @@ void plan_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
 // 4555 / 4520).
 constexpr int REFINE_OPS = 96, FINISH_BATCH = 65536;
 void choose_refine(const wcfe_ctx *ctx, Batch &b, int elem_size) {
-  for (CellParams &p : b.cp_h) p.refine = 0;
-  b.tail = false;
   b.finish = b.T <= FINISH_BATCH;
   for (const CellParams &p : b.cp_h) b.finish = b.finish && p.n_elems <= FINISH_ELEMS;
-  if (!b.solve_wg) return;
+  bool fits = b.solve_wg;
   int ops = 0;
-  for (int c = 0; c < b.ncell; ++c) {
-    if (b.cp_h[c].csr) continue;
+  for (int c = 0; c < b.ncell && fits; ++c) {
+    if (b.cp_h[c].csr || !b.plans[c]) continue;
     const SweepPart &w = b.plans[c]->whole;
-    if ((size_t)w.nloc * NB * elem_size > refine_max_dynamic(ctx->max_lds)) return;
+    fits = (size_t)w.nloc * NB * elem_size <= refine_max_dynamic(ctx->max_lds);
     ops = std::max(ops, w.nop);
   }
-  const bool all = ops <= REFINE_OPS;
-  b.tail = !all;
-  for (CellParams &p : b.cp_h) p.refine = all && !p.csr;
+  const bool all = fits && ops <= REFINE_OPS;
+  b.tail = fits && !all;
+  for (CellParams &p : b.cp_h) p.refine = !p.csr && (all || p.smw);
 }
 
 // The band plans' tables on the device, the LU schedule and the sweeps'
@@ -1164,16 +1162,21 @@ void upload_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
   std::vector<RefineWG> rwg;
   b.refine_at.assign(b.ncell, -1);
   for (int c : order) {
-    if (b.cp_h[c].csr) continue;
-    if (!b.cp_h[c].refine) spread.push_back(c);
-    if (!b.cp_h[c].refine && !b.tail) continue;
+    if (!b.cp_h[c].csr && !b.cp_h[c].refine) spread.push_back(c);
+  }
+  auto one_wg = [&](int c) {
     const At &o = at[plans[c]];
     auto put = [&](const SweepPart &q) { return SweepPart{q.op0 + o.op, q.nop, q.loc0 + o.loc, q.nloc}; };
     b.refine_at[c] = (int)rwg.size();
     rwg.push_back(RefineWG{c, put(plans[c]->whole), put(plans[c]->whole_bwd)});
     b.refine_loc = std::max(b.refine_loc, plans[c]->whole.nloc);
-  }
+  };
+  for (int c : order)
+    if (b.cp_h[c].refine) one_wg(c);
   b.nrefine = (int)rwg.size();
+  if (b.tail)
+    for (int c : spread) one_wg(c);
+  b.ntail = (int)rwg.size() - b.nrefine;
   b.rwg = dupload(rwg);
   b.sweeps = lists_of(spread);
   b.sweeps_cell.clear();
@@ -1259,46 +1262,59 @@ void build_batch(wcfe_ctx *ctx, Batch &b, const std::vector<HostCell> &hc, int e
   b.kpool = kp;
   // dense cells under static pivoting: a band-reducing node numbering (RCM
   // when it narrows the band) and the LU restricted to the band; partial
-  // pivoting (row swaps widen the band), the area term (rank-one coupling of
-  // the whole boundary) and ctx->opt.band == 0 keep the natural numbering and
-  // the full matrix
+  // pivoting (row swaps widen the band) and ctx->opt.band == 0 keep the natural
+  // numbering and the full matrix.  The area term couples the whole boundary,
+  // by a matrix of rank one: area cells get the band without it
+  // (k_band_refine adds it by Sherman-Morrison) where every cell's sweeps run
+  // in one workgroup, else the full matrix.
   b.kpos_h.assign(b.ncell, {});
-  parallel_cells(b.ncell, [&](int c) {
-    CellParams &p = b.cp_h[c];
-    const HostCell &h = hc[c];
-    std::vector<int> ident(h.n_nodes);
-    for (int i = 0; i < h.n_nodes; ++i) ident[i] = i;
-    const int full = std::max(p.nblk - 1, 0);
-    p.bw = full;
-    b.kpos_h[c] = ident;
-    if (!p.csr && ctx->opt.band && ctx->opt.pivoting == WCFE_PIVOT_STATIC && !(p.bterm & BT_AREA) && p.nblk > 1) {
-      if (h.bw_rcm < 0 || h.rcm_hash != h.topo_hash || (int)h.rcm_pos.size() != h.n_nodes) {  // once per mesh
-        h.bw_nat = block_bandwidth(h.n_tris, h.tris.data(), ident);
-        h.rcm_pos = rcm_positions(h.n_nodes, h.n_tris, h.tris.data());
-        h.bw_rcm = block_bandwidth(h.n_tris, h.tris.data(), h.rcm_pos);
-        h.rcm_hash = h.topo_hash;
-      }
-      if (h.bw_rcm < h.bw_nat) {
-        b.kpos_h[c] = h.rcm_pos;
-        p.bw = std::min(full, h.bw_rcm);
-      } else {
-        p.bw = std::min(full, h.bw_nat);
-      }
-    }
-  });
-  // automatic LU schedule: narrow bands are latency bound (one block step per
-  // round, one stream); wide or full matrices are throughput bound (delayed
-  // updates over 4 block steps, 4 concurrent cell groups)
   bool narrow = true;
+  auto number = [&](bool area_band) {
+    parallel_cells(b.ncell, [&](int c) {
+      CellParams &p = b.cp_h[c];
+      const HostCell &h = hc[c];
+      std::vector<int> ident(h.n_nodes);
+      for (int i = 0; i < h.n_nodes; ++i) ident[i] = i;
+      const int full = std::max(p.nblk - 1, 0);
+      p.bw = full;
+      p.smw = 0;
+      b.kpos_h[c] = ident;
+      const bool area = (p.bterm & BT_AREA) != 0;
+      if (!p.csr && ctx->opt.band && ctx->opt.pivoting == WCFE_PIVOT_STATIC && (!area || area_band) && p.nblk > 1) {
+        p.smw = area;
+        if (h.bw_rcm < 0 || h.rcm_hash != h.topo_hash || (int)h.rcm_pos.size() != h.n_nodes) {  // once per mesh
+          h.bw_nat = block_bandwidth(h.n_tris, h.tris.data(), ident);
+          h.rcm_pos = rcm_positions(h.n_nodes, h.n_tris, h.tris.data());
+          h.bw_rcm = block_bandwidth(h.n_tris, h.tris.data(), h.rcm_pos);
+          h.rcm_hash = h.topo_hash;
+        }
+        if (h.bw_rcm < h.bw_nat) {
+          b.kpos_h[c] = h.rcm_pos;
+          p.bw = std::min(full, h.bw_rcm);
+        } else {
+          p.bw = std::min(full, h.bw_nat);
+        }
+      }
+    });
+    // automatic LU schedule: narrow bands are latency bound (one block step per
+    // round, one stream); wide or full matrices are throughput bound (delayed
+    // updates over 4 block steps, 4 concurrent cell groups)
+    narrow = true;
+    for (const CellParams &p : b.cp_h)
+      if (!p.csr && p.bw > SOLVE_WG_MAX_BW) narrow = false;
+    b.lu_depth = ctx->opt.lu_depth > 0 ? ctx->opt.lu_depth : (narrow ? 1 : 4);
+    b.lu_groups = ctx->opt.lu_groups > 0 ? ctx->opt.lu_groups : (narrow ? 1 : AUTO_GROUPS_MAX);
+    // narrow bands: one workgroup per cell runs each triangular sweep (no
+    // cross-workgroup hops); otherwise the block rows of all cells are spread
+    // over workgroups (k_lu_solve_mw)
+    b.solve_wg = ctx->opt.pivoting == WCFE_PIVOT_STATIC && narrow && b.max_npad > 0 &&
+                 lu_solve_lds_bytes(b.max_npad, elem_size) <= lu_solve_max_dynamic(ctx->max_lds);
+  };
+  number(true);
+  bool whole = b.solve_wg;  // every area cell's refinement fits one workgroup
   for (const CellParams &p : b.cp_h)
-    if (!p.csr && p.bw > SOLVE_WG_MAX_BW) narrow = false;
-  b.lu_depth = ctx->opt.lu_depth > 0 ? ctx->opt.lu_depth : (narrow ? 1 : 4);
-  b.lu_groups = ctx->opt.lu_groups > 0 ? ctx->opt.lu_groups : (narrow ? 1 : AUTO_GROUPS_MAX);
-  // narrow bands: one workgroup per cell runs each triangular sweep (no
-  // cross-workgroup hops); otherwise the block rows of all cells are spread
-  // over workgroups (k_lu_solve_mw)
-  b.solve_wg = ctx->opt.pivoting == WCFE_PIVOT_STATIC && narrow && b.max_npad > 0 &&
-               lu_solve_lds_bytes(b.max_npad, elem_size) <= lu_solve_max_dynamic(ctx->max_lds);
+    whole = whole && (!p.smw || (size_t)p.npad * elem_size <= refine_max_dynamic(ctx->max_lds));
+  if (!whole && std::any_of(b.cp_h.begin(), b.cp_h.end(), [](const CellParams &p) { return p.smw != 0; })) number(false);
   b.max_bw = 0;
   for (CellParams &p : b.cp_h) {
     const int full = std::max(p.nblk - 1, 0);
@@ -1307,6 +1323,7 @@ void build_batch(wcfe_ctx *ctx, Batch &b, const std::vector<HostCell> &hc, int e
     p.env = std::min(full, p.bw + std::max(b.lu_depth - 1, b.solve_wg ? 0 : 1));
     if (!p.csr) b.max_bw = std::max(b.max_bw, p.bw);
   }
+  for (const CellParams &p : b.cp_h) b.any_gdot |= (p.bterm & BT_AREA) && !p.smw;
   plan_bands(ctx, b, elem_size);
   // colour-major element order
   b.color_start.assign(b.ncolor + 1, 0);
@@ -2000,29 +2017,33 @@ template <class T> void enqueue_solve_refine(wcfe_ctx *ctx, Batch &b, const Scop
   View v = make_view(ctx, b);
   const int piv = ctx->opt.pivoting == WCFE_PIVOT_PARTIAL;
   const long long v0 = 2LL * sc.node_begin, vn = 2LL * (sc.node_end - sc.node_begin);
-  const bool one_wg = sc.cell < 0 ? b.nrefine > 0 : b.solve_wg && b.refine_at[sc.cell] >= 0;
+  // the scope's cells in rwg: [w0, w0 + nref) whole, [w0 + nref, w0 + nref + ntail) after the second sweep
+  int w0 = 0, nref = b.nrefine, ntail = b.ntail;
+  if (sc.cell >= 0) {
+    w0 = b.solve_wg ? std::max(b.refine_at[sc.cell], 0) : 0;
+    nref = b.cp_h[sc.cell].refine;
+    ntail = b.solve_wg && !nref && b.refine_at[sc.cell] >= 0;
+  }
+  const bool spread = nref < sc.ncell;  // cells left for the launches below
   {
     PhaseScope ph(ctx, WCFE_PH_REFINE);
     // the fused block steps and the one-workgroup refinement read G themselves
-    if (b.any_csr || !(b.solve_wg && (b.plan.fused || (one_wg && !b.tail)))) launch_neg_copy(s, b.G + v0, b.r + v0, vn);
+    if (spread && (b.any_csr || !(b.solve_wg && b.plan.fused))) launch_neg_copy(s, b.G + v0, b.r + v0, vn);
   }
   const int max_refine = std::max(1, ctx->opt.max_refine);
-  auto refine = [&](int it0) {
+  auto refine = [&](int first, int n, int it0) {
     PhaseScope ph(ctx, WCFE_PH_SOLVE);
-    launch_band_refine<T>(s, b.cp, b.cs, b.rwg + (sc.cell < 0 ? 0 : b.refine_at[sc.cell]),
-                          sc.cell < 0 ? b.nrefine : 1, b.refine_loc, b.sops, b.slocs, b.saccs, K,
+    launch_band_refine<T>(s, b.cp, b.cs, b.rwg + first, n, b.refine_loc, b.sops, b.slocs, b.saccs, K,
                           static_cast<const T *>(b.Dinv), b.kinv, sweep_vec<T>(b, b.plan.fused),
                           RefineArgs{b.el_tri, b.adj_start, b.adj, b.Ke64, b.G, b.r, b.delta, b.rp, b.dp,
                                      bnd_view(ctx, b), ctx->opt.lin_rtol, it0, max_refine, b.plan.fused ? 1 : 0});
   };
-  if (one_wg && !b.tail) {
-    refine(0);
-    if (!b.any_csr) return;
-  }
+  refine(w0, nref, 0);
+  if (!spread) return;
   const int npad = sc.cell < 0 ? b.max_npad : b.cp_h[sc.cell].npad;
   for (int it = 0; it < max_refine; ++it) {
-    if (one_wg && b.tail && it == 2 && !b.any_csr) {
-      refine(2);
+    if (ntail > 0 && it == 2 && !b.any_csr) {
+      refine(w0 + nref, ntail, 2);
       break;
     }
     {
@@ -2048,7 +2069,7 @@ template <class T> void enqueue_solve_refine(wcfe_ctx *ctx, Batch &b, const Scop
     }
     PhaseScope ph(ctx, WCFE_PH_REFINE);
     const BndView bv = bnd_view(ctx, b);
-    if (b.any_area) launch_cell_gdot(s, b.cp, sc.cells, sc.ncell, bv, b.delta);
+    if (b.any_gdot) launch_cell_gdot(s, b.cp, sc.cells, sc.ncell, bv, b.delta);
     launch_matvec_ir(s, v, b.node_cell, b.adj_start, b.adj, b.Ke64, b.G, b.delta, b.r, sc.node_begin, sc.node_end,
                      b.cs, bv);
     launch_cell_norm<T>(s, b.cp, b.cs, sc.cells, sc.ncell, b.r, 1, 1, ctx->opt.lin_rtol, b.norm_work());
@@ -3166,16 +3187,36 @@ int wcfe_assembled_system(wcfe_ctx *ctx, int32_t cell, double *K, double *G) {
       HIPCHECK(hipMemcpy(raw.data(), static_cast<unsigned char *>(b.K) + (size_t)p.k_off * es, raw.size(),
                          hipMemcpyDeviceToHost));
       const std::vector<int> &kp = b.kpos_h[cell];  // back to the natural numbering
+      // the area term's k g g^T, which a cell with smw keeps out of its band
+      std::vector<double> g(p.ndof, 0.0);
+      if (p.smw && p.n_bnd > 0) {
+        std::vector<int2> frame(p.n_bnd);
+        std::vector<double2> gb(p.n_bnd);
+        std::vector<int> node(p.n_bnd);
+        HIPCHECK(hipMemcpy(frame.data(), b.bt_frame + p.bnd_off, sizeof(int2) * p.n_bnd, hipMemcpyDeviceToHost));
+        HIPCHECK(hipMemcpy(gb.data(), b.bt_g + p.bnd_off, sizeof(double2) * p.n_bnd, hipMemcpyDeviceToHost));
+        HIPCHECK(hipMemcpy(node.data(), b.bt_node + p.bnd_off, sizeof(int) * p.n_bnd, hipMemcpyDeviceToHost));
+        for (int k = 0; k < p.n_bnd; ++k) {
+          if (frame[k].x < 0) continue;
+          g[2 * (node[k] - p.node_off)] = gb[k].x;
+          g[2 * (node[k] - p.node_off) + 1] = gb[k].y;
+        }
+      }
+      auto put = [&](int i, int j, double v) {
+        const double a = p.k_area * g[i] * g[j];
+        if (p.smw) v = es == 4 ? (double)((float)v + (float)a) : v + a;
+        K[(size_t)i * p.ndof + j] = v;
+      };
       for (int i = 0; i < p.ndof; ++i)
         for (int j = 0; j < p.ndof; ++j) {
           const int pi = 2 * kp[i / 2] + i % 2, pj = 2 * kp[j / 2] + j % 2;
           if (std::abs(pi / NB - pj / NB) > p.env) {  // outside the fill envelope: zero, never stored
-            K[(size_t)i * p.ndof + j] = 0.0;
+            put(i, j, 0.0);
             continue;
           }
           const size_t o = (size_t)pi * p.npad + pj;
-          K[(size_t)i * p.ndof + j] =
-              es == 4 ? (double)reinterpret_cast<float *>(raw.data())[o] : reinterpret_cast<double *>(raw.data())[o];
+          put(i, j,
+              es == 4 ? (double)reinterpret_cast<float *>(raw.data())[o] : reinterpret_cast<double *>(raw.data())[o]);
         }
     }
   });
