@@ -104,6 +104,24 @@ template <int NT> __device__ __forceinline__ double block_sum(double v, double *
   return red[0];
 }
 
+// Strain increment and lumped mass of one node of a UL cell, over its elements
+// in element order.
+__device__ __forceinline__ void node_strain(const View &v, int i, const int *adj_start, const int *adj, double *Rea,
+                                            double *MM) {
+  double re[3] = {0.0, 0.0, 0.0}, m = 0.0;
+  for (int k = adj_start[i]; k < adj_start[i + 1]; ++k) {
+    const int e = adj[k] >> 2, a = adj[k] & 3;
+    double rea[9], mm[3];
+    element_strain(v, e, rea, mm);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) re[q] += a == 0 ? rea[q] : a == 1 ? rea[3 + q] : rea[6 + q];
+    m += a == 0 ? mm[0] : a == 1 ? mm[1] : mm[2];
+  }
+#pragma unroll
+  for (int q = 0; q < 3; ++q) Rea[3 * i + q] = re[q];
+  MM[i] = m;
+}
+
 // UL:607-612 strain update; UL:2046-2171 mean-field bond kinetics with a rigid
 // substrate (subs_u = 0): fa_u += x - X, catch-slip k_off, forward Euler c_C,
 // dissipative rescale; the new reference configuration is the converged x.

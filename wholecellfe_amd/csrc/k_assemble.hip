@@ -315,6 +315,24 @@ template void launch_assemble_gather<double>(hipStream_t, const View &, int, int
                                              const int *, const GatherPlan &, int, int, double *, double *, double *,
                                              double *, double *, int);
 
+// One thread per node, each of its elements computed where it is needed: three
+// times the (few) operations, but one launch and no intermediate arrays
+// instead of two fills and a launch per colour.
+__global__ __launch_bounds__(128) void k_node_strain(View v, const int *node_cell, const int *adj_start,
+                                                     const int *adj, int n0, int n1, double *Rea, double *MM) {
+  const int i = n0 + blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n1) return;
+  const int c = node_cell ? node_cell[i] : 0;
+  if (!v.cs[c].converged || v.cp[c].law != LAW_UL) return;
+  node_strain(v, i, adj_start, adj, Rea, MM);
+}
+void launch_node_strain(hipStream_t s, const View &v, const int *node_cell, const int *adj_start, const int *adj,
+                        int n0, int n1, double *Rea, double *MM) {
+  if (n1 <= n0) return;
+  hipLaunchKernelGGL(k_node_strain, dim3((n1 - n0 + 127) / 128), dim3(128), 0, s, v, node_cell, adj_start, adj, n0, n1,
+                     Rea, MM);
+}
+
 __global__ __launch_bounds__(128) void k_element_dump(View v, int e_begin, int e_end, double *Ge, double *Ke) {
   const int e = e_begin + blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= e_end) return;

@@ -529,20 +529,7 @@ __global__ __launch_bounds__(FINISH_THREADS) void k_cell_finish(View v, FinishAr
   __syncthreads();
   if (!conv) return;
   if (p.law == LAW_UL) {  // strain increments and lumped masses, every node over its elements in element order
-    for (int i = n0 + tid; i < n1; i += FINISH_THREADS) {
-      double re[3] = {0.0, 0.0, 0.0}, m = 0.0;
-      for (int k = f.adj_start[i]; k < f.adj_start[i + 1]; ++k) {
-        const int e = f.adj[k] >> 2, a = f.adj[k] & 3;
-        double rea[9], mm[3];
-        element_strain(v, e, rea, mm);
-#pragma unroll
-        for (int q = 0; q < 3; ++q) re[q] += a == 0 ? rea[q] : a == 1 ? rea[3 + q] : rea[6 + q];
-        m += a == 0 ? mm[0] : a == 1 ? mm[1] : mm[2];
-      }
-#pragma unroll
-      for (int q = 0; q < 3; ++q) f.Rea[3 * i + q] = re[q];
-      f.MM[i] = m;
-    }
+    for (int i = n0 + tid; i < n1; i += FINISH_THREADS) node_strain(v, i, f.adj_start, f.adj, f.Rea, f.MM);
     __syncthreads();
   }
   const unsigned step = (unsigned)cs[c].step;

@@ -92,16 +92,23 @@ __device__ __forceinline__ bool tri_contains(const double *q0, const double *q1,
   return A1 >= 0.0 && A2 >= 0.0 && A3 >= 0.0;
 }
 
+// One wave per node: its lanes test the candidate triangles of the node's grid
+// cell at once (a chain of dependent loads per candidate: one thread per node
+// walked them one after the other, 480 nodes 18 and 57 us; now 11 and 13, of
+// which most is the launch and two cold memory round trips).
+constexpr int POINT_WAVES = 4;  // nodes per workgroup
+
 // updateFA 11-argument form (UL:2026-2174, law 1; UL1:2005-2115, law 0), one
-// thread per cell node.  The substrate point X - fa_u is located among the
+// wave per cell node.  The substrate point X - fa_u is located among the
 // substrate triangles (reference configuration) of its grid cell with the
 // reference's z-sign tests; the last containing triangle wins (UL:2098).
-__global__ __launch_bounds__(256) void k_ref_update_fa(int n_nodes, const double *X, const double *x, double *cA,
-                                                       double *cC, double *fau, double dt, PointGrid grid,
-                                                       const int *stris, const double *SX, const double *Sx, int law,
-                                                       double kint, int *n_unlocated) {
+__global__ __launch_bounds__(64 * POINT_WAVES) void k_ref_update_fa(int n_nodes, const double *X, const double *x,
+                                                                    double *cA, double *cC, double *fau, double dt,
+                                                                    PointGrid grid, const int *stris,
+                                                                    const double *SX, const double *Sx, int law,
+                                                                    double kint, int *n_unlocated) {
 #pragma clang fp contract(off)
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = blockIdx.x * POINT_WAVES + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (i >= n_nodes) return;
   double cell_u[3], sX[3], subs_u[3] = {0.0, 0.0, 0.0};
   for (int c = 0; c < 3; ++c) {
@@ -110,17 +117,29 @@ __global__ __launch_bounds__(256) void k_ref_update_fa(int n_nodes, const double
   }
   bool located = false;
   const int gc = grid_cell(grid, sX[0], sX[1]);
-  for (int k = grid.start[gc]; k < grid.start[gc + 1]; ++k) {  // last containing triangle wins (UL:2098)
-    const int *t = stris + 3 * grid.list[k];
-    double A_tri, A1, A2, A3;
-    if (tri_contains(SX + 3 * t[0], SX + 3 * t[1], SX + 3 * t[2], sX, A_tri, A1, A2, A3)) {
-      for (int c = 0; c < 3; ++c)
-        subs_u[c] = (A1 / A_tri) * (Sx[3 * t[0] + c] - SX[3 * t[0] + c]) +
-                    (A2 / A_tri) * (Sx[3 * t[1] + c] - SX[3 * t[1] + c]) +
-                    (A3 / A_tri) * (Sx[3 * t[2] + c] - SX[3 * t[2] + c]);
+  const int k1 = grid.start[gc + 1];
+  for (int k0 = grid.start[gc]; k0 < k1; k0 += 64) {
+    const int k = k0 + lane;
+    bool in = false;
+    double w[3] = {0.0, 0.0, 0.0};
+    if (k < k1) {
+      const int *t = stris + 3 * grid.list[k];
+      double A_tri, A1, A2, A3;
+      in = tri_contains(SX + 3 * t[0], SX + 3 * t[1], SX + 3 * t[2], sX, A_tri, A1, A2, A3);
+      if (in)
+        for (int c = 0; c < 3; ++c)
+          w[c] = (A1 / A_tri) * (Sx[3 * t[0] + c] - SX[3 * t[0] + c]) +
+                 (A2 / A_tri) * (Sx[3 * t[1] + c] - SX[3 * t[1] + c]) +
+                 (A3 / A_tri) * (Sx[3 * t[2] + c] - SX[3 * t[2] + c]);
+    }
+    const unsigned long long hit = __ballot(in);
+    if (hit) {  // last containing triangle wins (UL:2098)
+      const int last = 63 - __clzll((long long)hit);
+      for (int c = 0; c < 3; ++c) subs_u[c] = __shfl(w[c], last, 64);
       located = true;
     }
   }
+  if (lane != 0) return;
   if (!located) atomicAdd(n_unlocated, 1);
   double u[3];
   for (int c = 0; c < 3; ++c) u[c] = fau[3 * i + c] + cell_u[c] - subs_u[c];
@@ -149,35 +168,45 @@ void launch_ref_update_fa(hipStream_t s, int n_nodes, const double *X, const dou
                           double *fau, double dt, const PointGrid &grid, const int *stris, const double *SX,
                           const double *Sx, int law, double kint, int *n_unlocated) {
   if (n_nodes <= 0) return;
-  hipLaunchKernelGGL(k_ref_update_fa, dim3((n_nodes + 255) / 256), dim3(256), 0, s, n_nodes, X, x, cA, cC, fau, dt,
+  hipLaunchKernelGGL(k_ref_update_fa, dim3((n_nodes + POINT_WAVES - 1) / POINT_WAVES), dim3(64 * POINT_WAVES), 0, s,
+                     n_nodes, X, x, cA, cC, fau, dt,
                      grid, stris, SX, Sx, law, kint, n_unlocated);
 }
 
 // calculateForce_FA_subs (UL:1305-1475, law 1 MD table; UL1:1297, law 0
-// linear kint), one thread per cell node: the node's integrin force at the
+// linear kint), one wave per cell node: the node's integrin force at the
 // substrate point x_cell - fa_u, for every substrate triangle containing it
 // in the substrate's current positions, split by barycentric weight.  Each
 // hit's 9 contributions are written out (hits in increasing triangle order,
 // at most SUBS_MAX_HITS per node) and summed on the host in the reference's
 // order.
-__global__ __launch_bounds__(256) void k_ref_force_fa_subs(int n_nodes, const int *ring_start, const int *ring,
-                                                           const int *tris, const double *x_cell, const double *cC,
-                                                           const double *fau, PointGrid grid, const int *stris,
-                                                           const double *Sx, int law, double kint, int *hit_tri,
-                                                           double *hit_val, int *n_hits, int *overflow) {
+__global__ __launch_bounds__(64 * POINT_WAVES) void k_ref_force_fa_subs(int n_nodes, const int *ring_start,
+                                                                        const int *ring, const int *tris,
+                                                                        const double *x_cell, const double *cC,
+                                                                        const double *fau, PointGrid grid,
+                                                                        const int *stris, const double *Sx, int law,
+                                                                        double kint, SubsHits hits) {
 #pragma clang fp contract(off)
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = blockIdx.x * POINT_WAVES + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (i >= n_nodes) return;
   const double p[3] = {x_cell[3 * i] - fau[3 * i], x_cell[3 * i + 1] - fau[3 * i + 1],
                        x_cell[3 * i + 2] - fau[3 * i + 2]};
   const int gc = grid_cell(grid, p[0], p[1]);
   int h = 0;
   double Asum = -1.0, fs[3] = {0.0, 0.0, 0.0};
-  for (int k = grid.start[gc]; k < grid.start[gc + 1]; ++k) {
-    const int e = grid.list[k];
-    const int *t = stris + 3 * e;
-    double A_tri, A1, A2, A3;
-    if (!tri_contains(Sx + 3 * t[0], Sx + 3 * t[1], Sx + 3 * t[2], p, A_tri, A1, A2, A3)) continue;
+  const int k1 = grid.start[gc + 1];
+  for (int k0 = grid.start[gc]; k0 < k1; k0 += 64) {
+    const int k = k0 + lane;
+    int e = 0;
+    bool in = false;
+    double A_tri = 1.0, A1 = 0.0, A2 = 0.0, A3 = 0.0;
+    if (k < k1) {
+      e = grid.list[k];
+      const int *t = stris + 3 * e;
+      in = tri_contains(Sx + 3 * t[0], Sx + 3 * t[1], Sx + 3 * t[2], p, A_tri, A1, A2, A3);
+    }
+    const unsigned long long hit = __ballot(in);
+    if (!hit) continue;
     if (Asum < 0.0) {  // first hit: the node's one-ring area / 3 and its spring force
       Asum = 0.0;
       for (int r = ring_start[i]; r < ring_start[i + 1]; ++r) {
@@ -198,28 +227,54 @@ __global__ __launch_bounds__(256) void k_ref_force_fa_subs(int n_nodes, const in
         for (int c = 0; c < 3; ++c) fs[c] = D == 0.0 ? 0.0 : f * (u[c] / D);
       }
     }
-    if (h == SUBS_MAX_HITS) {
-      atomicAdd(overflow, 1);
-      break;
+    const int at = h + __popcll(hit & ((1ull << lane) - 1ull));
+    h += __popcll(hit);
+    if (in && at < SUBS_MAX_HITS) {
+      const bool near = at < SUBS_FIRST_HITS;
+      const long long o = (long long)(near ? at : at - SUBS_FIRST_HITS) * n_nodes + i;
+      (near ? hits.tri : hits.tri_more)[o] = e;
+      double *v = (near ? hits.val : hits.val_more) + 9 * o;
+      const double w[3] = {A1 / A_tri, A2 / A_tri, A3 / A_tri};
+      const double rho_i_max = 100.0;  // UL:1391
+      for (int a = 0; a < 3; ++a)
+        for (int c = 0; c < 3; ++c) v[3 * a + c] = cC[i] * fs[c] * w[a] * Asum * rho_i_max;
     }
-    const double w[3] = {A1 / A_tri, A2 / A_tri, A3 / A_tri};
-    hit_tri[i * SUBS_MAX_HITS + h] = e;
-    double *v = hit_val + 9LL * (i * SUBS_MAX_HITS + h);
-    const double rho_i_max = 100.0;  // UL:1391
-    for (int a = 0; a < 3; ++a)
-      for (int c = 0; c < 3; ++c) v[3 * a + c] = cC[i] * fs[c] * w[a] * Asum * rho_i_max;
-    ++h;
+    if (h > SUBS_MAX_HITS) break;
   }
-  n_hits[i] = h;
+  if (lane != 0) return;
+  if (h > SUBS_MAX_HITS) atomicAdd(hits.overflow, 1);
+  hits.n[i] = min(h, SUBS_MAX_HITS);
 }
 void launch_ref_force_fa_subs(hipStream_t s, int n_nodes, const int *ring_start, const int *ring, const int *tris,
                               const double *x_cell, const double *cC, const double *fau, const PointGrid &grid,
-                              const int *stris, const double *Sx, int law, double kint, int *hit_tri,
-                              double *hit_val, int *n_hits, int *overflow) {
+                              const int *stris, const double *Sx, int law, double kint, const SubsHits &hits) {
   if (n_nodes <= 0) return;
-  hipLaunchKernelGGL(k_ref_force_fa_subs, dim3((n_nodes + 255) / 256), dim3(256), 0, s, n_nodes, ring_start, ring,
-                     tris, x_cell, cC, fau, grid, stris, Sx, law, kint, hit_tri, hit_val, n_hits, overflow);
+  hipLaunchKernelGGL(k_ref_force_fa_subs, dim3((n_nodes + POINT_WAVES - 1) / POINT_WAVES), dim3(64 * POINT_WAVES), 0, s,
+                     n_nodes, ring_start, ring, tris, x_cell, cC, fau, grid, stris, Sx, law, kint, hits);
 }
+
+// The working-precision copy of the caller's matrices, one wave per row (24 systems
+// of 60 to 700: 15 us; made on the host and sent as well it took 900).
+template <class T>
+__global__ __launch_bounds__(256) void k_dense_load(const CellParams *cp, const double *A64, const long long *a_off,
+                                                    T *K) {
+  const CellParams &p = cp[blockIdx.y];
+  const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (r >= p.npad) return;
+  const double *A = A64 + a_off[blockIdx.y] + (long long)r * p.ndof;
+  T *row = K + p.k_off + (long long)r * p.npad;
+  for (int j = lane; j < p.npad; j += 64) row[j] = r < p.ndof && j < p.ndof ? (T)A[j] : (r == j ? T(1) : T(0));
+}
+template <class T>
+void launch_dense_load(hipStream_t s, const CellParams *cp, int n_sys, int max_npad, const double *A64,
+                       const long long *a_off, T *K) {
+  if (n_sys <= 0 || max_npad <= 0) return;
+  hipLaunchKernelGGL(k_dense_load<T>, dim3((max_npad + 3) / 4, n_sys), dim3(256), 0, s, cp, A64, a_off, K);
+}
+template void launch_dense_load<float>(hipStream_t, const CellParams *, int, int, const double *, const long long *,
+                                       float *);
+template void launch_dense_load<double>(hipStream_t, const CellParams *, int, int, const double *, const long long *,
+                                        double *);
 
 // r = b - A x in FP64 for dense systems; systems whose refinement has
 // converged are skipped.  Bound by reading A once: one wave per row, its lanes

@@ -11,6 +11,7 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
+#include <mutex>
 #include <memory>
 #include <string>
 #include <thread>
@@ -534,7 +535,8 @@ struct LuPlan {
     d_ranges = dupload(ranges);
   }
 
-  void build(const std::vector<CellParams> &cp, int piv, int groups, int lu_depth) {
+  // host: the work lists stay there, for the caller to upload and own
+  void build(const std::vector<CellParams> &cp, int piv, int groups, int lu_depth, std::vector<int> *host = nullptr) {
     if (lu_depth < 1 || groups < 1) throw ApiError{WCFE_ERR_ARG, "LU schedule needs depth and groups >= 1"};
     pivoting = piv;
     depth = lu_depth;
@@ -610,7 +612,8 @@ struct LuPlan {
     }
     solve_single.assign(n, SolveLists{});
     for (int c = 0; c < n; ++c) solve_single[c] = add_lists(std::vector<int>{c});
-    d_prefix = dupload(buf);
+    if (host) *host = std::move(buf);
+    else d_prefix = dupload(buf);
   }
 };
 
@@ -778,8 +781,43 @@ struct FrameSlot {
   hipEvent_t done = nullptr;
 };
 
+// One device allocation and one pinned host allocation for the stateless calls
+// (Scratch).
+struct Arena {
+  unsigned char *dev = nullptr, *host = nullptr;
+  size_t dev_cap = 0, host_cap = 0;
+  void reserve(size_t d, size_t h) {
+    if (d > dev_cap) {
+      if (dev) (void)hipFree(dev);
+      dev = nullptr;
+      dev_cap = 0;
+      const size_t n = std::max<size_t>(d + d / 4, 1u << 20);
+      dev = dalloc<unsigned char>(n);
+      dev_cap = n;
+    }
+    if (h > host_cap) {
+      if (host) (void)hipHostFree(host);
+      host = nullptr;
+      host_cap = 0;
+      const size_t n = std::max<size_t>(h + h / 4, 1u << 20);
+      void *p = nullptr;
+      const hipError_t e = hipHostMalloc(&p, n, hipHostMallocDefault);
+      if (e != hipSuccess) fail(WCFE_ERR_OOM, "hipHostMalloc of %zu bytes failed: %s", n, hipGetErrorString(e));
+      host = static_cast<unsigned char *>(p);
+      host_cap = n;
+    }
+  }
+  void release() {
+    if (dev) (void)hipFree(dev);
+    if (host) (void)hipHostFree(host);
+    *this = Arena();
+  }
+};
+
 struct wcfe_ctx {
   wcfe_options opt;
+  Arena arena;  // held by the call that holds arena_mutex
+  std::mutex arena_mutex;
   std::string err;
   int device = 0;
   hipStream_t stream = nullptr;
@@ -2138,7 +2176,9 @@ template <class T> void enqueue_newton(wcfe_ctx *ctx, Batch &b, const Scope &sc)
   // 5. commit converged cells
   PhaseScope ph(ctx, WCFE_PH_COMMIT);
   const bool any_ul = sc.cell < 0 ? b.any_ul : (b.cp_h[sc.cell].law == LAW_UL);
-  if (any_ul) {
+  if (any_ul && sc.cell < 0) {
+    launch_node_strain(s, make_view(ctx, b), b.node_cell, b.adj_start, b.adj, sc.node_begin, sc.node_end, b.Rea, b.MM);
+  } else if (any_ul) {
     launch_fill(s, b.Rea + 3LL * sc.node_begin, 3LL * (sc.node_end - sc.node_begin), 0.0);
     launch_fill(s, b.MM + sc.node_begin, sc.node_end - sc.node_begin, 0.0);
     enqueue_assemble<T>(ctx, b, sc, ASM_STRAIN);
@@ -2322,6 +2362,7 @@ int wcfe_destroy(wcfe_ctx *ctx) {
   if (ctx->gexec) (void)hipGraphExecDestroy(ctx->gexec);
   if (ctx->graph) (void)hipGraphDestroy(ctx->graph);
   ctx->b.release();
+  ctx->arena.release();
   if (ctx->tab_px) (void)hipFree(ctx->tab_px);
   if (ctx->tab_py) (void)hipFree(ctx->tab_py);
   if (ctx->tab_k) (void)hipFree(ctx->tab_k);
@@ -3236,23 +3277,102 @@ int wcfe_get_colors(wcfe_ctx *ctx, int32_t cell, int32_t *color) {
 namespace {
 
 // Device buffers owned for the duration of one stateless call.
+// Buffers of one stateless call.  They come out of the context's arena: one
+// device allocation and one pinned host allocation, kept between calls up to
+// ARENA_KEEP bytes and freed with the context, so a call makes no allocation,
+// one copy to the device and one back (a call of a 900-triangle cell made up
+// to fifteen of each, 10 to 30 us apiece).  A second thread in a call on the
+// same context gets buffers of its own.  Declare every buffer (in, inout, out,
+// zeros, work), commit(), launch, fetch().  Arrays above ARENA_DIRECT bytes
+// are copied from and to the caller's memory without the pinned copy.
+constexpr size_t ARENA_KEEP = 64u << 20, ARENA_DIRECT = 1u << 20;
 struct Scratch {
-  std::vector<void *> ptrs;
-  template <class T> T *up(const T *h, size_t n) {
-    T *d = dalloc<T>(n);
-    ptrs.push_back(d);
-    if (n && h) HIPCHECK(hipMemcpy(d, h, n * sizeof(T), hipMemcpyHostToDevice));
-    return d;
-  }
-  template <class T> T *zeros(size_t n) {
-    T *d = dalloc<T>(n);
-    ptrs.push_back(d);
-    HIPCHECK(hipMemset(d, 0, std::max<size_t>(n, 1) * sizeof(T)));
-    return d;
-  }
+  explicit Scratch(wcfe_ctx *c) : ctx(c), lock(c->arena_mutex, std::try_to_lock), A(lock ? &c->arena : &own) {}
+  Scratch(const Scratch &) = delete;
+  Scratch &operator=(const Scratch &) = delete;
   ~Scratch() {
-    for (void *p : ptrs) (void)hipFree(p);
+    if (sent) (void)hipStreamSynchronize(ctx->stream);
+    if (A == &own || A->dev_cap + A->host_cap > ARENA_KEEP) A->release();
   }
+  template <class T> void in(const T *&d, const T *h, size_t n) { add(&d, h, nullptr, n * sizeof(T), IN); }
+  template <class T> void in(T *&d, const T *h, size_t n) { add(&d, h, nullptr, n * sizeof(T), IN); }
+  // h null: zeros
+  template <class T> void inout(T *&d, const T *h, T *back, size_t n) { add(&d, h, back, n * sizeof(T), INOUT); }
+  template <class T> void out(T *&d, T *back, size_t n) { add(&d, nullptr, back, n * sizeof(T), OUT); }
+  template <class T> void zeros(T *&d, size_t n) { add(&d, nullptr, nullptr, n * sizeof(T), ZERO); }
+  template <class T> void work(T *&d, size_t n) { add(&d, nullptr, nullptr, n * sizeof(T), WORK); }
+  void commit() {
+    // mirrored: IN, INOUT, OUT in this order, then device only: ZERO, the large ones, WORK
+    size_t off = 0, up0 = 0;
+    auto place = [&](int kind, bool direct) {
+      for (Buf &q : bufs)
+        if (q.kind == kind && q.direct == direct) {
+          q.off = off;
+          off += (q.bytes + 255) & ~(size_t)255;
+        }
+    };
+    place(IN, false);
+    down0 = off;
+    place(INOUT, false);
+    up0 = off;
+    place(OUT, false);
+    down1 = off;
+    place(ZERO, false);
+    const size_t zero1 = off;
+    for (int k : {IN, INOUT, OUT, ZERO, WORK})
+      if (k != ZERO) place(k, true);
+    place(WORK, false);
+    A->reserve(off, down1);
+    for (Buf &q : bufs) {
+      void *d = A->dev + q.off;
+      memcpy(q.slot, &d, sizeof d);
+      if (q.direct || q.kind == OUT || q.kind == ZERO || q.kind == WORK || !q.bytes) continue;
+      if (q.h) memcpy(A->host + q.off, q.h, q.bytes);
+      else memset(A->host + q.off, 0, q.bytes);
+    }
+    sent = true;
+    if (up0) HIPCHECK(hipMemcpyAsync(A->dev, A->host, up0, hipMemcpyHostToDevice, ctx->stream));
+    if (zero1 > down1) HIPCHECK(hipMemsetAsync(A->dev + down1, 0, zero1 - down1, ctx->stream));
+    for (Buf &q : bufs) {
+      if (!q.direct || !q.bytes) continue;
+      if (q.h) HIPCHECK(hipMemcpyAsync(A->dev + q.off, q.h, q.bytes, hipMemcpyHostToDevice, ctx->stream));
+      else if (q.kind == INOUT) HIPCHECK(hipMemsetAsync(A->dev + q.off, 0, q.bytes, ctx->stream));
+    }
+  }
+  // every inout and out array in the caller's memory
+  void fetch() {
+    HIPCHECK(hipGetLastError());
+    if (down1 > down0)
+      HIPCHECK(hipMemcpyAsync(A->host + down0, A->dev + down0, down1 - down0, hipMemcpyDeviceToHost, ctx->stream));
+    for (Buf &q : bufs)
+      if (q.direct && q.back && q.bytes)
+        HIPCHECK(hipMemcpyAsync(q.back, A->dev + q.off, q.bytes, hipMemcpyDeviceToHost, ctx->stream));
+    HIPCHECK(hipStreamSynchronize(ctx->stream));
+    sent = false;
+    for (Buf &q : bufs)
+      if (!q.direct && q.back && q.bytes) memcpy(q.back, A->host + q.off, q.bytes);
+  }
+
+ private:
+  enum { IN, INOUT, OUT, ZERO, WORK };
+  struct Buf {
+    void *slot;
+    const void *h;
+    void *back;
+    size_t bytes, off;
+    int kind;
+    bool direct;
+  };
+  void add(void *slot, const void *h, void *back, size_t bytes, int kind) {
+    bufs.push_back(Buf{slot, h, back, bytes, 0, kind, kind < ZERO && bytes > ARENA_DIRECT});
+  }
+  wcfe_ctx *ctx;
+  Arena own;
+  std::unique_lock<std::mutex> lock;
+  Arena *A;
+  std::vector<Buf> bufs;
+  size_t down0 = 0, down1 = 0;
+  bool sent = false;
 };
 
 template <class T>
@@ -3293,40 +3413,41 @@ void dense_solve_impl(wcfe_ctx *ctx, int n_sys, const int32_t *n, const double *
   if (ctx->opt.pivoting == WCFE_PIVOT_PARTIAL &&
       lu_solve_lds_bytes(max_npad, sizeof(T)) > lu_solve_max_dynamic(ctx->max_lds))
     fail(WCFE_ERR_ARG, "system of %d unknowns exceeds the LDS-resident triangular solve", max_npad);
-  std::vector<T> Kh((size_t)kp, T(0));
-  for (int i = 0; i < n_sys; ++i) {
-    const CellParams &p = cp[i];
-    for (int r = 0; r < p.npad; ++r)
-      for (int c = 0; c < p.npad; ++c)
-        Kh[(size_t)p.k_off + (size_t)r * p.npad + c] =
-            (r < p.ndof && c < p.ndof) ? (T)A[a_off[i] + (long long)r * p.ndof + c] : (r == c ? T(1) : T(0));
-  }
   std::vector<CellState> cs(n_sys);
   for (auto &q : cs) memset(&q, 0, sizeof q);
-  std::vector<int> ident(n_sys);
+  std::vector<int> ident(n_sys), prefix;
   for (int i = 0; i < n_sys; ++i) ident[i] = i;
-  Scratch sc;
-  T *dK = sc.up(Kh.data(), Kh.size());
-  double *dA = sc.up(A, (size_t)ap);
-  long long *dAoff = sc.up(a_off.data(), a_off.size());
-  double *db = sc.up(b, (size_t)vo);
-  double *dr = sc.zeros<double>((size_t)vo);
-  double *dx = sc.zeros<double>((size_t)vo);
-  CellParams *dcp = sc.up(cp.data(), cp.size());
-  CellState *dcs = sc.up(cs.data(), cs.size());
-  int *dcells = sc.up(ident.data(), ident.size());
-  int *dipiv = sc.zeros<int>((size_t)std::max(sys, 1));
-  T *dDinv = sc.zeros<T>((size_t)std::max(sys, 1) * 128);
   LuPlan plan;
-  plan.build(cp, ctx->opt.pivoting, 1, ctx->opt.lu_depth > 0 ? ctx->opt.lu_depth : 4);  // full matrices
-  sc.ptrs.push_back(plan.d_prefix);
+  plan.build(cp, ctx->opt.pivoting, 1, ctx->opt.lu_depth > 0 ? ctx->opt.lu_depth : 4, &prefix);  // full matrices
   const bool piv = ctx->opt.pivoting == WCFE_PIVOT_PARTIAL;
+  std::vector<int> pv(std::max(sys, 1));
+  Scratch sc(ctx);
+  double *dA, *db, *dr, *dx;
+  long long *dAoff;
+  CellParams *dcp;
+  CellState *dcs;
+  int *dcells, *dipiv, *dsync;
+  T *dK, *dDinv;
+  unsigned char *dy;
+  sc.in(dA, A, (size_t)ap);
+  sc.in(dAoff, a_off.data(), a_off.size());
+  sc.in(db, b, (size_t)vo);
+  sc.in(dr, b, (size_t)vo);
+  sc.in(dcp, cp.data(), cp.size());
+  sc.in(dcells, ident.data(), ident.size());
+  sc.in(plan.d_prefix, prefix.data(), prefix.size());
+  sc.inout(dcs, cs.data(), cs.data(), cs.size());
+  sc.inout<double>(dx, nullptr, x, (size_t)vo);
+  sc.inout<int>(dipiv, nullptr, pv.data(), pv.size());
+  sc.zeros(dDinv, (size_t)std::max(sys, 1) * 128);
+  sc.zeros(dy, lu_solve_exchange_bytes(std::max(sys, 1), sizeof(T)));
+  sc.zeros(dsync, SOLVE_SYNC_INTS);
+  sc.work(dK, (size_t)kp);
+  sc.commit();
+  launch_dense_load<T>(s, dcp, n_sys, max_npad, dA, dAoff, dK);
   // refinement: r = b; repeat { d = LU^-1 r; x += d; r = b - A x (FP64) }
   launch_cell_norm<T>(s, dcp, dcs, dcells, n_sys, db, 0, 0, -1.0, NormWork(), piv ? nullptr : dK);
   enqueue_lu<T>(ctx, ctx->stream, plan, plan.batched, dcp, dcs, dK, dDinv, dipiv);
-  HIPCHECK(hipMemcpyAsync(dr, db, sizeof(double) * vo, hipMemcpyDeviceToDevice, s));
-  unsigned char *dy = sc.zeros<unsigned char>(lu_solve_exchange_bytes(std::max(sys, 1), sizeof(T)));
-  int *dsync = sc.zeros<int>((size_t)SOLVE_SYNC_INTS);
   for (int it = 0; it < std::max(1, ctx->opt.max_refine); ++it) {
     if (piv)
       launch_lu_solve<T>(s, dcp, dcs, dcells, n_sys, dK, dDinv, dipiv, piv, dr, dx, max_npad, it > 0);
@@ -3338,10 +3459,7 @@ void dense_solve_impl(wcfe_ctx *ctx, int n_sys, const int32_t *n, const double *
     launch_dense_residual(s, dcp, dcs, dcells, n_sys, max_npad, dA, dAoff, db, dx, dr);
     launch_cell_norm<T>(s, dcp, dcs, dcells, n_sys, dr, 1, 1, ctx->opt.lin_rtol);
   }
-  HIPCHECK(hipGetLastError());
-  HIPCHECK(hipStreamSynchronize(s));
-  HIPCHECK(hipMemcpy(x, dx, sizeof(double) * vo, hipMemcpyDeviceToHost));
-  HIPCHECK(hipMemcpy(cs.data(), dcs, sizeof(CellState) * n_sys, hipMemcpyDeviceToHost));
+  sc.fetch();
   for (int i = 0; i < n_sys; ++i) {
     if (relres) relres[i] = cs[i].lin_relres;
     if (iters) iters[i] = cs[i].ir_iters;
@@ -3349,8 +3467,6 @@ void dense_solve_impl(wcfe_ctx *ctx, int n_sys, const int32_t *n, const double *
     if (cs[i].solve_stall) fail(WCFE_ERR_HIP, "system %d: triangular-solve wait exceeded its bound", i);
   }
   if (ipiv_out) {
-    std::vector<int> pv(std::max(sys, 1));
-    HIPCHECK(hipMemcpy(pv.data(), dipiv, sizeof(int) * pv.size(), hipMemcpyDeviceToHost));
     int o = 0;
     for (int i = 0; i < n_sys; ++i)
       for (int j = 0; j < n[i]; ++j) ipiv_out[o++] = pv[cp[i].sys_off + j];
@@ -3439,11 +3555,10 @@ HostGrid build_point_grid(int n_snodes, int n_stris, const int32_t *stris, const
   h.g = PointGrid{ox, oy, inv_h, gx, gy, nullptr, nullptr};
   return h;
 }
-PointGrid upload_grid(Scratch &sc, const HostGrid &h) {
-  PointGrid g = h.g;
-  g.start = sc.up(h.start.data(), h.start.size());
-  g.list = sc.up(h.list.data(), std::max<size_t>(h.list.size(), 1));
-  return g;
+void upload_grid(Scratch &sc, const HostGrid &h, PointGrid &g) {
+  g = h.g;
+  sc.in(g.start, h.start.data(), h.start.size());
+  sc.in(g.list, h.list.data(), h.list.size());
 }
 
 void check_mesh(int n_nodes, int n_tris, const int32_t *tris) {
@@ -3461,13 +3576,13 @@ int wcfe_eval_exp(wcfe_ctx *ctx, int64_t n, const double *x, double *y) {
   return guarded(ctx, [&] {
     HIPCHECK(hipSetDevice(ctx->opt.device));
     if (n == 0) return;
-    Scratch sc;
-    const double *dx = sc.up(x, (size_t)n);
-    double *dy = sc.zeros<double>((size_t)n);
+    Scratch sc(ctx);
+    double *dx, *dy;
+    sc.in(dx, x, (size_t)n);
+    sc.out(dy, y, (size_t)n);
+    sc.commit();
     launch_eval_exp(ctx->stream, n, dx, dy);
-    HIPCHECK(hipGetLastError());
-    HIPCHECK(hipStreamSynchronize(ctx->stream));
-    HIPCHECK(hipMemcpy(y, dy, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost));
+    sc.fetch();
   });
 }
 
@@ -3489,60 +3604,94 @@ int wcfe_calculate_res(wcfe_ctx *ctx, int32_t n_nodes, int32_t n_tris, const int
     check_mesh(n_nodes, n_tris, tris);
     if (mat != 1 && mat != 2) fail(WCFE_ERR_ARG, "mat must be 1 (cell) or 2 (substrate)");
     HIPCHECK(hipSetDevice(ctx->opt.device));
-    HostCell h;
-    h.n_nodes = n_nodes;
-    h.n_tris = n_tris;
-    h.law = WCFE_LAW_UL;
-    h.mu = mat == 2 ? 1.0e6 : 1000.0;  // UL:724-727
-    h.passive = mat == 2;              // t_act = 0 (UL:763)
-    h.thick = 1.0;                     // UL:768
-    h.X.resize(2 * (size_t)n_nodes);
-    h.x.resize(2 * (size_t)n_nodes);
-    h.ea.resize(3 * (size_t)n_nodes);
+    // the planar data of the reference's arrays
+    const size_t N = (size_t)n_nodes;
+    std::vector<double2> Xp(N), xp(N);
+    std::vector<double> ea3(3 * N);
     for (int i = 0; i < n_nodes; ++i) {
       if (X[3 * i + 2] != 0.0 || x[3 * i + 2] != 0.0)
         fail(WCFE_ERR_ARG, "node %d is off the plane z = 0 (the reference's planar cell, iomesh.cpp:519)", i);
       const double *e6 = ea + 6 * (size_t)i;
       if (fabs(e6[2]) > 1e-10 || fabs(e6[4]) > 1e-10 || fabs(e6[5]) > 1e-10)
         fail(WCFE_ERR_ARG, "node %d carries out-of-plane strain", i);
-      h.X[2 * i] = X[3 * i]; h.X[2 * i + 1] = X[3 * i + 1];
-      h.x[2 * i] = x[3 * i]; h.x[2 * i + 1] = x[3 * i + 1];
-      h.ea[3 * i] = e6[0]; h.ea[3 * i + 1] = e6[1]; h.ea[3 * i + 2] = e6[3];
+      Xp[i] = make_double2(X[3 * i], X[3 * i + 1]);
+      xp[i] = make_double2(x[3 * i], x[3 * i + 1]);
+      ea3[3 * i] = e6[0]; ea3[3 * i + 1] = e6[1]; ea3[3 * i + 2] = e6[3];
     }
-    h.tris.assign(tris, tris + 3 * (size_t)n_tris);
-    Batch tb;
-    try {
-      build_batch(ctx, tb, std::vector<HostCell>{h}, 8);
-      CellState cs;
-      memset(&cs, 0, sizeof cs);
-      cs.time = time;
-      cs.converged = 1;
-      HIPCHECK(hipMemcpy(tb.cs, &cs, sizeof cs, hipMemcpyHostToDevice));
-      Scope sc = scope_all(tb);
-      enqueue_assemble<double>(ctx, tb, sc, ASM_RESIDUAL);
-      launch_fill(ctx->stream, tb.Rea, 3LL * n_nodes, 0.0);
-      launch_fill(ctx->stream, tb.MM, n_nodes, 0.0);
-      enqueue_assemble<double>(ctx, tb, sc, ASM_STRAIN);
-      HIPCHECK(hipGetLastError());
-      HIPCHECK(hipStreamSynchronize(ctx->stream));
-      std::vector<double> G(2 * (size_t)n_nodes), R(3 * (size_t)n_nodes);
-      HIPCHECK(hipMemcpy(G.data(), tb.G, sizeof(double) * G.size(), hipMemcpyDeviceToHost));
-      HIPCHECK(hipMemcpy(R.data(), tb.Rea, sizeof(double) * R.size(), hipMemcpyDeviceToHost));
-      HIPCHECK(hipMemcpy(MM, tb.MM, sizeof(double) * n_nodes, hipMemcpyDeviceToHost));
-      int degenerate = 0;
-      HIPCHECK(hipMemcpy(&cs, tb.cs, sizeof cs, hipMemcpyDeviceToHost));
-      degenerate = cs.degenerate;
-      for (int i = 0; i < n_nodes; ++i) {
-        Res[3 * i] = G[2 * i]; Res[3 * i + 1] = G[2 * i + 1]; Res[3 * i + 2] = 0.0;
-        double *o = Res_ea + 6 * (size_t)i;
-        o[0] = R[3 * i]; o[1] = R[3 * i + 1]; o[2] = 0.0; o[3] = R[3 * i + 2]; o[4] = 0.0; o[5] = 0.0;
+    // a cell as the batches lay it out: elements colour by colour
+    std::vector<int> color;
+    const int nc = color_elements(n_nodes, n_tris, tris, color);
+    if (nc < 0) fail(WCFE_ERR_ARG, "cell %d needs more than 64 element colours", 0);
+    if (36LL * n_tris >= (1LL << 31))
+      fail(WCFE_ERR_ARG, "batch of %d elements exceeds the gather plan's 32-bit offsets", n_tris);
+    const int npad = 2 * n_nodes > ctx->opt.dense_max_dof ? 0 : ((2 * n_nodes + NB - 1) / NB) * NB;
+    if (ctx->opt.pivoting == WCFE_PIVOT_PARTIAL &&
+        lu_solve_lds_bytes(npad, 8) > lu_solve_max_dynamic(ctx->max_lds))
+      fail(WCFE_ERR_ARG, "system of %d unknowns exceeds the LDS-resident triangular solve (%zu bytes max)", npad,
+           ctx->max_lds);
+    std::vector<int> first(std::max(nc, 0) + 1, 0), el_tri(3 * (size_t)n_tris), adj_start(N + 1, 0),
+        adj(3 * (size_t)n_tris);
+    for (int e = 0; e < n_tris; ++e) ++first[color[e] + 1];
+    for (int k = 0; k < nc; ++k) first[k + 1] += first[k];
+    for (int e = 0; e < n_tris; ++e) {
+      const int pos = first[color[e]]++;
+      for (int a = 0; a < 3; ++a) {
+        el_tri[3 * (size_t)pos + a] = tris[3 * e + a];
+        ++adj_start[tris[3 * e + a] + 1];
       }
-      tb.release();
-      if (degenerate) fail(WCFE_ERR_DEGENERATE, "zero-area or inverted element");
-    } catch (...) {
-      tb.release();
-      throw;
     }
+    for (size_t i = 0; i < N; ++i) adj_start[i + 1] += adj_start[i];
+    {
+      std::vector<int> fill(adj_start.begin(), adj_start.end() - 1);
+      for (int e = 0; e < n_tris; ++e)
+        for (int a = 0; a < 3; ++a) adj[fill[el_tri[3 * (size_t)e + a]]++] = 4 * e + a;
+    }
+    CellParams p;
+    memset(&p, 0, sizeof p);
+    p.law = WCFE_LAW_UL;
+    p.mu = mat == 2 ? 1.0e6 : 1000.0;  // UL:724-727
+    p.passive = mat == 2;              // t_act = 0 (UL:763)
+    p.thick = 1.0;                     // UL:768
+    p.n_nodes = n_nodes;
+    p.n_elems = n_tris;
+    CellState cs;
+    memset(&cs, 0, sizeof cs);
+    cs.time = time;
+    cs.converged = 1;
+    std::vector<double> G(2 * N), R(3 * N);
+    Scratch sc(ctx);
+    View v;
+    memset(&v, 0, sizeof v);
+    v.kappa = ctx->opt.kappa;
+    CellState *dcs;
+    int *zero, *das, *dadj;
+    double *dGe, *dG, *dR, *dM;
+    sc.in(v.X, Xp.data(), N);
+    sc.in(v.x, xp.data(), N);
+    sc.in(v.ea, ea3.data(), 3 * N);
+    sc.in(v.el_tri, el_tri.data(), el_tri.size());
+    sc.in(v.cp, &p, 1);
+    sc.in(das, adj_start.data(), adj_start.size());
+    sc.in(dadj, adj.data(), adj.size());
+    sc.inout(dcs, &cs, &cs, 1);
+    sc.out(dG, G.data(), G.size());
+    sc.out(dR, R.data(), R.size());
+    sc.out(dM, MM, N);
+    sc.zeros(zero, 2 * (size_t)n_tris);  // one cell, no springs
+    sc.work(dGe, 6 * (size_t)n_tris);
+    sc.commit();
+    v.cs = dcs;
+    v.el_cell = v.el_spr = zero;
+    launch_assemble_gather<double>(ctx->stream, v, 0, n_tris, ASM_RESIDUAL, nullptr, das, dadj, GatherPlan{}, 0,
+                                   n_nodes, dGe, nullptr, dG, nullptr, nullptr, 0);
+    launch_node_strain(ctx->stream, v, nullptr, das, dadj, 0, n_nodes, dR, dM);
+    sc.fetch();
+    for (int i = 0; i < n_nodes; ++i) {
+      Res[3 * i] = G[2 * i]; Res[3 * i + 1] = G[2 * i + 1]; Res[3 * i + 2] = 0.0;
+      double *o = Res_ea + 6 * (size_t)i;
+      o[0] = R[3 * i]; o[1] = R[3 * i + 1]; o[2] = 0.0; o[3] = R[3 * i + 2]; o[4] = 0.0; o[5] = 0.0;
+    }
+    if (cs.degenerate) fail(WCFE_ERR_DEGENERATE, "zero-area or inverted element");
   });
 }
 
@@ -3555,15 +3704,19 @@ int wcfe_force_fa(wcfe_ctx *ctx, int32_t n_nodes, int32_t n_tris, const int32_t 
     HIPCHECK(hipSetDevice(ctx->opt.device));
     std::vector<int> st, li;
     one_rings(n_nodes, n_tris, tris, st, li);
-    Scratch sc;
-    int *dst = sc.up(st.data(), st.size()), *dli = sc.up(li.data(), li.size());
-    int *dtr = sc.up(tris, 3 * (size_t)n_tris);
-    double *dx = sc.up(x, 3 * (size_t)n_nodes), *dc = sc.up(cC, (size_t)n_nodes);
-    double *df = sc.up(fau, 3 * (size_t)n_nodes), *dF = sc.zeros<double>(3 * (size_t)n_nodes);
+    Scratch sc(ctx);
+    int *dst, *dli, *dtr;
+    double *dx, *dc, *df, *dF;
+    sc.in(dst, st.data(), st.size());
+    sc.in(dli, li.data(), li.size());
+    sc.in(dtr, tris, 3 * (size_t)n_tris);
+    sc.in(dx, x, 3 * (size_t)n_nodes);
+    sc.in(dc, cC, (size_t)n_nodes);
+    sc.in(df, fau, 3 * (size_t)n_nodes);
+    sc.out(dF, F, 3 * (size_t)n_nodes);
+    sc.commit();
     launch_ref_force_fa(ctx->stream, n_nodes, dst, dli, dtr, dx, dc, df, law, kint, dF);
-    HIPCHECK(hipGetLastError());
-    HIPCHECK(hipStreamSynchronize(ctx->stream));
-    HIPCHECK(hipMemcpy(F, dF, sizeof(double) * 3 * n_nodes, hipMemcpyDeviceToHost));
+    sc.fetch();
   });
 }
 
@@ -3589,21 +3742,24 @@ int wcfe_update_fa(wcfe_ctx *ctx, int32_t n_nodes, const double *X, const double
     check_mesh(n_snodes, n_stris, stris);
     if (law != 0 && law != 1) fail(WCFE_ERR_ARG, "law must be 0 (linear kint) or 1 (MD table)");
     HIPCHECK(hipSetDevice(ctx->opt.device));
-    Scratch sc;
-    double *dX = sc.up(X, 3 * (size_t)n_nodes), *dx = sc.up(x, 3 * (size_t)n_nodes);
-    double *dA = sc.up(cA, (size_t)n_nodes), *dC = sc.up(cC, (size_t)n_nodes), *dF = sc.up(fau, 3 * (size_t)n_nodes);
-    int *dst = sc.up(stris, 3 * (size_t)n_stris);
-    double *dSX = sc.up(SX, 3 * (size_t)n_snodes), *dSx = sc.up(Sx, 3 * (size_t)n_snodes);
-    int *dun = sc.zeros<int>(1);
-    const PointGrid grid = upload_grid(sc, build_point_grid(n_snodes, n_stris, stris, SX));
+    Scratch sc(ctx);
+    double *dX, *dx, *dA, *dC, *dF, *dSX, *dSx;
+    int *dst, *dun, un = 0;
+    PointGrid grid;
+    const HostGrid hg = build_point_grid(n_snodes, n_stris, stris, SX);
+    sc.in(dX, X, 3 * (size_t)n_nodes);
+    sc.in(dx, x, 3 * (size_t)n_nodes);
+    sc.in(dst, stris, 3 * (size_t)n_stris);
+    sc.in(dSX, SX, 3 * (size_t)n_snodes);
+    sc.in(dSx, Sx, 3 * (size_t)n_snodes);
+    upload_grid(sc, hg, grid);
+    sc.inout(dA, cA, cA, (size_t)n_nodes);
+    sc.inout(dC, cC, cC, (size_t)n_nodes);
+    sc.inout(dF, fau, fau, 3 * (size_t)n_nodes);
+    sc.inout<int>(dun, nullptr, &un, 1);
+    sc.commit();
     launch_ref_update_fa(ctx->stream, n_nodes, dX, dx, dA, dC, dF, dt, grid, dst, dSX, dSx, law, kint, dun);
-    HIPCHECK(hipGetLastError());
-    HIPCHECK(hipStreamSynchronize(ctx->stream));
-    HIPCHECK(hipMemcpy(cA, dA, sizeof(double) * n_nodes, hipMemcpyDeviceToHost));
-    HIPCHECK(hipMemcpy(cC, dC, sizeof(double) * n_nodes, hipMemcpyDeviceToHost));
-    HIPCHECK(hipMemcpy(fau, dF, sizeof(double) * 3 * n_nodes, hipMemcpyDeviceToHost));
-    int un = 0;
-    HIPCHECK(hipMemcpy(&un, dun, sizeof(int), hipMemcpyDeviceToHost));
+    sc.fetch();
     if (n_unlocated) *n_unlocated = un;
   });
 }
@@ -3619,32 +3775,50 @@ int wcfe_force_fa_subs(wcfe_ctx *ctx, int32_t n_nodes, int32_t n_tris, const int
     HIPCHECK(hipSetDevice(ctx->opt.device));
     std::vector<int> st, li;
     one_rings(n_nodes, n_tris, tris, st, li);
-    Scratch sc;
-    int *drs = sc.up(st.data(), st.size()), *dri = sc.up(li.data(), std::max<size_t>(li.size(), 1));
-    int *dtr = sc.up(tris, 3 * (size_t)n_tris), *dst = sc.up(stris, 3 * (size_t)n_stris);
-    double *dx = sc.up(x_cell, 3 * (size_t)n_nodes), *dc = sc.up(cC, (size_t)n_nodes);
-    double *df = sc.up(fau, 3 * (size_t)n_nodes), *dSx = sc.up(Sx, 3 * (size_t)n_snodes);
-    const PointGrid grid = upload_grid(sc, build_point_grid(n_snodes, n_stris, stris, Sx));
-    int *dht = sc.zeros<int>((size_t)n_nodes * SUBS_MAX_HITS), *dnh = sc.zeros<int>((size_t)n_nodes);
-    double *dhv = sc.zeros<double>((size_t)n_nodes * SUBS_MAX_HITS * 9);
-    int *dov = sc.zeros<int>(1);
-    launch_ref_force_fa_subs(ctx->stream, n_nodes, drs, dri, dtr, dx, dc, df, grid, dst, dSx, law, kint, dht, dhv,
-                             dnh, dov);
-    HIPCHECK(hipGetLastError());
-    HIPCHECK(hipStreamSynchronize(ctx->stream));
+    Scratch sc(ctx);
+    int *drs, *dri, *dtr, *dst;
+    double *dx, *dc, *df, *dSx;
+    PointGrid grid;
+    const HostGrid hg = build_point_grid(n_snodes, n_stris, stris, Sx);
+    sc.in(drs, st.data(), st.size());
+    sc.in(dri, li.data(), li.size());
+    sc.in(dtr, tris, 3 * (size_t)n_tris);
+    sc.in(dst, stris, 3 * (size_t)n_stris);
+    sc.in(dx, x_cell, 3 * (size_t)n_nodes);
+    sc.in(dc, cC, (size_t)n_nodes);
+    sc.in(df, fau, 3 * (size_t)n_nodes);
+    sc.in(dSx, Sx, 3 * (size_t)n_snodes);
+    upload_grid(sc, hg, grid);
+    // hit k of node i at k n_nodes + i: a point lies in one or two triangles,
+    // so the first planes come back with the counts, the others if needed
+    const size_t N = (size_t)n_nodes;
+    SubsHits hits;
+    std::vector<int> nh(N), ht(SUBS_FIRST_HITS * N);
+    std::vector<double> hv(9 * ht.size());
     int ov = 0;
-    HIPCHECK(hipMemcpy(&ov, dov, sizeof(int), hipMemcpyDeviceToHost));
+    sc.inout<int>(hits.overflow, nullptr, &ov, 1);
+    sc.out(hits.n, nh.data(), N);
+    sc.out(hits.tri, ht.data(), ht.size());
+    sc.out(hits.val, hv.data(), hv.size());
+    sc.work(hits.tri_more, (SUBS_MAX_HITS - SUBS_FIRST_HITS) * N);
+    sc.work(hits.val_more, 9 * (SUBS_MAX_HITS - SUBS_FIRST_HITS) * N);
+    sc.commit();
+    launch_ref_force_fa_subs(ctx->stream, n_nodes, drs, dri, dtr, dx, dc, df, grid, dst, dSx, law, kint, hits);
+    sc.fetch();
     if (ov) fail(WCFE_ERR_ARG, "%d cell nodes lie in more than %d substrate triangles", ov, SUBS_MAX_HITS);
-    std::vector<int> ht((size_t)n_nodes * SUBS_MAX_HITS), nh(n_nodes);
-    std::vector<double> hv(ht.size() * 9);
-    HIPCHECK(hipMemcpy(ht.data(), dht, sizeof(int) * ht.size(), hipMemcpyDeviceToHost));
-    HIPCHECK(hipMemcpy(nh.data(), dnh, sizeof(int) * nh.size(), hipMemcpyDeviceToHost));
-    HIPCHECK(hipMemcpy(hv.data(), dhv, sizeof(double) * hv.size(), hipMemcpyDeviceToHost));
+    const int most = *std::max_element(nh.begin(), nh.end());
+    if (most > SUBS_FIRST_HITS) {
+      const size_t m = (size_t)(most - SUBS_FIRST_HITS) * N, o = ht.size();
+      ht.resize(o + m);
+      hv.resize(9 * (o + m));
+      HIPCHECK(hipMemcpy(ht.data() + o, hits.tri_more, sizeof(int) * m, hipMemcpyDeviceToHost));
+      HIPCHECK(hipMemcpy(hv.data() + 9 * o, hits.val_more, sizeof(double) * 9 * m, hipMemcpyDeviceToHost));
+    }
     // the reference's accumulation order: cell node, then triangle, ascending
     std::fill(F, F + 3 * (size_t)n_snodes, 0.0);
     for (int i = 0; i < n_nodes; ++i)
       for (int k = 0; k < nh[i]; ++k) {
-        const size_t hk = (size_t)i * SUBS_MAX_HITS + k;
+        const size_t hk = (size_t)k * N + i;
         const int32_t *t = stris + 3 * (size_t)ht[hk];
         for (int a = 0; a < 3; ++a)
           for (int c = 0; c < 3; ++c) F[3 * (size_t)t[a] + c] += hv[9 * hk + 3 * a + c];
@@ -3672,13 +3846,15 @@ int wcfe_area_tot(wcfe_ctx *ctx, int32_t n_nodes, int32_t n_tris, const int32_t 
     check_mesh(n_nodes, n_tris, tris);
     if (n_tris <= 0) fail(WCFE_ERR_ARG, "no triangles");
     HIPCHECK(hipSetDevice(ctx->opt.device));
-    Scratch sc;
-    int *dtr = sc.up(tris, 3 * (size_t)n_tris);
-    double *dx = sc.up(x, 3 * (size_t)n_nodes), *dout = sc.zeros<double>(4);
+    Scratch sc(ctx);
+    int *dtr;
+    double *dx, *dout;
+    sc.in(dtr, tris, 3 * (size_t)n_tris);
+    sc.in(dx, x, 3 * (size_t)n_nodes);
+    sc.out(dout, out, 4);
+    sc.commit();
     launch_ref_area_tot(ctx->stream, n_tris, dtr, dx, dout);
-    HIPCHECK(hipGetLastError());
-    HIPCHECK(hipStreamSynchronize(ctx->stream));
-    HIPCHECK(hipMemcpy(out, dout, sizeof(double) * 4, hipMemcpyDeviceToHost));
+    sc.fetch();
   });
 }
 
@@ -3696,18 +3872,19 @@ int ref_boundary_call(wcfe_ctx *ctx, int which, int n_nodes, int n_tris, const i
     std::vector<int> cst;
     std::vector<int2> cand;
     boundary_candidates(n_nodes, n_tris, tris, cst, cand);
-    Scratch sc;
-    int *dcs = sc.up(cst.data(), cst.size());
-    int2 *dca = sc.up(cand.data(), cand.size());
-    double *dx = sc.up(x, 3 * (size_t)n_nodes), *dF = sc.zeros<double>(3 * (size_t)n_nodes);
-    double *du = u ? sc.up(u, (size_t)n_nodes) : nullptr;
-    int *dopen = sc.zeros<int>(1);
+    Scratch sc(ctx);
+    int *dcs, *dopen, op = 0;
+    int2 *dca;
+    double *dx, *du = nullptr, *dF;
+    sc.in(dcs, cst.data(), cst.size());
+    sc.in(dca, cand.data(), cand.size());
+    sc.in(dx, x, 3 * (size_t)n_nodes);
+    if (u) sc.in(du, u, (size_t)n_nodes);
+    sc.inout<double>(dF, nullptr, F, 3 * (size_t)n_nodes);
+    sc.inout<int>(dopen, nullptr, &op, 1);
+    sc.commit();
     launch_ref_boundary(ctx->stream, which, n_nodes, dcs, dca, dx, a, du, dF, dopen);
-    HIPCHECK(hipGetLastError());
-    HIPCHECK(hipStreamSynchronize(ctx->stream));
-    HIPCHECK(hipMemcpy(F, dF, sizeof(double) * 3 * n_nodes, hipMemcpyDeviceToHost));
-    int op = 0;
-    HIPCHECK(hipMemcpy(&op, dopen, sizeof(int), hipMemcpyDeviceToHost));
+    sc.fetch();
     if (n_open) *n_open = op;
   });
 }
@@ -3848,7 +4025,6 @@ int wcfe_remesh_cell(wcfe_ctx *ctx, int32_t cell, int32_t n_nodes, int32_t n_tri
     }
     // the cell's new nodes from its old ones, on the device
     HIPCHECK(hipStreamSynchronize(ctx->stream));
-    Scratch sc;
     std::vector<int> s0(n_nodes), s1(n_nodes);
     std::vector<double> ww(n_nodes, 1.0);
     for (int i = 0; i < n_nodes; ++i) {
@@ -3856,28 +4032,42 @@ int wcfe_remesh_cell(wcfe_ctx *ctx, int32_t cell, int32_t n_nodes, int32_t n_tri
       s1[i] = src1 ? src1[i] : i;
       if (w) ww[i] = w[i];
     }
-    const int *ds0 = sc.up(s0.data(), s0.size()), *ds1 = sc.up(s1.data(), s1.size());
-    const double *dw = sc.up(ww.data(), ww.size());
-    double2 *Xn = sc.zeros<double2>(n_nodes), *xn = sc.zeros<double2>(n_nodes), *fn = sc.zeros<double2>(n_nodes);
-    double *en = sc.zeros<double>(3 * (size_t)n_nodes), *cn = sc.zeros<double>(n_nodes);
+    std::vector<double2> Xh(n_nodes), xh(n_nodes), fh(n_nodes);
+    std::vector<double> eh(3 * (size_t)n_nodes), ch(n_nodes);
+    Scratch sc(ctx);
+    int *ds0, *ds1;
+    double *dw, *en, *cn;
+    double2 *Xn, *xn, *fn;
+    sc.in(ds0, s0.data(), s0.size());
+    sc.in(ds1, s1.data(), s1.size());
+    sc.in(dw, ww.data(), ww.size());
+    sc.out(Xn, Xh.data(), Xh.size());
+    sc.out(xn, xh.data(), xh.size());
+    sc.out(fn, fh.data(), fh.size());
+    sc.out(en, eh.data(), eh.size());
+    sc.out(cn, ch.data(), ch.size());
+    sc.commit();
     launch_remap_nodes(ctx->stream, n_nodes, ds0, ds1, dw, p.node_off, b.X, b.x, b.ea, b.cC, b.fau, Xn, xn, en, cn, fn);
-    HIPCHECK(hipGetLastError());
+    sc.fetch();
     state_to_host(ctx);  // every cell's state (this cell's springs too)
     HostCell h = old;
     h.n_nodes = n_nodes;
     h.n_tris = n_tris;
     h.tris.assign(tris, tris + 3LL * n_tris);
     h.topo_hash = hash;
-    h.X.resize(2 * (size_t)n_nodes);
-    h.x.resize(2 * (size_t)n_nodes);
-    h.ea.resize(3 * (size_t)n_nodes);
-    h.cC.resize(n_nodes);
-    h.fau.resize(2 * (size_t)n_nodes);
-    HIPCHECK(hipMemcpy(h.X.data(), Xn, sizeof(double2) * n_nodes, hipMemcpyDeviceToHost));
-    HIPCHECK(hipMemcpy(h.x.data(), xn, sizeof(double2) * n_nodes, hipMemcpyDeviceToHost));
-    HIPCHECK(hipMemcpy(h.ea.data(), en, sizeof(double) * 3 * n_nodes, hipMemcpyDeviceToHost));
-    HIPCHECK(hipMemcpy(h.cC.data(), cn, sizeof(double) * n_nodes, hipMemcpyDeviceToHost));
-    HIPCHECK(hipMemcpy(h.fau.data(), fn, sizeof(double2) * n_nodes, hipMemcpyDeviceToHost));
+    auto flat = [&](const std::vector<double2> &v) {
+      std::vector<double> o(2 * v.size());
+      for (size_t i = 0; i < v.size(); ++i) {
+        o[2 * i] = v[i].x;
+        o[2 * i + 1] = v[i].y;
+      }
+      return o;
+    };
+    h.X = flat(Xh);
+    h.x = flat(xh);
+    h.fau = flat(fh);
+    h.ea = eh;
+    h.cC = ch;
     if (x_new) h.x.assign(x_new, x_new + 2 * (size_t)n_nodes);
     if (!h.f_ext.empty()) {  // a constant load per node does not interpolate: the host sets it again
       h.f_ext.assign(2 * (size_t)n_nodes, 0.0);

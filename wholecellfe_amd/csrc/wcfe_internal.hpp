@@ -43,6 +43,10 @@ template <class T>
 void launch_assemble_gather(hipStream_t s, const View &v, int e_begin, int e_end, int mode, const int *node_cell,
                             const int *adj_start, const int *adj, const GatherPlan &gp, int n0, int n1, double *Ge,
                             double *Ke64, double *G, T *K, T *Kb, int lower_only);
+// UL strain increments and lumped masses: every node of the range over its
+// elements in element order (node_cell null: cell 0; else converged UL cells)
+void launch_node_strain(hipStream_t s, const View &v, const int *node_cell, const int *adj_start, const int *adj,
+                        int n0, int n1, double *Rea, double *MM);
 void launch_element_dump(hipStream_t s, const View &v, int e_begin, int e_end, double *Ge, double *Ke);
 // per-cell norms of cells above NORM_CHUNK entries: partial sums per chunk
 // (stride per cell = the batch's largest chunk count) and an arrival counter
@@ -284,10 +288,20 @@ constexpr int SUBS_MAX_HITS = 16;  // containing substrate triangles per cell no
 void launch_ref_update_fa(hipStream_t s, int n_nodes, const double *X, const double *x, double *cA, double *cC,
                           double *fau, double dt, const PointGrid &grid, const int *stris, const double *SX,
                           const double *Sx, int law, double kint, int *n_unlocated);
+// substrate hits: hit k of node i at k n_nodes + i, the first SUBS_FIRST_HITS
+// planes apart from the others; 9 values per hit
+constexpr int SUBS_FIRST_HITS = 2;
+struct SubsHits {
+  int *n, *overflow, *tri, *tri_more;
+  double *val, *val_more;
+};
 void launch_ref_force_fa_subs(hipStream_t s, int n_nodes, const int *ring_start, const int *ring, const int *tris,
                               const double *x_cell, const double *cC, const double *fau, const PointGrid &grid,
-                              const int *stris, const double *Sx, int law, double kint, int *hit_tri,
-                              double *hit_val, int *n_hits, int *overflow);
+                              const int *stris, const double *Sx, int law, double kint, const SubsHits &hits);
+// K from the caller's dense matrices (FP64, packed), identity in the padding
+template <class T>
+void launch_dense_load(hipStream_t s, const CellParams *cp, int n_sys, int max_npad, const double *A64,
+                       const long long *a_off, T *K);
 void launch_dense_residual(hipStream_t s, const CellParams *cp, const CellState *cs, const int *cells, int ncell,
                            int max_ndof, const double *A64, const long long *a_off, const double *b, const double *x,
                            double *r);
