@@ -69,3 +69,19 @@ def test_area_term_in_the_band_equals_the_full_matrix(K, prec):
     assert np.abs(Ks - Kf).max() <= 1e-12 * np.abs(Kf).max()  # the same sums, rounded alike
     # relative residual 1e-12 at a condition number below 1e6
     assert np.linalg.norm(xs - xf) <= 1e-6 * np.linalg.norm(xf - np.asarray(d["x"]).ravel())
+
+
+# 7994 and 8438 unknowns: one and two partial sums of the norms
+@pytest.mark.parametrize("K", [36, 37])
+def test_norms_of_large_cells(K):
+    print("case norm", K, flush=True)
+    d = cells.cst_cell(K=K, n_spr=500, seed=K, time=1.0)
+    # tolerances of zero: the load step stays open, its residual at time t0
+    with W.Context(t0=1.0, newton_rtol=0.0, newton_atol=0.0) as c:
+        cells.add_to_context(c, d)
+        c.finalize()
+        g0 = np.linalg.norm(c.residual(0))
+        st = c.newton_step()
+        g1 = np.linalg.norm(c.residual(0))
+    # 8438 rounded squares, and the residual summed in another order
+    assert abs(st["max_newton_rel"] - g1 / g0) <= 1e-9 * (g1 / g0) + 1e-15

@@ -55,10 +55,11 @@ void launch_fill_systems(hipStream_t s, const CellParams *cp, const int *cells, 
                          const int *rank, int lower_only) {
   if (ncell <= 0) return;
   // 16 (FP64: 8) rows per workgroup and pass; at most 64 workgroups per cell
-  // (the largest cells loop) so that small cells launch few empty ones
+  // of a large batch (the largest cells loop) so that small cells launch few
+  // empty ones, and 2048 together of a small one (one cell of 20600 rows: 42 us
+  // on 64 workgroups, 8 on 1284)
   const int rows = 4 * Vec16<T>::n;
-  int gx = (max_npad + rows - 1) / rows < 64 ? (max_npad + rows - 1) / rows : 64;
-  if (gx < 1) gx = 1;
+  const int gx = std::max(1, std::min((max_npad + rows - 1) / rows, std::max(64, 2048 / ncell)));
   hipLaunchKernelGGL(k_fill_systems<T>, dim3(gx, ncell), dim3(256), 0, s, cp, cells, ncell, K, rank, lower_only);
 }
 template void launch_fill_systems<float>(hipStream_t, const CellParams *, const int *, int, int, float *, const int *,
@@ -354,14 +355,14 @@ void launch_element_dump(hipStream_t s, const View &v, int e_begin, int e_end, d
 //        iterate), 1 = refinement residual (rnorm), 2 = residual after the
 //        update (gnorm)
 // ---------------------------------------------------------------------------
-// One workgroup per cell (blockIdx.x) and chunk of NORM_CHUNK entries
-// (blockIdx.y).  A cell of one chunk is summed by its one workgroup; a larger
+// One workgroup per cell (blockIdx.x) and chunk (norm_chunks; blockIdx.y).  A cell of one chunk is summed by its one workgroup; a larger
 // cell's chunks write partial sums and the last chunk to arrive adds them in
 // chunk order (fixed order: bitwise reproducible).
 // K (which 0, dense cells): also the factorization's pivot threshold from the
-// diagonal.  Bound by latency: 16 waves, four entries of both in flight each
-// (10300 nodes: 10 + 28 us as a norm and a threshold kernel of 4 waves).
-constexpr int NORM_THREADS = 1024;
+// diagonal.  Bound by latency: 16 waves, NORM_U entries of both in flight each
+// (10300 nodes: 10 + 28 us as a norm and a threshold kernel of 4 waves, four
+// entries in flight; now 7).
+constexpr int NORM_THREADS = 1024, NORM_U = 8;
 template <class T>
 __global__ __launch_bounds__(NORM_THREADS) void k_cell_norm(const CellParams *cp, CellState *cs, const int *cells,
                                                             const double *vec, int which, int only_active,
@@ -369,35 +370,38 @@ __global__ __launch_bounds__(NORM_THREADS) void k_cell_norm(const CellParams *cp
   const int c = cells[blockIdx.x];
   const CellParams &p = cp[c];
   if (only_active && (cs[c].ir_done || p.refine)) return;
-  const int nch = nw.part ? (p.ndof + NORM_CHUNK - 1) / NORM_CHUNK : 1;
+  const int nch = nw.part ? norm_chunks(p.ndof) : 1;
+  const int per = (p.ndof + nch - 1) / nch;
   const int chunk = blockIdx.y;
   if (chunk >= nch) return;
   const double *v = vec + (long long)p.vec_off;
-  const int lo = nch > 1 ? chunk * NORM_CHUNK : 0;
-  const int hi = nch > 1 ? min(p.ndof, lo + NORM_CHUNK) : p.ndof;
+  const int lo = chunk * per, hi = min(p.ndof, lo + per);
   const bool tau = K && !p.csr;
   const T *A = K + p.k_off;
-  double acc[4] = {0.0, 0.0, 0.0, 0.0}, m = 0.0;
-  for (int i0 = lo + threadIdx.x; i0 < hi; i0 += 4 * NORM_THREADS) {
-    T d[4] = {T(0), T(0), T(0), T(0)};
-    if (tau) {
+  double acc[NORM_U], m = 0.0;
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const long long i = min(i0 + NORM_THREADS * u, hi - 1);
-        d[u] = A[i * p.npad + i];
-      }
+  for (int u = 0; u < NORM_U; ++u) acc[u] = 0.0;
+  for (int i0 = lo + threadIdx.x; i0 < hi; i0 += NORM_U * NORM_THREADS) {
+    T d[NORM_U];
+    double x[NORM_U];
+#pragma unroll
+    for (int u = 0; u < NORM_U; ++u) {
+      const long long i = min(i0 + NORM_THREADS * u, hi - 1);
+      x[u] = v[i];
+      d[u] = tau ? A[i * p.npad + i] : T(0);
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int i = i0 + NORM_THREADS * u;
-      const double x = i < hi ? v[i] : 0.0;
-      acc[u] += x * x;
+    for (int u = 0; u < NORM_U; ++u) {
+      if (i0 + NORM_THREADS * u < hi) acc[u] += x[u] * x[u];
+      m = fmax(m, fabs((double)d[u]));  // fmax: a NaN is left out
     }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) m = fmax(m, fabs((double)d[u]));  // fmax: a NaN is left out
   }
+#pragma unroll
+  for (int w = NORM_U / 2; w > 0; w >>= 1)
+#pragma unroll
+    for (int u = 0; u < w; ++u) acc[u] += acc[u + w];
   __shared__ double red[NORM_THREADS], redm[NORM_THREADS];
-  red[threadIdx.x] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+  red[threadIdx.x] = acc[0];
   redm[threadIdx.x] = m;
   __syncthreads();
   for (int w = NORM_THREADS / 2; w > 0; w >>= 1) {

@@ -101,13 +101,19 @@ __global__ __launch_bounds__(CG_ROWS) void k_pcg_init(const int4 *chunks, const 
 // LANES / 4 passes.  The lane sums: xor butterfly (every lane gets the same
 // bits); the partial sums: per thread over its passes in order, xor butterfly
 // over a wave's rows, then the waves by a fixed tree (bitwise reproducible).
-constexpr int SPMV_THREADS = 1024;
+// Bound by latency: row_ptr, then col, then u and the block, each a round
+// trip, 16 waves per compute unit.  SPMV_U passes go through each of them
+// together (one pass after the other 12 us for 250,000 rows, so 10, of which
+// the launch and three round trips are about 6); 4 waves per SIMD keep the
+// compiler from trading the loads in flight for registers.
+constexpr int SPMV_THREADS = 1024, SPMV_U = 4;
 template <class T, int LANES>
-__global__ __launch_bounds__(SPMV_THREADS) void k_pcg_spmv_dot(const int4 *chunks, int cbase, const CgState *cg,
+__global__ __launch_bounds__(SPMV_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_pcg_spmv_dot(const int4 *chunks, int cbase, const CgState *cg,
                                                                const int *row_ptr, const int *col, const T *val,
                                                                const T *r, const T *u, T *w, double *partials,
                                                                long long pstride) {
   constexpr int NW = SPMV_THREADS / 64, RPP = SPMV_THREADS / LANES;
+  constexpr int FIRST = LANES == 4 ? 2 : 1;  // blocks of a row a lane always asks for (a planar mesh has about 7)
   static_assert(CG_ROWS % RPP == 0, "a chunk is a whole number of passes");
   __shared__ double red[3][NW];
   const int4 ch = chunks[blockIdx.x];
@@ -120,33 +126,65 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_pcg_spmv_dot(const int4 *chunk
   v2 *w2 = reinterpret_cast<v2 *>(w);
   const int lane = threadIdx.x & 63, slot = threadIdx.x & (LANES - 1), wave = threadIdx.x >> 6;
   double ru = 0.0, wu = 0.0, rr = 0.0;
+#pragma unroll 1
+  for (int pass0 = 0; pass0 < CG_ROWS / RPP; pass0 += SPMV_U) {
+    int i[SPMV_U], ks[SPMV_U], ke[SPMV_U], cj[SPMV_U][FIRST];
+    T y0[SPMV_U], y1[SPMV_U];
 #pragma unroll
-  for (int pass = 0; pass < CG_ROWS / RPP; ++pass) {
-    const int i = ch.y + pass * RPP + threadIdx.x / LANES;
-    T y0 = T(0), y1 = T(0);
-    if (i < ch.z) {
-      const int ke = row_ptr[i + 1];
-      for (int k = row_ptr[i] + slot; k < ke; k += LANES) {
-        const v2 uj = u2[col[k]];
-        const v4 B = B4[k];
-        y0 += B.x * uj.x + B.y * uj.y;
-        y1 += B.z * uj.x + B.w * uj.y;
+    for (int q = 0; q < SPMV_U; ++q) {
+      i[q] = ch.y + (pass0 + q) * RPP + threadIdx.x / LANES;
+      const int ii = min(i[q], ch.z - 1);
+      ks[q] = row_ptr[ii] + slot;
+      ke[q] = i[q] < ch.z ? row_ptr[ii + 1] : 0;
+    }
+#pragma unroll
+    for (int q = 0; q < SPMV_U; ++q)
+#pragma unroll
+      for (int f = 0; f < FIRST; ++f) cj[q][f] = col[ks[q] + f * LANES < ke[q] ? ks[q] + f * LANES : 0];
+    __builtin_amdgcn_sched_barrier(0);
+    v2 uj[SPMV_U][FIRST];
+    v4 B[SPMV_U][FIRST];
+#pragma unroll
+    for (int q = 0; q < SPMV_U; ++q)
+#pragma unroll
+      for (int f = 0; f < FIRST; ++f) {
+        B[q][f] = B4[ks[q] + f * LANES < ke[q] ? ks[q] + f * LANES : 0];
+        uj[q][f] = u2[cj[q][f]];
+      }
+    __builtin_amdgcn_sched_barrier(0);  // every load before the first use
+#pragma unroll
+    for (int q = 0; q < SPMV_U; ++q) {
+      y0[q] = y1[q] = T(0);
+#pragma unroll
+      for (int f = 0; f < FIRST; ++f) {
+        if (ks[q] + f * LANES >= ke[q]) continue;
+        y0[q] += B[q][f].x * uj[q][f].x + B[q][f].y * uj[q][f].y;
+        y1[q] += B[q][f].z * uj[q][f].x + B[q][f].w * uj[q][f].y;
+      }
+      for (int k = ks[q] + FIRST * LANES; k < ke[q]; k += LANES) {
+        const v2 ur = u2[col[k]];
+        const v4 Br = B4[k];
+        y0[q] += Br.x * ur.x + Br.y * ur.y;
+        y1[q] += Br.z * ur.x + Br.w * ur.y;
       }
     }
 #pragma unroll
-    for (int o = 1; o < LANES; o <<= 1) {
-      y0 += __shfl_xor(y0, o);
-      y1 += __shfl_xor(y1, o);
-    }
-    if (slot == 0 && i < ch.z) {
-      v2 wi;
-      wi.x = y0;
-      wi.y = y1;
-      w2[i] = wi;
-      const v2 ui = u2[i], ri = r2[i];
-      ru += (double)(ri.x * ui.x + ri.y * ui.y);
-      wu += (double)(y0 * ui.x + y1 * ui.y);
-      rr += (double)(ri.x * ri.x + ri.y * ri.y);
+    for (int q = 0; q < SPMV_U; ++q) {
+#pragma unroll
+      for (int o = 1; o < LANES; o <<= 1) {
+        y0[q] += __shfl_xor(y0[q], o);
+        y1[q] += __shfl_xor(y1[q], o);
+      }
+      if (slot == 0 && i[q] < ch.z) {
+        v2 wi;
+        wi.x = y0[q];
+        wi.y = y1[q];
+        w2[i[q]] = wi;
+        const v2 ui = u2[i[q]], ri = r2[i[q]];
+        ru += (double)(ri.x * ui.x + ri.y * ui.y);
+        wu += (double)(y0[q] * ui.x + y1[q] * ui.y);
+        rr += (double)(ri.x * ri.x + ri.y * ri.y);
+      }
     }
   }
 #pragma unroll

@@ -1597,7 +1597,7 @@ void build_batch(wcfe_ctx *ctx, Batch &b, const std::vector<HostCell> &hc, int e
     int max_ndof = 0;
     for (int c = 0; c < b.ncell; ++c) max_ndof = std::max(max_ndof, b.cp_h[c].ndof);
     if (max_ndof > NORM_CHUNK) {
-      b.norm_stride = (max_ndof + NORM_CHUNK - 1) / NORM_CHUNK;
+      b.norm_stride = norm_chunks(max_ndof);
       b.norm_part = dalloc<double>(2 * (size_t)b.ncell * b.norm_stride);
       b.norm_cnt = dalloc<unsigned>(b.ncell);
       HIPCHECK(hipMemset(b.norm_cnt, 0, sizeof(unsigned) * b.ncell));
