@@ -173,7 +173,30 @@ static void check(int n, int bw, int sym, int cuts, std::mt19937 &rng) {
   if (P.top.nloc) sweep(P.top, x, x, sl, d, false);
   for (const SweepPart &S : P.bwd) sweep(S, x, x, sl, d, false);
   solved(d, "refinement solve");
+  if (P.root.nloc) {  // separator by separator
+    x.assign(N, NAN);
+    d.assign(N, NAN);
+    sweep(P.root_bwd, y, x, sl, d, true);
+    for (const auto &level : P.sep_bwd)
+      for (const SweepPart &S : level) sweep(S, y, x, sl, d, true);
+    for (const SweepPart &S : P.bwd) sweep(S, y, x, sl, d, true);
+    solved(d, "first solve by separators");
+    x.assign(N, NAN);
+    d.assign(N, NAN);
+    sl.assign(P.nslot * B, NAN);
+    for (const SweepPart &S : P.fwd) sweep(S, x, x, sl, d, false);
+    for (size_t q = P.sep_fwd.size(); q-- > 0;)
+      for (const SweepPart &S : P.sep_fwd[q]) sweep(S, x, x, sl, d, false);
+    sweep(P.root, x, x, sl, d, false);
+    for (const auto &level : P.sep_bwd)
+      for (const SweepPart &S : level) sweep(S, x, x, sl, d, false);
+    for (const SweepPart &S : P.bwd) sweep(S, x, x, sl, d, false);
+    solved(d, "refinement solve by separators");
+  }
   if (P.whole.nloc) {
+    d.assign(N, NAN);
+    sweep(P.whole_bwd, y, x, sl, d, true);
+    solved(d, "first solve in one part");
     d.assign(N, NAN);
     sweep(P.whole, x, x, sl, d, false);
     solved(d, "one-part solve");

@@ -85,3 +85,22 @@ def test_norms_of_large_cells(K):
         g1 = np.linalg.norm(c.residual(0))
     # 8438 rounded squares, and the residual summed in another order
     assert abs(st["max_newton_rel"] - g1 / g0) <= 1e-9 * (g1 / g0) + 1e-15
+
+
+# 9600 and 15000 elements alone: a band cut deep enough that the separators are
+# swept by depth, against the uncut band
+@pytest.mark.parametrize("prec", [W.PREC_MIXED, W.PREC_FP64])
+@pytest.mark.parametrize("sym", [1, 0])
+@pytest.mark.parametrize("K", [40, 50])
+def test_separators_by_depth_equal_the_uncut_band(K, sym, prec):
+    print("case depth", K, sym, prec, flush=True)
+    d = cells.cst_cell(K=K, n_spr=400, seed=K, time=1.0)
+    out = []
+    for twist in (1, 0):
+        with W.Context(precision=prec, t0=1.0, symmetric=sym, twist=twist, lin_rtol=1e-12, max_refine=8) as c:
+            cells.add_to_context(c, d)
+            c.finalize()
+            c.newton_step()
+            out.append(c.positions(0))
+    # relative residual 1e-12 at a condition number below 1e6
+    assert np.linalg.norm(out[0] - out[1]) <= 1e-6 * np.linalg.norm(out[1] - d["x"])

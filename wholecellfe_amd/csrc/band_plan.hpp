@@ -84,10 +84,12 @@ struct BandPlan {
   std::vector<BlockRef> refs;
   std::vector<FwdOp> fops;
   // sweeps: per leaf its forward and backward part; the separators' part
-  // (forward and backward, or backward only); the whole sweep by one
-  // workgroup (likewise)
+  // (forward and backward, or backward only), or (three and more separators)
+  // one part per separator, by the number of cuts above it, the first cut's
+  // forward and backward in one; the whole sweep by one workgroup
   std::vector<SweepPart> fwd, bwd;
-  SweepPart top, top_bwd, whole, whole_bwd;
+  SweepPart top, top_bwd, root, root_bwd, whole, whole_bwd;
+  std::vector<std::vector<SweepPart>> sep_fwd, sep_bwd;  // [0] empty
   std::vector<SweepOp> ops;
   std::vector<SweepLoc> locs;
   std::vector<int> accs;
@@ -95,7 +97,7 @@ struct BandPlan {
 
 namespace band_detail {
 struct Node {
-  int lo, hi, desc, leaf, start;
+  int lo, hi, desc, leaf, start, lvl;  // lvl: cuts above it
 };
 // last level of a band of len blocks cut `depth` times, and the left part's length
 inline int last_level(int len, int depth, int bw, std::map<std::pair<int, int>, std::pair<int, int>> &memo) {
@@ -116,19 +118,19 @@ inline int last_level(int len, int depth, int bw, std::map<std::pair<int, int>, 
   return best;
 }
 inline int cut(std::vector<Node> &nodes, int lo, int hi, int depth, int bw, bool hasl, bool hasr,
-               std::map<std::pair<int, int>, std::pair<int, int>> &memo) {
+               std::map<std::pair<int, int>, std::pair<int, int>> &memo, int lvl = 0) {
   const int len = hi - lo;
   last_level(len, depth, bw, memo);
   auto it = memo.find({len, depth});
   if (depth == 0 || it == memo.end() || it->second.second == 0) {
-    nodes.push_back(Node{lo, hi, hasl && !hasr ? 1 : 0, 1, 0});
+    nodes.push_back(Node{lo, hi, hasl && !hasr ? 1 : 0, 1, 0, lvl});
     return len - 1;
   }
   const int a = it->second.second, m = lo + a;
-  const int l = cut(nodes, lo, m, depth - 1, bw, hasl, true, memo);
-  const int r = cut(nodes, m + bw, hi, depth - 1, bw, true, hasr, memo);
+  const int l = cut(nodes, lo, m, depth - 1, bw, hasl, true, memo, lvl + 1);
+  const int r = cut(nodes, m + bw, hi, depth - 1, bw, true, hasr, memo, lvl + 1);
   const int start = std::max(l, r) + (l == r ? 2 : 1);
-  nodes.push_back(Node{m, m + bw, 0, 0, start});
+  nodes.push_back(Node{m, m + bw, 0, 0, start, lvl});
   return start + bw - 1;
 }
 }  // namespace band_detail
@@ -339,6 +341,65 @@ inline BandPlan make_band_plan(int n, int bw, bool sym, int depth) {
     bwd_rows(mine[v]);
     part(b, o0, l0);
     P.bwd.push_back(b);
+  }
+  // separator by separator, the deepest first
+  int depth_of = 0, nsep = 0;
+  for (const Node &d : nodes)
+    if (!d.leaf) {
+      depth_of = std::max(depth_of, d.lvl);
+      ++nsep;
+    }
+  if (nsep >= 3) {
+    P.sep_fwd.resize(depth_of + 1);
+    P.sep_bwd.resize(depth_of + 1);
+    std::vector<std::vector<int>> exts(nn);
+    for (int v = 0; v < nn; ++v)
+      for (int t : mine[v])
+        for (int i : st[t])
+          if (node_of[i] != v && std::find(exts[v].begin(), exts[v].end(), i) == exts[v].end()) exts[v].push_back(i);
+    auto own_cols = [&](int i, int v) {
+      std::vector<int> cols;
+      for (int t : pre[i])
+        if (node_of[t] == v) cols.push_back(t);
+      return cols;
+    };
+    for (int lvl = depth_of; lvl >= 0; --lvl)
+      for (int v = 0; v < nn; ++v) {
+        if (nodes[v].leaf || nodes[v].lvl != lvl) continue;
+        // forward: the right-hand side minus what every part below left for its rows
+        int o0 = (int)P.ops.size(), l0 = (int)P.locs.size();
+        for (int b : mine[v]) {
+          add_loc(b, SL_RHS, lvl == 0 ? SL_OUT_Y | SL_OUT_D : SL_OUT_Y, l0);
+          for (int u = 0; u < nn; ++u)
+            if (u != v && std::find(exts[u].begin(), exts[u].end(), b) != exts[u].end()) {
+              P.accs.push_back(slot_of(u, b));
+              ++P.locs.back().nacc;
+            }
+        }
+        for (int b : mine[v]) row(b, own_cols(b, v), SW_FWD, local[b]);
+        if (lvl == 0) {
+          const int o1 = (int)P.ops.size();
+          bwd_rows(mine[v]);
+          part(P.root, o0, l0);
+          part(P.root_bwd, o1, l0);
+          continue;
+        }
+        for (int i : exts[v]) {
+          int &sl = slot_of(v, i);
+          if (sl < 0) sl = P.nslot++;
+          row(i, own_cols(i, v), SW_ACC, sl);
+        }
+        SweepPart f, b;
+        part(f, o0, l0);
+        P.sep_fwd[lvl].push_back(f);
+        o0 = (int)P.ops.size();
+        l0 = (int)P.locs.size();
+        for (int t : mine[v]) add_loc(t, SL_Y, SL_OUT_Y | SL_OUT_D, l0);
+        for (int i : exts[v]) add_loc(i, SL_X, 0, l0);
+        bwd_rows(mine[v]);
+        part(b, o0, l0);
+        P.sep_bwd[lvl].push_back(b);
+      }
   }
   {
     const int o0 = (int)P.ops.size(), l0 = (int)P.locs.size();

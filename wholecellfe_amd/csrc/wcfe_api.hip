@@ -12,6 +12,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <set>
 #include <memory>
 #include <string>
 #include <thread>
@@ -706,8 +707,10 @@ struct Batch {
   };
   struct SweepLists {
     SweepList fwd, top, top_bwd, bwd, whole;
+    std::vector<SweepList> sep_fwd, sep_bwd;  // separators below the first cut, by depth (by_level)
     bool split = false;
   };
+  bool by_level = false;  // separators swept by depth instead of by one workgroup per cell
   SweepLists sweeps;                    // every cell
   std::vector<SweepLists> sweeps_cell;  // one cell's (per-cell Newton steps)
   // cells whose refinement one workgroup runs: whole (CellParams::refine), then
@@ -863,6 +866,8 @@ template <class F> int guarded(wcfe_ctx *ctx, F &&f) {
     return set_err(ctx, WCFE_ERR_HIP, std::string(e.what) + ": " + hipGetErrorString(e.e));
   } catch (const std::bad_alloc &) {
     return set_err(ctx, WCFE_ERR_OOM, "host allocation failed");
+  } catch (const std::exception &e) {
+    return set_err(ctx, WCFE_ERR_STATE, e.what());
   }
 }
 
@@ -943,6 +948,9 @@ template <class F> void parallel_cells(int ncell, F f) {
 // one FP64.
 double step_slots(const wcfe_ctx *ctx, int elem_size) { return (elem_size == 4 ? 1.0 : 0.75) * ctx->n_cu; }
 
+// time of one block product of a sweep's stream
+double sweep_op_us(int elem_size) { return elem_size == 8 ? 0.5 : 0.25; }
+
 // Which cells' bands are cut, and how deep (band_plan.hpp).  A cut halves a
 // cell's chain of dependent block steps and adds the fill of the separators:
 // about twice the products of that cell.  A batch takes as many launches as
@@ -1000,7 +1008,7 @@ void plan_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
         if (!b.cp_h[c].csr && b.cp_h[c].nblk > chain2) depth[c] = 1;
     } else {
       const int f64 = elem_size == 8;
-      const double t_op = f64 ? 0.5 : 0.25, slots = step_slots(ctx, elem_size);
+      const double t_op = sweep_op_us(elem_size), slots = step_slots(ctx, elem_size);
       // cells of one shape count once
       std::map<std::array<int, 3>, int> shapes;
       for (const CellParams &p : b.cp_h)
@@ -1010,6 +1018,28 @@ void plan_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
         for (int d = 0; d <= MAX_CUTS; ++d) cand.push_back(band_steps(sh.first[0], sh.first[1], d));
       std::sort(cand.begin(), cand.end());
       cand.erase(std::unique(cand.begin(), cand.end()), cand.end());
+      {  // the plans the candidates ask for, on the host's threads
+        std::set<std::array<int, 4>> need;
+        for (int C : cand)
+          for (auto &sh : shapes) {
+            CellParams p{};
+            p.nblk = sh.first[0];
+            p.bw = sh.first[1];
+            p.sym = sh.first[2];
+            need.insert({p.nblk, p.bw, p.sym, cuts_for(p, C, MAX_CUTS)});
+          }
+        std::vector<std::pair<std::array<int, 4>, std::shared_ptr<BandPlan>>> todo;
+        for (auto it = need.rbegin(); it != need.rend(); ++it) todo.push_back({*it, nullptr});  // largest first
+        parallel_cells((int)todo.size(), [&](int i) {
+          const std::array<int, 4> &k = todo[i].first;
+          try {
+            todo[i].second = std::make_shared<BandPlan>(make_band_plan(k[0], k[1], k[2] != 0, k[3]));
+          } catch (...) {  // made again below, where the caller can see the exception
+          }
+        });
+        for (auto &t : todo)
+          if (t.second) made[t.first] = t.second;
+      }
       double best = 1e300;
       int best_c = INT_MAX;
       for (int C : cand) {
@@ -1032,7 +1062,11 @@ void plan_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
             w = std::max(w, P->bwd[q].nop);
           }
           split |= P->top.nop > 0;
-          sweep = std::max(sweep, t_op * (f + 2.0 * w + P->top.nop + P->top_bwd.nop));
+          double top = t_op * (P->top.nop + P->top_bwd.nop), apart = t_op * (P->root.nop + P->root_bwd.nop);
+          for (size_t q = 1; q < P->sep_fwd.size(); ++q)
+            apart += 15.0 + t_op * (P->sep_fwd[q][0].nop + 2.0 * P->sep_bwd[q][0].nop);
+          if (P->root.nloc > 0) top = std::min(top, apart);
+          sweep = std::max(sweep, t_op * (f + 2.0 * w) + top);
         }
         double t = sweep + (split ? 30.0 : 0.0);
         for (int l = 0; l < levels; ++l) {
@@ -1185,8 +1219,22 @@ void upload_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
     typedef std::vector<const SweepPart *> Parts;
     if (S.split) {
       list(S.fwd, [&](const BandPlan &P) { return each(P.fwd); });
-      list(S.top, [&](const BandPlan &P) { return Parts{&P.top}; });
-      list(S.top_bwd, [&](const BandPlan &P) { return Parts{&P.top_bwd}; });
+      // by depth where the plan has the parts, the others' top as their root
+      auto lv = [&](const BandPlan &P) { return b.by_level && P.root.nloc > 0; };
+      list(S.top, [&](const BandPlan &P) { return Parts{lv(P) ? &P.root : &P.top}; });
+      list(S.top_bwd, [&](const BandPlan &P) { return Parts{lv(P) ? &P.root_bwd : &P.top_bwd}; });
+      size_t deep = 0;
+      for (int c : cells)
+        if (lv(*plans[c])) deep = std::max(deep, plans[c]->sep_fwd.size());
+      for (size_t d = 1; d < deep; ++d) {
+        auto at_depth = [&](const BandPlan &P, const std::vector<std::vector<SweepPart>> &v) {
+          return lv(P) && d < v.size() ? each(v[d]) : Parts{};
+        };
+        S.sep_fwd.emplace_back();
+        S.sep_bwd.emplace_back();
+        list(S.sep_fwd.back(), [&](const BandPlan &P) { return at_depth(P, P.sep_fwd); });
+        list(S.sep_bwd.back(), [&](const BandPlan &P) { return at_depth(P, P.sep_bwd); });
+      }
     } else {
       list(S.whole, [&](const BandPlan &P) { return Parts{&P.whole}; });
     }
@@ -1216,6 +1264,28 @@ void upload_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
     for (int c : spread) one_wg(c);
   b.ntail = (int)rwg.size() - b.nrefine;
   b.rwg = dupload(rwg);
+  // separators by depth if that is the shorter: per cell the longest part of
+  // each depth instead of the sum of all, for two launches more per depth and
+  // refinement sweep and one in the first solve (one cell of 20000 elements,
+  // 16 leaves: 387 us for the separators of both solves by one workgroup)
+  double together = 0.0;
+  std::vector<double> depth_ops;
+  for (int c : spread) {
+    const BandPlan &P = *plans[c];
+    together = std::max(together, (double)P.top.nop + P.top_bwd.nop);
+    if (P.root.nloc == 0) continue;
+    depth_ops.resize(std::max(depth_ops.size(), P.sep_fwd.size()), 0.0);
+    depth_ops[0] = std::max(depth_ops[0], (double)P.root.nop + P.root_bwd.nop);
+    for (size_t d = 1; d < P.sep_fwd.size(); ++d) {
+      double f = 0.0, w = 0.0;
+      for (const SweepPart &q : P.sep_fwd[d]) f = std::max(f, (double)q.nop);
+      for (const SweepPart &q : P.sep_bwd[d]) w = std::max(w, (double)q.nop);
+      depth_ops[d] = std::max(depth_ops[d], f + 2.0 * w);
+    }
+  }
+  double apart = depth_ops.empty() ? 1e300 : 0.0;
+  for (double o : depth_ops) apart += o;
+  b.by_level = apart < 1e300 && sweep_op_us(elem_size) * (together - apart) > 5.0 * 3.0 * (depth_ops.size() - 1.0);
   b.sweeps = lists_of(spread);
   b.sweeps_cell.clear();
   if (!ctx->opt.batched)
@@ -1878,10 +1948,13 @@ void enqueue_sweeps(hipStream_t s, const Batch &b, const Batch::SweepLists &L, b
   };
   if (first) {
     go(L.top_bwd);
+    for (const auto &l : L.sep_bwd) go(l);
     go(L.bwd);
   } else if (L.split) {
     go(L.fwd);
+    for (size_t d = L.sep_fwd.size(); d-- > 0;) go(L.sep_fwd[d]);
     go(L.top);
+    for (const auto &l : L.sep_bwd) go(l);
     go(L.bwd);
   } else {
     go(L.whole);
