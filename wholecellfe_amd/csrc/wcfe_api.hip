@@ -856,6 +856,22 @@ int set_err(wcfe_ctx *ctx, int code, const std::string &m) {
   return code;
 }
 
+// Drops the captured step and frees the batch.  A captured step with concurrent
+// cell groups runs on streams of the runtime's own: unless the device is
+// synchronized before the graph goes and again after the memory is freed, that
+// memory is not given back and a second large context finds none (1,024
+// replicas: 167 GB).
+void release_batch(wcfe_ctx *ctx) {
+  (void)hipSetDevice(ctx->opt.device);
+  (void)hipDeviceSynchronize();
+  if (ctx->gexec) (void)hipGraphExecDestroy(ctx->gexec);
+  if (ctx->graph) (void)hipGraphDestroy(ctx->graph);
+  ctx->gexec = nullptr;
+  ctx->graph = nullptr;
+  ctx->b.release();
+  (void)hipDeviceSynchronize();
+}
+
 template <class F> int guarded(wcfe_ctx *ctx, F &&f) {
   try {
     f();
@@ -2431,10 +2447,7 @@ int wcfe_create(const wcfe_options *opt, wcfe_ctx **out) {
 
 int wcfe_destroy(wcfe_ctx *ctx) {
   if (!ctx) return WCFE_OK;
-  if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
-  if (ctx->gexec) (void)hipGraphExecDestroy(ctx->gexec);
-  if (ctx->graph) (void)hipGraphDestroy(ctx->graph);
-  ctx->b.release();
+  release_batch(ctx);
   ctx->arena.release();
   if (ctx->tab_px) (void)hipFree(ctx->tab_px);
   if (ctx->tab_py) (void)hipFree(ctx->tab_py);
@@ -2658,11 +2671,7 @@ void step_impl(wcfe_ctx *ctx) {
 // from the host copies of the cells (the state the cells were added with).
 void rebuild_batch(wcfe_ctx *ctx) {
   HIPCHECK(hipStreamSynchronize(ctx->stream));
-  if (ctx->gexec) (void)hipGraphExecDestroy(ctx->gexec);
-  if (ctx->graph) (void)hipGraphDestroy(ctx->graph);
-  ctx->gexec = nullptr;
-  ctx->graph = nullptr;
-  ctx->b.release();
+  release_batch(ctx);
   build_batch(ctx, ctx->b, ctx->cells, mixed(ctx) ? 4 : 8);
   ctx->stepped = false;
   ++ctx->layout;
@@ -2713,12 +2722,7 @@ int wcfe_autotune(wcfe_ctx *ctx, int32_t flags, int32_t steps, int32_t *chosen, 
         if (e.code != WCFE_ERR_OOM) throw;
         // this candidate does not fit (its batch or a workspace of its
         // first step): skip it
-        (void)hipStreamSynchronize(ctx->stream);
-        if (ctx->gexec) (void)hipGraphExecDestroy(ctx->gexec);
-        if (ctx->graph) (void)hipGraphDestroy(ctx->graph);
-        ctx->gexec = nullptr;
-        ctx->graph = nullptr;
-        ctx->b.release();
+        release_batch(ctx);
         (void)hipGetLastError();
         return 1e300;
       }
@@ -2826,7 +2830,7 @@ int wcfe_autotune(wcfe_ctx *ctx, int32_t flags, int32_t steps, int32_t *chosen, 
         break;
       } catch (const ApiError &e) {
         if (e.code != WCFE_ERR_OOM || q + 1 == tried.size()) throw;
-        ctx->b.release();
+        release_batch(ctx);
         (void)hipGetLastError();
       }
     }
