@@ -104,3 +104,17 @@ def test_separators_by_depth_equal_the_uncut_band(K, sym, prec):
             out.append(c.positions(0))
     # relative residual 1e-12 at a condition number below 1e6
     assert np.linalg.norm(out[0] - out[1]) <= 1e-6 * np.linalg.norm(out[1] - d["x"])
+
+
+# The first FP32 solve, whose forward substitution ran beside the
+# factorization: a sweep that reads the wrong vector leaves the residual at 1
+@pytest.mark.parametrize("sym", [1, 0])
+@pytest.mark.parametrize("K", [1, 4, 11, 17, 40])
+def test_first_solve_reduces_the_residual(K, sym):
+    print("case first solve", K, sym, flush=True)
+    d = cells.cst_cell(K=K, n_spr=10 * K, seed=K, time=1.0)
+    with W.Context(precision=W.PREC_MIXED, t0=1.0, symmetric=sym, max_refine=1, lin_rtol=0.1) as c:
+        cells.add_to_context(c, d)
+        c.finalize()
+        # FP32 roundoff 6e-8 times a condition number below 1e6
+        assert c.newton_step()["max_lin_relres"] <= 0.1
