@@ -1311,6 +1311,7 @@ void upload_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
 
 void build_batch(wcfe_ctx *ctx, Batch &b, const std::vector<HostCell> &hc, int elem_size) {
   b.ncell = (int)hc.size();
+  if (b.ncell >= (1 << 11)) fail(WCFE_ERR_ARG, "at most 2047 systems per batch");  // as checkpoints and the LU's work lists
   std::vector<std::vector<int>> colors(b.ncell);
   b.ncolors_cell.assign(b.ncell, 0);
   b.ncolor = 0;
