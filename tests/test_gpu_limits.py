@@ -1,4 +1,7 @@
-"""What a context refuses."""
+"""What a context refuses, and the device memory that its calls take."""
+import ctypes
+import threading
+
 import numpy as np
 import pytest
 
@@ -7,6 +10,13 @@ from wholecellfe_amd import mesh
 pytestmark = pytest.mark.gpu
 
 W = pytest.importorskip("wholecellfe_amd")
+
+
+def free_bytes():
+    """Free device memory, from the HIP runtime that the library is linked to."""
+    free, total = ctypes.c_size_t(0), ctypes.c_size_t(0)
+    assert W.lib().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
 
 
 # a checkpoint holds at most 2047 cells, and the LU's work lists 11 bits of them
@@ -23,3 +33,37 @@ def test_batches_above_2047_cells_are_refused():
             with pytest.raises(W.WcfeError) as e:
                 c.finalize()
             assert e.value.code == W.ERR_ARG
+
+
+def solve(c, n, seed):
+    rng = np.random.default_rng(seed)
+    A = rng.standard_normal((n, n)) / np.sqrt(n) + 3.0 * np.eye(n)
+    b = rng.standard_normal(n)
+    return A, b, c.dense_solve([A], [b])[0][0]
+
+
+# A (FP64), the factors (FP64) and 128 entries per row of diagonal inverses
+def test_large_dense_solve_takes_what_it_needs():
+    n = 6000
+    need = 8 * (n * n + 6016 * 6016 + 128 * 6016)
+    with W.Context(precision=W.PREC_FP64) as c:
+        solve(c, 200, 1)  # code and streams are loaded
+        before, least, stop = free_bytes(), [1 << 62], threading.Event()
+
+        def watch():
+            while not stop.is_set():
+                least[0] = min(least[0], free_bytes())
+
+        t = threading.Thread(target=watch)
+        t.start()
+        try:
+            A, b, x = solve(c, n, 2)
+        finally:
+            stop.set()
+            t.join()
+        after = free_bytes()
+    used = before - least[0]
+    print("needed %d, taken %d, kept %d" % (need, used, before - after), flush=True)
+    assert np.linalg.norm(A @ x - b) <= 1e-8 * np.linalg.norm(b)
+    assert 0.9 * need < used <= 1.1 * need  # vectors and 2 MiB granules beside the matrices
+    assert before - after <= 64 << 20

@@ -785,16 +785,23 @@ struct FrameSlot {
 };
 
 // One device allocation and one pinned host allocation for the stateless calls
-// (Scratch).
+// (Scratch), kept between calls up to ARENA_KEEP bytes together.
+constexpr size_t ARENA_KEEP = 64u << 20;
 struct Arena {
   unsigned char *dev = nullptr, *host = nullptr;
   size_t dev_cap = 0, host_cap = 0;
+  // a quarter more than asked for, so that a growing call seldom allocates
+  // again, but never above what is kept: a larger buffer goes back after its
+  // call, and a call may need most of the device's memory
+  static size_t capacity(size_t need) {
+    return std::max({need, std::min(need + need / 4, ARENA_KEEP), (size_t)1 << 20});
+  }
   void reserve(size_t d, size_t h) {
     if (d > dev_cap) {
       if (dev) (void)hipFree(dev);
       dev = nullptr;
       dev_cap = 0;
-      const size_t n = std::max<size_t>(d + d / 4, 1u << 20);
+      const size_t n = capacity(d);
       dev = dalloc<unsigned char>(n);
       dev_cap = n;
     }
@@ -802,7 +809,7 @@ struct Arena {
       if (host) (void)hipHostFree(host);
       host = nullptr;
       host_cap = 0;
-      const size_t n = std::max<size_t>(h + h / 4, 1u << 20);
+      const size_t n = capacity(h);
       void *p = nullptr;
       const hipError_t e = hipHostMalloc(&p, n, hipHostMallocDefault);
       if (e != hipSuccess) fail(WCFE_ERR_OOM, "hipHostMalloc of %zu bytes failed: %s", n, hipGetErrorString(e));
@@ -3354,7 +3361,6 @@ int wcfe_get_colors(wcfe_ctx *ctx, int32_t cell, int32_t *color) {
 
 namespace {
 
-// Device buffers owned for the duration of one stateless call.
 // Buffers of one stateless call.  They come out of the context's arena: one
 // device allocation and one pinned host allocation, kept between calls up to
 // ARENA_KEEP bytes and freed with the context, so a call makes no allocation,
@@ -3363,7 +3369,7 @@ namespace {
 // same context gets buffers of its own.  Declare every buffer (in, inout, out,
 // zeros, work), commit(), launch, fetch().  Arrays above ARENA_DIRECT bytes
 // are copied from and to the caller's memory without the pinned copy.
-constexpr size_t ARENA_KEEP = 64u << 20, ARENA_DIRECT = 1u << 20;
+constexpr size_t ARENA_DIRECT = 1u << 20;
 struct Scratch {
   explicit Scratch(wcfe_ctx *c) : ctx(c), lock(c->arena_mutex, std::try_to_lock), A(lock ? &c->arena : &own) {}
   Scratch(const Scratch &) = delete;
