@@ -1,10 +1,11 @@
-"""What a context refuses, and the device memory that its calls take."""
+"""What a context refuses, and the device memory that it takes and gives back."""
 import ctypes
 import threading
 
 import numpy as np
 import pytest
 
+import cells
 from wholecellfe_amd import mesh
 
 pytestmark = pytest.mark.gpu
@@ -67,3 +68,43 @@ def test_large_dense_solve_takes_what_it_needs():
     assert np.linalg.norm(A @ x - b) <= 1e-8 * np.linalg.norm(b)
     assert 0.9 * need < used <= 1.1 * need  # vectors and 2 MiB granules beside the matrices
     assert before - after <= 64 << 20
+
+
+# each thread's calls are its own, whichever holds the context's buffers
+def test_two_threads_in_one_context():
+    with W.Context(precision=W.PREC_FP64) as c:
+        bad = []
+
+        def work(seed):
+            for k in range(12):
+                A, b, x = solve(c, 40 + 90 * ((seed + k) % 4), 100 * seed + k)
+                if not np.linalg.norm(A @ x - b) <= 1e-8 * np.linalg.norm(b):
+                    bad.append((seed, k))
+
+        ts = [threading.Thread(target=work, args=(s,)) for s in range(3)]
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+    assert not bad
+
+
+# two concurrent cell groups: the captured step runs on streams of its own
+@pytest.mark.parametrize("groups", [0, 2])
+def test_closed_contexts_give_their_memory_back(groups):
+    ds = [cells.cst_cell(K=28, n_spr=100, seed=k, time=1.0) for k in range(4)]
+
+    def one():
+        with W.Context(t0=1.0, lu_groups=groups) as c:
+            for d in ds * 4:
+                cells.add_to_context(c, d)
+            c.finalize()
+            c.newton_step()
+            return free_bytes()
+
+    one()
+    before = free_bytes()
+    inside = [one() for _ in range(3)]
+    # 16 cells of 4704 elements: 16 x 4872^2 x 4 bytes of matrices
+    assert before - min(inside) > 1.4e9
+    assert before - free_bytes() <= 64 << 20
