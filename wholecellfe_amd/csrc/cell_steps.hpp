@@ -44,13 +44,13 @@ __device__ __forceinline__ void newton_finish(CellState &s, double rtol, double 
   if (!s.ir_done) s.lin_failed = 1;
 }
 
-// r = -G - K d of one node, from the stored FP64 element matrices over its
-// elements in element order, and the node terms (drag diagonal, the boundary
-// vertex's 2 x 6 block, the area term's rank-one part k g_i (sum_m g_m . d_m),
-// gd the sum).
-__device__ __forceinline__ double2 residual_node(int i, int c, const int *el_tri, const int *adj_start, const int *adj,
-                                                 const double *Ke64, const double *G, const double *delta,
-                                                 const CellParams &p, const BndView &bv, double gd) {
+// K d of one node, from the stored FP64 element matrices over its elements in
+// element order, and the node terms (drag diagonal, the boundary vertex's
+// 2 x 6 block, the area term's rank-one part k g_i (sum_m g_m . d_m), gd the
+// sum).
+__device__ __forceinline__ double2 product_node(int i, const int *el_tri, const int *adj_start, const int *adj,
+                                                const double *Ke64, const double *delta, const CellParams &p,
+                                                const BndView &bv, double gd) {
   const double2 *d2 = reinterpret_cast<const double2 *>(delta);
   double y0 = 0.0, y1 = 0.0;
   for (int k = adj_start[i]; k < adj_start[i + 1]; ++k) {
@@ -87,7 +87,14 @@ __device__ __forceinline__ double2 residual_node(int i, int c, const int *el_tri
       }
     }
   }
-  return make_double2(-G[2 * i] - y0, -G[2 * i + 1] - y1);
+  return make_double2(y0, y1);
+}
+// r = -G - K d of one node
+__device__ __forceinline__ double2 residual_node(int i, const int *el_tri, const int *adj_start, const int *adj,
+                                                 const double *Ke64, const double *G, const double *delta,
+                                                 const CellParams &p, const BndView &bv, double gd) {
+  const double2 y = product_node(i, el_tri, adj_start, adj, Ke64, delta, p, bv, gd);
+  return make_double2(-G[2 * i] - y.x, -G[2 * i + 1] - y.y);
 }
 
 // Sum over a workgroup of NT threads (a power of two), in every thread: a

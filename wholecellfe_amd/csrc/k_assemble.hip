@@ -478,7 +478,7 @@ __global__ __launch_bounds__(256) void k_matvec_ir(const int *el_tri, const int 
   if (i >= node_end) return;
   const int c = node_cell[i];
   if (cs[c].ir_done || cp[c].refine) return;
-  const double2 ri = residual_node(i, c, el_tri, adj_start, adj, Ke64, G, delta, cp[c], bv, bv.gd ? bv.gd[c] : 0.0);
+  const double2 ri = residual_node(i, el_tri, adj_start, adj, Ke64, G, delta, cp[c], bv, bv.gd ? bv.gd[c] : 0.0);
   r[2 * i] = ri.x;
   r[2 * i + 1] = ri.y;
 }

@@ -680,6 +680,22 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_band_sweep(const CellParams *
 // Morrison 1950), the dots in FP64; the residual is the full K's.  The full
 // matrix is dense (the boundary couples to itself): n^3 instead of n bw^2
 // (905 elements, load step of two to three Newton steps: 1600 -> 610 us).
+// z stays as the factors give it: refined against B it would no longer belong
+// to the matrix that was factored (B with rounding and replaced pivots).
+// B can be singular where K is not (the area off area_0 by a pressure that the
+// cell's stiffness balances); then y and z are large, almost cancel, and the
+// sweeps stall.  From the first sweep that leaves more than REFINE_POOR of the
+// residual, or if max_refine end above lin_rtol, the solve is mixed block
+// elimination (Govaerts and Pryce 1990; its solve with the transpose taken as
+// z / k, which the mostly symmetric B allows): a first guess of the rank one's
+// part leaves the right-hand side before B^-1 is applied.  The updates then are
+// search directions (generalized conjugate residuals, Eisenstat, Elman and
+// Schultz 1983): of all their combinations the one of least residual, so that
+// what is left wrong in a few directions costs a sweep each.  At most
+// REFINE_MORE sweeps above max_refine; with B singular to rounding and K of
+// condition 2e3 to 4e5 three to six in all to 1e-8, where sweeps by the rank
+// one formula alone stood at 0.03 to 0.8 of the residual after four.
+constexpr double REFINE_POOR = 1.0 / 16.0, REFINE_FLOOR = 1e-13;  // FLOOR: rounding of the FP64 residual
 template <class T>
 __global__ __launch_bounds__(SWEEP_THREADS) void k_band_refine(const CellParams *cp, CellState *cs,
                                                                const RefineWG *wgs, const SweepOp *ops,
@@ -706,74 +722,150 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_band_refine(const CellParams 
     }
     return block_sum<SWEEP_THREADS>(a, red);
   };
+  auto g_of = [&](int i) {
+    const int b = ra.bv.bidx[i];
+    return b >= 0 && ra.bv.frame[b].x >= 0 ? ra.bv.g[b] : make_double2(0.0, 0.0);
+  };
   double den = 1.0;
   if (p.smw) {
-    // z from the factors of B, and while k g.B^-1 g is large again from its
-    // FP64 residual k g - B z: an error e of z leaves K e (g.y) / (1 + g.z) in
-    // the residual, and the area term makes K e large
-    double gz = 0.0;
-    for (int t = 0; t < 3; ++t) {
-      for (int i = n0 + threadIdx.x; i < n1; i += SWEEP_THREADS) {
-        const int b = ra.bv.bidx[i];
-        const bool on = b >= 0 && ra.bv.frame[b].x >= 0;
-        const double2 g = on ? ra.bv.g[b] : make_double2(0.0, 0.0);
-        double2 q = make_double2(p.k_area * g.x, p.k_area * g.y);
-        if (t > 0) {
-          const double2 ri = residual_node(i, c, ra.el_tri, ra.adj_start, ra.adj, ra.Ke64, ra.G, ra.z, p, ra.bv, 0.0);
-          q.x += ri.x + ra.G[2 * i];
-          q.y += ri.y + ra.G[2 * i + 1];
-        }
-        ra.inc[2 * i] = q.x;
-        ra.inc[2 * i + 1] = q.y;
-      }
-      __syncthreads();
-      SweepVec<T> v = sv;
-      v.rhs = ra.inc;
-      v.delta = ra.z;
-      v.from_y = 0;
-      sweep_part<T>(p, wg.whole, ops, locs, accs, K, Dinv, kinv, v, t > 0, y, rowb);
-      __syncthreads();
-      gz = gdot(ra.z);
-      if (!(fabs(gz) > 16.0)) break;
+    for (int i = n0 + threadIdx.x; i < n1; i += SWEEP_THREADS) {
+      const double2 g = g_of(i);
+      ra.inc[2 * i] = p.k_area * g.x;
+      ra.inc[2 * i + 1] = p.k_area * g.y;
     }
-    den = 1.0 + gz;
+    __syncthreads();
+    SweepVec<T> v = sv;
+    v.rhs = ra.inc;
+    v.delta = ra.z;
+    v.from_y = 0;
+    sweep_part<T>(p, wg.whole, ops, locs, accs, K, Dinv, kinv, v, 0, y, rowb);
+    __syncthreads();
+    den = 1.0 + gdot(ra.z);
   }
+  bool rank1 = fabs(den) > 0.0 && fabs(den) < 1e300;
   if (ra.it0 == 0 && !ra.fwd_done) {
     for (int i = 2 * n0 + threadIdx.x; i < 2 * n1; i += SWEEP_THREADS) ra.r[i] = -ra.G[i];
     __syncthreads();
   }
-  for (int it = ra.it0; it < ra.max_refine; ++it) {
-    SweepVec<T> v = sv;
-    v.rhs = ra.r;
-    v.from_y = it == 0 && ra.fwd_done ? 1 : 0;
-    v.delta = p.smw ? ra.inc : ra.delta;
-    sweep_part<T>(p, v.from_y ? wg.bwd : wg.whole, ops, locs, accs, K, Dinv, kinv, v, p.smw ? 0 : it > 0, y, rowb);
-    __syncthreads();
-    if (p.smw) {
-      const double t = gdot(ra.inc) / den;
-      for (int i = 2 * n0 + threadIdx.x; i < 2 * n1; i += SWEEP_THREADS) {
-        const double d = ra.inc[i] - ra.z[i] * t;
-        ra.delta[i] = it > 0 ? ra.delta[i] + d : d;
-      }
-      __syncthreads();
-    }
+  auto residual = [&]() {  // r, and its squared norm
     const double gd = p.bterm & BT_AREA ? gdot(ra.delta) : 0.0;
     double rr = 0.0;
     for (int i = n0 + threadIdx.x; i < n1; i += SWEEP_THREADS) {
-      const double2 ri =
-          residual_node(i, c, ra.el_tri, ra.adj_start, ra.adj, ra.Ke64, ra.G, ra.delta, p, ra.bv, gd);
+      const double2 ri = residual_node(i, ra.el_tri, ra.adj_start, ra.adj, ra.Ke64, ra.G, ra.delta, p, ra.bv, gd);
       ra.r[2 * i] = ri.x;
       ra.r[2 * i + 1] = ri.y;
       rr += ri.x * ri.x + ri.y * ri.y;
     }
-    rr = block_sum<SWEEP_THREADS>(rr, red);
+    return block_sum<SWEEP_THREADS>(rr, red);
+  };
+  auto step = [&](int i, double t) { return t != 0.0 ? ra.inc[i] - ra.z[i] * t : ra.inc[i]; };
+  // cells with smw: the step as direction nd, orthogonal (its K times) to the
+  // ones before it, and delta along it to the least residual; false: no direction
+  int nd = -1;  // -1: plain refinement
+  auto direction = [&](double t) {
+    const int n2 = 2 * p.n_nodes;
+    double *P0 = ra.dirs + wg.dirs;
+    double *P = P0 + 2LL * nd * n2, *Q = P + n2;
+    for (int i = threadIdx.x; i < n2; i += SWEEP_THREADS) P[i] = step(2 * n0 + i, t);
+    __syncthreads();
+    const double gd = gdot(P - 2 * n0);
+    for (int i = threadIdx.x; i < p.n_nodes; i += SWEEP_THREADS) {
+      const double2 q =
+          product_node(n0 + i, ra.el_tri, ra.adj_start, ra.adj, ra.Ke64, P - 2 * n0, p, ra.bv, gd);
+      Q[2 * i] = q.x;
+      Q[2 * i + 1] = q.y;
+    }
+    __syncthreads();
+    auto dot = [&](const double *a, const double *b) {
+      double v = 0.0;
+      for (int i = threadIdx.x; i < n2; i += SWEEP_THREADS) v += a[i] * b[i];
+      return block_sum<SWEEP_THREADS>(v, red);
+    };
+#pragma unroll 1
+    for (int k = 0; k < 2 * nd; ++k) {  // twice: one pass leaves what cancellation made
+      const double *Pk = P0 + 2LL * (k % nd) * n2, *Qk = Pk + n2;
+      const double a = dot(Qk, Q);
+      for (int i = threadIdx.x; i < n2; i += SWEEP_THREADS) {
+        P[i] -= a * Pk[i];
+        Q[i] -= a * Qk[i];
+      }
+    }
+    const double qq = dot(Q, Q), s = 1.0 / sqrt(qq);
+    if (!(qq > 0.0 && s > 0.0)) return false;  // nothing new, or not finite
+    const double a = s * s * dot(Q, ra.r + 2 * n0);
+    for (int i = threadIdx.x; i < n2; i += SWEEP_THREADS) {
+      ra.delta[2 * n0 + i] += a * P[i];
+      P[i] *= s;
+      Q[i] *= s;
+    }
+    __syncthreads();
+    nd = nd + 1 < REFINE_DIRS ? nd + 1 : 0;
+    return true;
+  };
+  const double bnorm = cs[c].bnorm;
+  double last = bnorm, y1 = 0.0;  // y1: the first guess of g . d
+  int most = ra.max_refine;
+  for (int it = ra.it0; it < most; ++it) {
+    SweepVec<T> v = sv;
+    v.rhs = ra.r;
+    v.from_y = it == 0 && ra.fwd_done ? 1 : 0;
+    v.delta = p.smw ? ra.inc : ra.delta;
+    if (nd >= 0) {
+      double s = 0.0;
+      for (int i = 2 * n0 + threadIdx.x; i < 2 * n1; i += SWEEP_THREADS) s += ra.z[i] * ra.r[i];
+      s = rank1 ? block_sum<SWEEP_THREADS>(s, red) / den : 0.0;
+      y1 = s / p.k_area;
+      for (int i = n0 + threadIdx.x; i < n1; i += SWEEP_THREADS) {
+        const double2 g = g_of(i);
+        ra.inc[2 * i] = ra.r[2 * i] - g.x * s;
+        ra.inc[2 * i + 1] = ra.r[2 * i + 1] - g.y * s;
+      }
+      __syncthreads();
+      v.rhs = ra.inc;
+    }
+    sweep_part<T>(p, v.from_y ? wg.bwd : wg.whole, ops, locs, accs, K, Dinv, kinv, v, p.smw ? 0 : it > 0, y, rowb);
+    __syncthreads();
+    const double t = p.smw && rank1 ? (gdot(ra.inc) - y1) / den : 0.0;
+    bool stop = false;
+    double rr;
+    if (nd < 0) {
+      if (p.smw) {
+        for (int i = 2 * n0 + threadIdx.x; i < 2 * n1; i += SWEEP_THREADS) {
+          const double d = step(i, t);
+          ra.delta[i] = it > 0 ? ra.delta[i] + d : d;
+        }
+        __syncthreads();
+      }
+      rr = residual();
+      const double nrm = sqrt(rr);
+      if (p.smw && !(nrm <= ra.lin_rtol * bnorm) && !(nrm <= REFINE_FLOOR * bnorm) &&
+          (!(nrm <= REFINE_POOR * last) || it + 1 == ra.max_refine)) {
+        if (!(nrm <= last)) {  // worse than before the sweep: without it
+          for (int i = 2 * n0 + threadIdx.x; i < 2 * n1; i += SWEEP_THREADS) {
+            const double b = it > 0 ? ra.delta[i] - step(i, t) : 0.0;
+            ra.delta[i] = fabs(b) < 1e300 ? b : 0.0;
+          }
+          __syncthreads();
+          rr = residual();
+        }
+        nd = 0;
+        most = ra.max_refine + REFINE_MORE;
+      }
+      last = nrm;
+    } else {
+      stop = !direction(t);
+      if (stop && rank1) {  // without the rank one: B alone, one direction more
+        rank1 = stop = false;
+      }
+      rr = residual();
+    }
     if (threadIdx.x == 0) {
       CellState &s = cs[c];
       norm_finish(s, 1, sqrt(rr), ra.lin_rtol);
       done = s.ir_done;
     }
     __syncthreads();
-    if (done) return;
+    if (done || stop) return;
   }
 }
 size_t refine_max_dynamic(size_t max_lds) { return max_lds > 8192 ? max_lds - 8192 : 0; }

@@ -716,6 +716,7 @@ struct Batch {
   // cells whose refinement one workgroup runs: whole (CellParams::refine), then
   // (tail) those of which it runs the sweeps after the second, which few need
   RefineWG *rwg = nullptr;
+  double *dirs = nullptr;
   int nrefine = 0, ntail = 0, refine_loc = 0;
   std::vector<int> refine_at;  // per cell: its place in rwg, or -1
   bool tail = false;
@@ -738,7 +739,7 @@ struct Batch {
 
   void release() {
     void *ptrs[] = {X, x, fau, ea, cC, el_tri, el_cell, el_spr, sp_bary, sp_anchor, sp_state, sp_cell, sp_elem,
-                    sp_local, cp, cs, node_cell, adj_start, adj, Ge, g_start, g_col, g_bpos, g_cstart, g_ke, g_node, Ke64, G, r, delta, Rea, MM, K, Dinv, ysol, sync, ipiv, cells, celem, rwg,
+                    sp_local, cp, cs, node_cell, adj_start, adj, Ge, g_start, g_col, g_bpos, g_cstart, g_ke, g_node, Ke64, G, r, delta, Rea, MM, K, Dinv, ysol, sync, ipiv, cells, celem, rwg, dirs,
                     replica, transitions, plan.d_prefix, row_ptr, bcol, diag_pos, el_bpos, csr_cells, chunks, Kb,
                     cgvec, cg, partials, norm_part, norm_cnt, kpos, kinv, yfwd, ysw, slots, rank, refs, fops, sops, slocs, saccs, swg, plan.d_items, plan.d_ranges, plan.d_solve, rp, dp, bt_bidx, bt_node, bt_cst, crange, bt_cand, bt_frame, bt_g, bt_J, bt_area,
                     bt_gd, bt_fext};
@@ -1269,6 +1270,7 @@ void upload_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
   for (int c = 0; c < b.ncell; ++c) order[c] = c;
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return b.cp_h[x].nblk > b.cp_h[y].nblk; });
   std::vector<RefineWG> rwg;
+  long long dirs = 0;
   b.refine_at.assign(b.ncell, -1);
   for (int c : order) {
     if (!b.cp_h[c].csr && !b.cp_h[c].refine) spread.push_back(c);
@@ -1277,7 +1279,8 @@ void upload_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
     const At &o = at[plans[c]];
     auto put = [&](const SweepPart &q) { return SweepPart{q.op0 + o.op, q.nop, q.loc0 + o.loc, q.nloc}; };
     b.refine_at[c] = (int)rwg.size();
-    rwg.push_back(RefineWG{c, put(plans[c]->whole), put(plans[c]->whole_bwd)});
+    rwg.push_back(RefineWG{c, put(plans[c]->whole), put(plans[c]->whole_bwd), dirs});
+    if (b.cp_h[c].smw) dirs += 4LL * REFINE_DIRS * b.cp_h[c].n_nodes;
     b.refine_loc = std::max(b.refine_loc, plans[c]->whole.nloc);
   };
   for (int c : order)
@@ -1287,6 +1290,7 @@ void upload_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
     for (int c : spread) one_wg(c);
   b.ntail = (int)rwg.size() - b.nrefine;
   b.rwg = dupload(rwg);
+  if (dirs > 0) b.dirs = dalloc<double>(dirs);
   // separators by depth if that is the shorter: per cell the longest part of
   // each depth instead of the sum of all, for two launches more per depth and
   // refinement sweep and one in the first solve (one cell of 20000 elements,
@@ -2170,7 +2174,7 @@ template <class T> void enqueue_solve_refine(wcfe_ctx *ctx, Batch &b, const Scop
     PhaseScope ph(ctx, WCFE_PH_SOLVE);
     launch_band_refine<T>(s, b.cp, b.cs, b.rwg + first, n, b.refine_loc, b.sops, b.slocs, b.saccs, K,
                           static_cast<const T *>(b.Dinv), b.kinv, sweep_vec<T>(b, b.plan.fused),
-                          RefineArgs{b.el_tri, b.adj_start, b.adj, b.Ke64, b.G, b.r, b.delta, b.rp, b.dp,
+                          RefineArgs{b.el_tri, b.adj_start, b.adj, b.Ke64, b.G, b.r, b.delta, b.rp, b.dp, b.dirs,
                                      bnd_view(ctx, b), ctx->opt.lin_rtol, it0, max_refine, b.plan.fused ? 1 : 0});
   };
   refine(w0, nref, 0);

@@ -212,15 +212,18 @@ void launch_band_sweep(hipStream_t s, const CellParams *cp, const CellState *cs,
 // refinement sweeps it0 .. max_refine - 1 of a cell by one workgroup (solve,
 // FP64 residual, norm and control); parts: the cell's whole sweep and its
 // backward half (the first solve after the fused block steps); z, inc: batch
-// vectors for cells with smw
+// vectors for cells with smw; dirs: theirs too, 2 REFINE_DIRS vectors of a cell
+// from its dirs on
+constexpr int REFINE_DIRS = 12, REFINE_MORE = 8;
 struct RefineWG {
   int cell;
   SweepPart whole, bwd;
+  long long dirs;
 };
 struct RefineArgs {
   const int *el_tri, *adj_start, *adj;
   const double *Ke64, *G;
-  double *r, *delta, *z, *inc;
+  double *r, *delta, *z, *inc, *dirs;
   BndView bv;
   double lin_rtol;
   int it0, max_refine, fwd_done;
