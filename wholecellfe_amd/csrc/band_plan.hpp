@@ -72,9 +72,21 @@ struct BandPlan {
   struct Group {  // blocks and forward operations of one node in one level
     int ref0, nref, fop0, nfop;
   };
+  struct Count {  // pivots, or groups, with nref blocks (groups: with or without forward operations)
+    int nref, fwd, n;
+  };
+  static void count(std::vector<Count> &c, int nref, int fwd, int n) {
+    for (Count &q : c)
+      if (q.nref == nref && q.fwd == fwd) {
+        q.n += n;
+        return;
+      }
+    c.push_back(Count{nref, fwd, n});
+  }
   struct Level {
     std::vector<Pivot> piv;
     std::vector<Group> grp;
+    std::vector<Count> pivs, grps;  // the same, counted
     long long products = 0;
   };
   int n = 0, bw = 0, leaves = 1, nslot = 0;
@@ -135,10 +147,15 @@ inline int cut(std::vector<Node> &nodes, int lo, int hi, int depth, int bw, bool
 }
 }  // namespace band_detail
 
-// block steps (launches) of n blocks cut `depth` times
-inline int band_steps(int n, int bw, int depth) {
-  std::map<std::pair<int, int>, std::pair<int, int>> memo;
+// block steps (launches) of n blocks cut `depth` times; memo: of earlier calls
+// with the same bandwidth
+typedef std::map<std::pair<int, int>, std::pair<int, int>> StepMemo;
+inline int band_steps(int n, int bw, int depth, StepMemo &memo) {
   return n <= 0 ? 0 : band_detail::last_level(n, bw > 0 ? depth : 0, bw, memo) + 1;
+}
+inline int band_steps(int n, int bw, int depth) {
+  StepMemo memo;
+  return band_steps(n, bw, depth, memo);
 }
 
 inline BandPlan make_band_plan(int n, int bw, bool sym, int depth) {
@@ -179,27 +196,37 @@ inline BandPlan make_band_plan(int n, int bw, bool sym, int depth) {
   std::vector<int> slot((size_t)nn * n, -1);
   std::vector<char> written((size_t)nn * n, 0);
   auto slot_of = [&](int v, int i) -> int & { return slot[(size_t)v * n + i]; };
+  // the blocks that the pivots of the level before update, and where a block's
+  // target is (a table: a map of them took most of a plan's time)
+  struct Target {
+    int i, j, p0, p1, first;
+  };
+  std::vector<Target> tg;
+  std::vector<int> where((size_t)n * n, -1);
+  std::vector<std::vector<int>> by_node(nn);  // a level's other targets by the node of p0
+  std::vector<int> active;                    // nodes of the level, ascending
   P.lev.resize(nlev);
   for (int l = 0; l < nlev; ++l) {
     BandPlan::Level &L = P.lev[l];
     static const std::vector<int> none;
     const std::vector<int> &pend = l > 0 ? at[l - 1] : none;
-    // the blocks that the pivots of the level before update
-    struct Target {
-      int p0, p1, first;
-    };
-    std::map<std::pair<int, int>, Target> tg;  // by (row, column) block
+    tg.clear();
     for (int p : pend)
       for (int i : st[p])
         for (int j : st[p]) {
           if (sym && rank[i] < rank[j]) continue;
-          auto it = tg.find({i, j});
-          if (it == tg.end()) tg[{i, j}] = Target{p, -1, init[(size_t)i * n + j] ? 0 : 1};
-          else if (it->second.p1 < 0) it->second.p1 = p;
-          else throw std::logic_error("band plan: three updates of one block in one launch");
+          int &w = where[(size_t)i * n + j];
+          if (w < 0) {
+            w = (int)tg.size();
+            tg.push_back(Target{i, j, p, -1, init[(size_t)i * n + j] ? 0 : 1});
+          } else if (tg[w].p1 < 0) {
+            tg[w].p1 = p;
+          } else {
+            throw std::logic_error("band plan: three updates of one block in one launch");
+          }
           ++L.products;
         }
-    for (auto &t : tg) init[(size_t)t.first.first * n + t.first.second] = 1;
+    for (const Target &t : tg) init[(size_t)t.i * n + t.j] = 1;
     for (int s : at[l]) {
       for (int q = rank[s] + 1; q < n; ++q)
         if (nz[(size_t)s * n + order[q]]) st[s].push_back(order[q]);
@@ -208,20 +235,20 @@ inline BandPlan make_band_plan(int n, int bw, bool sym, int depth) {
         for (int j : st[s]) nz[(size_t)i * n + j] = 1;
       }
       BandPlan::Pivot pv{s, -1, (int)P.refs.size(), (int)st[s].size(), node_of[s]};
-      auto d = tg.find({s, s});
-      if (d != tg.end()) {
-        if (d->second.p1 >= 0) throw std::logic_error("band plan: two updates pending on a pivot");
-        pv.p = d->second.p0;
-        tg.erase(d);
+      const int d = where[(size_t)s * n + s];
+      if (d >= 0) {
+        if (tg[d].p1 >= 0) throw std::logic_error("band plan: two updates pending on a pivot");
+        pv.p = tg[d].p0;
+        tg[d].p0 = -1;  // taken
       }
       for (int i : st[s]) {
         BlockRef r{(int16_t)i, (int16_t)s, -1, -1, init[(size_t)i * n + s] ? 0 : 1, 0};
-        auto e = tg.find({i, s});
-        if (e != tg.end()) {
-          if (e->second.p1 >= 0 || e->second.p0 != pv.p) throw std::logic_error("band plan: column updates differ");
-          r.p0 = (int16_t)e->second.p0;
-          r.first = e->second.first;
-          tg.erase(e);
+        const int e = where[(size_t)i * n + s];
+        if (e >= 0) {
+          if (tg[e].p1 >= 0 || tg[e].p0 != pv.p) throw std::logic_error("band plan: column updates differ");
+          r.p0 = (int16_t)tg[e].p0;
+          r.first = tg[e].first;
+          tg[e].p0 = -1;
         }
         init[(size_t)i * n + s] = 1;
         if (!sym) init[(size_t)s * n + i] = 1;
@@ -233,16 +260,25 @@ inline BandPlan make_band_plan(int n, int bw, bool sym, int depth) {
     std::vector<size_t> done;  // slots that this level writes: readable from the next one on
     // the other updated blocks, by the node whose pivot updates them first,
     // and the forward substitution of the nodes that are active
-    std::map<int, std::vector<std::pair<std::pair<int, int>, Target>>> by_node;
-    for (const auto &t : tg) by_node[node_of[t.second.p0]].push_back(t);
-    for (int s : at[l]) by_node[node_of[s]];
-    for (int p : pend) by_node[node_of[p]];
-    for (const auto &nd : by_node) {
-      const int v = nd.first;
+    active.clear();
+    for (int s : at[l]) active.push_back(node_of[s]);
+    for (int p : pend) active.push_back(node_of[p]);
+    std::sort(active.begin(), active.end());
+    active.erase(std::unique(active.begin(), active.end()), active.end());
+    for (int v : active) by_node[v].clear();
+    for (size_t k = 0; k < tg.size(); ++k) {
+      where[(size_t)tg[k].i * n + tg[k].j] = -1;
+      if (tg[k].p0 >= 0) by_node[node_of[tg[k].p0]].push_back((int)k);
+    }
+    for (int v : active) {
       BandPlan::Group g{(int)P.refs.size(), 0, (int)P.fops.size(), 0};
-      for (const auto &t : nd.second)
-        P.refs.push_back(BlockRef{(int16_t)t.first.first, (int16_t)t.first.second, (int16_t)t.second.p0,
-                                  (int16_t)t.second.p1, t.second.first, 0});
+      std::sort(by_node[v].begin(), by_node[v].end(), [&](int a, int b) {
+        return tg[a].i != tg[b].i ? tg[a].i < tg[b].i : tg[a].j < tg[b].j;
+      });
+      for (int k : by_node[v]) {
+        const Target &t = tg[k];
+        P.refs.push_back(BlockRef{(int16_t)t.i, (int16_t)t.j, (int16_t)t.p0, (int16_t)t.p1, t.first, 0});
+      }
       auto op = [&](int kind, int i, int p, int sl) {
         P.fops.push_back(FwdOp{(int16_t)kind, (int16_t)i, (int16_t)p, 0, sl, 0});
       };
@@ -271,6 +307,8 @@ inline BandPlan make_band_plan(int n, int bw, bool sym, int depth) {
       if (g.nref || g.nfop) L.grp.push_back(g);
     }
     for (size_t q : done) written[q] = 1;
+    for (const BandPlan::Pivot &v : L.piv) BandPlan::count(L.pivs, v.nref, 0, 1);
+    for (const BandPlan::Group &g : L.grp) BandPlan::count(L.grps, g.nref, g.nfop > 0, 1);
   }
   // ---- sweeps ----
   auto part = [&](SweepPart &S, int ops0, int loc0) {

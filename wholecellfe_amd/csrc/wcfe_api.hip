@@ -398,15 +398,32 @@ struct LuPlan {
   struct Load {
     double total = 0.0, longest = 0.0;
     void add(double n, double t) {
+      if (n <= 0.0) return;
       total += n * t;
       longest = std::max(longest, t);
     }
   };
   static double inv_time(int cols, int f64) { return (cols ? 12.0 + 3.5 * (cols - 1) : 10.5) * (f64 ? 2.0 : 1.0); }
   static double tile_time(int tiles, int f64) { return (2.5 + 2.5 * tiles) * (f64 ? 2.0 : 1.0); }
-  static void level_load(const BandPlan::Level &L, const Deal &d, int f64, double n, Load &w) {
-    deal_level(L, d, [&](const BandPlan::Pivot &, int, int c, bool) { w.add(n, inv_time(c, f64)); },
-               [&](int, int t, int, int) { w.add(n, tile_time(t, f64)); });
+  // the items of deal_level, by the level's counts (times are halves of a
+  // microsecond, so the sums are exact in any order)
+  typedef std::vector<BandPlan::Count> Counts;
+  static Load level_load(const Counts &pivs, const Counts &grps, const Deal &d, int f64) {
+    Load w;
+    for (const BandPlan::Count &c : pivs) {
+      if (d.apart || c.nref == 0) w.add(c.n, inv_time(0, f64));
+      w.add((double)c.n * (c.nref / d.cols), inv_time(d.cols, f64));
+      if (c.nref % d.cols) w.add(c.n, inv_time(c.nref % d.cols, f64));
+    }
+    for (const BandPlan::Count &c : grps) {
+      const int k = d.apart ? ceil_div(c.nref, d.tiles) : std::max(1, ceil_div(c.nref, d.tiles));
+      if (k > 0) {
+        w.add((double)c.n * (c.nref % k), tile_time(c.nref / k + 1, f64));
+        w.add((double)c.n * (k - c.nref % k), tile_time(c.nref / k, f64));
+      }
+      if (d.apart && c.fwd) w.add(c.n, tile_time(0, f64));
+    }
+    return w;
   }
   static double load_time(const Load &w, double slots) { return 1.5 + std::max(w.longest, w.total / slots); }
   // fuse (the fused_step option): 1 the fastest by the estimate; 2 an item
@@ -421,14 +438,22 @@ struct LuPlan {
       for (int t : {1, 2, 4, 8}) d.push_back(Deal{c, t, 0});
     return d;
   }
-  static Deal choose_deal(const std::vector<std::pair<const BandPlan::Level *, double>> &levels, int fuse, int f64,
+  // levels: one level of several plans, and how many cells have it
+  static Deal choose_deal(const std::vector<std::pair<const BandPlan::Level *, int>> &levels, int fuse, int f64,
                           double slots, double *time = nullptr) {
+    Counts pivs, grps;
+    auto sum = [](Counts &to, const Counts &c, int n) {
+      for (const BandPlan::Count &q : c) BandPlan::count(to, q.nref, q.fwd, n * q.n);
+    };
+    for (const auto &l : levels) {
+      sum(pivs, l.first->pivs, l.second);
+      sum(grps, l.first->grps, l.second);
+    }
     Deal best{1, 1, 1};
     double bt = 1e300;
-    for (const Deal &d : deals(fuse)) {
-      Load w;
-      for (const auto &l : levels) level_load(*l.first, d, f64, l.second, w);
-      const double t = load_time(w, slots);
+    static const std::vector<Deal> by_time = deals(1);
+    for (const Deal &d : fuse == 1 ? by_time : deals(fuse)) {
+      const double t = load_time(level_load(pivs, grps, d, f64), slots);
       if (t < bt) {
         bt = t;
         best = d;
@@ -445,10 +470,10 @@ struct LuPlan {
                           const std::vector<const BandPlan *> &plans, const std::vector<int2> &base, int level,
                           int fuse, int f64, double slots) {
     Stage g{ST_STEP, level, 1, (int)buf.size(), 0, 0};
-    std::map<const BandPlan::Level *, double> count;
+    std::map<const BandPlan::Level *, int> count;
     for (int c : cells) {
       if (level >= (int)plans[c]->lev.size()) continue;
-      count[&plans[c]->lev[level]] += 1.0;
+      ++count[&plans[c]->lev[level]];
       g.work += plans[c]->lev[level].products;
     }
     const Deal d = choose_deal({count.begin(), count.end()}, fuse, f64, slots);
@@ -1004,12 +1029,12 @@ void plan_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
     return q;
   };
   std::vector<int> depth(b.ncell, 0);
-  auto cuts_for = [&](const CellParams &p, int levels, int most) {  // fewest cuts reaching `levels`, else the shortest
-    int best = 0, len = band_steps(p.nblk, p.bw, 0);
-    for (int d = 0; d <= most; ++d) {
-      const int e = band_steps(p.nblk, p.bw, d);
-      if (e < len) { len = e; best = d; }
-      if (e <= levels) return d;
+  // fewest cuts reaching `levels` steps, else the shortest; st: the steps by cuts
+  auto cuts_for = [](const std::array<int, MAX_CUTS + 1> &st, int levels) {
+    int best = 0;
+    for (int d = 0; d <= MAX_CUTS; ++d) {
+      if (st[d] < st[best]) best = d;
+      if (st[d] <= levels) return d;
     }
     return best;
   };
@@ -1038,48 +1063,62 @@ void plan_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
       for (const CellParams &p : b.cp_h)
         if (!p.csr && p.nblk > 0) ++shapes[{p.nblk, p.bw, p.sym}];
       std::vector<int> cand;
-      for (auto &sh : shapes)
-        for (int d = 0; d <= MAX_CUTS; ++d) cand.push_back(band_steps(sh.first[0], sh.first[1], d));
+      std::map<std::array<int, 2>, std::array<int, MAX_CUTS + 1>> steps;  // by blocks and bandwidth
+      std::map<int, StepMemo> memo;  // by bandwidth
+      for (auto &sh : shapes) {
+        auto &st = steps[{sh.first[0], sh.first[1]}];
+        for (int d = 0; d <= MAX_CUTS; ++d)
+          cand.push_back(st[d] = band_steps(sh.first[0], sh.first[1], d, memo[sh.first[1]]));
+      }
       std::sort(cand.begin(), cand.end());
       cand.erase(std::unique(cand.begin(), cand.end()), cand.end());
-      {  // the plans the candidates ask for, on the host's threads
-        std::set<std::array<int, 4>> need;
-        for (int C : cand)
-          for (auto &sh : shapes) {
-            CellParams p{};
-            p.nblk = sh.first[0];
-            p.bw = sh.first[1];
-            p.sym = sh.first[2];
-            need.insert({p.nblk, p.bw, p.sym, cuts_for(p, C, MAX_CUTS)});
-          }
+      // the plans that a candidate asks for and the ones before it did not
+      auto make_plans = [&](int C) {
         std::vector<std::pair<std::array<int, 4>, std::shared_ptr<BandPlan>>> todo;
-        for (auto it = need.rbegin(); it != need.rend(); ++it) todo.push_back({*it, nullptr});  // largest first
-        parallel_cells((int)todo.size(), [&](int i) {
+        double work = 0.0;  // about 75 ns each
+        for (auto it = shapes.rbegin(); it != shapes.rend(); ++it) {  // largest first
+          const std::array<int, 3> &k = it->first;
+          const std::array<int, 4> key{k[0], k[1], k[2], cuts_for(steps[{k[0], k[1]}], C)};
+          if (made.count(key)) continue;
+          todo.push_back({key, nullptr});
+          work += (double)k[0] * (k[1] + 1) * (k[1] + 1);
+        }
+        auto make = [&](int i) {
           const std::array<int, 4> &k = todo[i].first;
           try {
             todo[i].second = std::make_shared<BandPlan>(make_band_plan(k[0], k[1], k[2] != 0, k[3]));
           } catch (...) {  // made again below, where the caller can see the exception
           }
-        });
+        };
+        if (work > 16384.0) parallel_cells((int)todo.size(), make);
+        else for (int i = 0; i < (int)todo.size(); ++i) make(i);  // starting threads takes longer
         for (auto &t : todo)
           if (t.second) made[t.first] = t.second;
-      }
+      };
       double best = 1e300;
       int best_c = INT_MAX;
       for (int C : cand) {
         int levels = 0;
+        for (auto &sh : shapes) {
+          const auto &st = steps[{sh.first[0], sh.first[1]}];
+          levels = std::max(levels, st[cuts_for(st, C)]);
+        }
+        // every level holds a pivot: a candidate whose launches alone take longer needs no plans
+        if (levels * (1.5 + LuPlan::inv_time(0, f64)) >= best) continue;
+        make_plans(C);
+        levels = 0;
         double sweep = 0.0;
         bool split = false;
-        std::vector<std::vector<std::pair<const BandPlan::Level *, double>>> by_level;
+        std::vector<std::vector<std::pair<const BandPlan::Level *, int>>> by_level;
         for (auto &sh : shapes) {
           CellParams p{};
           p.nblk = sh.first[0];
           p.bw = sh.first[1];
           p.sym = sh.first[2];
-          const std::shared_ptr<BandPlan> P = plan_of(p, cuts_for(p, C, MAX_CUTS));
+          const std::shared_ptr<BandPlan> P = plan_of(p, cuts_for(steps[{p.nblk, p.bw}], C));
           levels = std::max(levels, (int)P->lev.size());
           by_level.resize(levels);
-          for (size_t l = 0; l < P->lev.size(); ++l) by_level[l].push_back({&P->lev[l], (double)sh.second});
+          for (size_t l = 0; l < P->lev.size(); ++l) by_level[l].push_back({&P->lev[l], sh.second});
           int f = 0, w = 0;
           for (size_t q = 0; q < P->fwd.size(); ++q) {
             f = std::max(f, P->fwd[q].nop);
@@ -1093,7 +1132,7 @@ void plan_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
           sweep = std::max(sweep, t_op * (f + 2.0 * w) + top);
         }
         double t = sweep + (split ? 30.0 : 0.0);
-        for (int l = 0; l < levels; ++l) {
+        for (int l = 0; l < levels && t < best; ++l) {
           double tl = 0.0;
           LuPlan::choose_deal(by_level[l], 1, f64, slots, &tl);  // the cuts do not depend on fused_step
           t += tl;
@@ -1104,7 +1143,8 @@ void plan_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
         }
       }
       for (int c = 0; c < b.ncell; ++c)
-        if (!b.cp_h[c].csr) depth[c] = cuts_for(b.cp_h[c], best_c, MAX_CUTS);
+        if (!b.cp_h[c].csr && b.cp_h[c].nblk > 0)
+          depth[c] = cuts_for(steps[{b.cp_h[c].nblk, b.cp_h[c].bw}], best_c);
     }
   }
   for (int c = 0; c < b.ncell; ++c) {
