@@ -670,6 +670,7 @@ struct Batch {
   std::vector<int> g_start_h;  // host copy of g_start
   double *Ke64 = nullptr, *G = nullptr, *r = nullptr, *delta = nullptr, *Rea = nullptr, *MM = nullptr;
   void *K = nullptr;
+  size_t K_bytes = 0;
   void *Dinv = nullptr;
   void *ysol = nullptr;  // triangular-solve intermediate, one per system row
   int *sync = nullptr;   // triangular-solve tickets and per-cell counters
@@ -877,6 +878,11 @@ struct wcfe_ctx {
   // frame output: two slots in flight, copied on their own stream
   FrameSlot frames[2];
   int next_frame = 0;
+  // the matrices of the batch that rebuild_batch replaces: the new ones take
+  // their memory if they need as much (freeing and taking tens of GB again
+  // stalled a replaced cell of 192 replicas for 0.1 to 3.6 s now and then)
+  void *old_K = nullptr;
+  size_t old_K_bytes = 0;
   int layout = 0;  // bumped whenever the batch is laid out (finalize, rebuild)
   hipStream_t copy_stream = nullptr;
   hipEvent_t frame_ready = nullptr;
@@ -903,6 +909,12 @@ void release_batch(wcfe_ctx *ctx) {
   ctx->graph = nullptr;
   ctx->b.release();
   (void)hipDeviceSynchronize();
+}
+
+void free_old_K(wcfe_ctx *ctx) {
+  if (ctx->old_K) (void)hipFree(ctx->old_K);
+  ctx->old_K = nullptr;
+  ctx->old_K_bytes = 0;
 }
 
 template <class F> int guarded(wcfe_ctx *ctx, F &&f) {
@@ -1436,6 +1448,8 @@ void build_batch(wcfe_ctx *ctx, Batch &b, const std::vector<HostCell> &hc, int e
   b.N = N;
   b.S = S;
   b.kpool = kp;
+  const size_t K_bytes = (size_t)kp * elem_size;
+  if (K_bytes > ctx->old_K_bytes || ctx->old_K_bytes - K_bytes > K_bytes / 16) free_old_K(ctx);
   // dense cells under static pivoting: a band-reducing node numbering (RCM
   // when it narrows the band) and the LU restricted to the band; partial
   // pivoting (row swaps widen the band) and ctx->opt.band == 0 keep the natural
@@ -1710,7 +1724,15 @@ void build_batch(wcfe_ctx *ctx, Batch &b, const std::vector<HostCell> &hc, int e
   b.MM = dalloc<double>(N);
   b.ipiv = dalloc<int>(std::max(sys, 1));
   HIPCHECK(hipMemset(b.ipiv, 0, sizeof(int) * std::max(sys, 1)));
-  b.K = (void *)dalloc<unsigned char>((size_t)kp * elem_size);
+  if (ctx->old_K) {
+    b.K = ctx->old_K;
+    b.K_bytes = ctx->old_K_bytes;
+    ctx->old_K = nullptr;
+    ctx->old_K_bytes = 0;
+  } else {
+    b.K = (void *)dalloc<unsigned char>(K_bytes);
+    b.K_bytes = K_bytes;
+  }
   b.Dinv = (void *)dalloc<unsigned char>((size_t)std::max(sys, 1) * 128 * elem_size);
   {
     std::vector<int> kinv(std::max(sys, 1), -1);
@@ -2723,8 +2745,16 @@ void step_impl(wcfe_ctx *ctx) {
 // from the host copies of the cells (the state the cells were added with).
 void rebuild_batch(wcfe_ctx *ctx) {
   HIPCHECK(hipStreamSynchronize(ctx->stream));
+  ctx->old_K = ctx->b.K;
+  ctx->old_K_bytes = ctx->b.K_bytes;
+  ctx->b.K = nullptr;
   release_batch(ctx);
-  build_batch(ctx, ctx->b, ctx->cells, mixed(ctx) ? 4 : 8);
+  try {
+    build_batch(ctx, ctx->b, ctx->cells, mixed(ctx) ? 4 : 8);
+  } catch (...) {
+    free_old_K(ctx);
+    throw;
+  }
   ctx->stepped = false;
   ++ctx->layout;
 }
