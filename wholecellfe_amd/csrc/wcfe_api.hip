@@ -1084,16 +1084,20 @@ void plan_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
       }
       std::sort(cand.begin(), cand.end());
       cand.erase(std::unique(cand.begin(), cand.end()), cand.end());
-      // the plans that a candidate asks for and the ones before it did not
-      auto make_plans = [&](int C) {
+      // the plans that some candidates ask for; threads where they save more than they take to start
+      auto key_of = [&](const std::array<int, 3> &k, int C) {
+        return std::array<int, 4>{k[0], k[1], k[2], cuts_for(steps.at({k[0], k[1]}), C)};
+      };
+      auto make_plans = [&](const std::vector<int> &cs) {
+        std::set<std::array<int, 4>> need;
+        for (int C : cs)
+          for (auto &sh : shapes) need.insert(key_of(sh.first, C));
         std::vector<std::pair<std::array<int, 4>, std::shared_ptr<BandPlan>>> todo;
         double work = 0.0;  // about 75 ns each
-        for (auto it = shapes.rbegin(); it != shapes.rend(); ++it) {  // largest first
-          const std::array<int, 3> &k = it->first;
-          const std::array<int, 4> key{k[0], k[1], k[2], cuts_for(steps[{k[0], k[1]}], C)};
-          if (made.count(key)) continue;
-          todo.push_back({key, nullptr});
-          work += (double)k[0] * (k[1] + 1) * (k[1] + 1);
+        for (auto it = need.rbegin(); it != need.rend(); ++it) {  // largest first
+          if (made.count(*it)) continue;
+          todo.push_back({*it, nullptr});
+          work += (double)(*it)[0] * ((*it)[1] + 1) * ((*it)[1] + 1);
         }
         auto make = [&](int i) {
           const std::array<int, 4> &k = todo[i].first;
@@ -1102,56 +1106,71 @@ void plan_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
           } catch (...) {  // made again below, where the caller can see the exception
           }
         };
-        if (work > 16384.0) parallel_cells((int)todo.size(), make);
-        else for (int i = 0; i < (int)todo.size(); ++i) make(i);  // starting threads takes longer
+        if (work > 4096.0) parallel_cells((int)todo.size(), make);
+        else for (int i = 0; i < (int)todo.size(); ++i) make(i);
         for (auto &t : todo)
-          if (t.second) made[t.first] = t.second;
+          made[t.first] = t.second ? t.second
+                                   : std::make_shared<BandPlan>(
+                                         make_band_plan(t.first[0], t.first[1], t.first[2] != 0, t.first[3]));
       };
-      double best = 1e300;
-      int best_c = INT_MAX;
-      for (int C : cand) {
-        int levels = 0;
-        for (auto &sh : shapes) {
-          const auto &st = steps[{sh.first[0], sh.first[1]}];
-          levels = std::max(levels, st[cuts_for(st, C)]);
-        }
-        // every level holds a pivot: a candidate whose launches alone take longer needs no plans
-        if (levels * (1.5 + LuPlan::inv_time(0, f64)) >= best) continue;
-        make_plans(C);
-        levels = 0;
+      // a candidate's estimated time (any value from `limit` on: not below it)
+      auto estimate = [&](int C, double limit) {
+        size_t levels = 0;
         double sweep = 0.0;
         bool split = false;
         std::vector<std::vector<std::pair<const BandPlan::Level *, int>>> by_level;
         for (auto &sh : shapes) {
-          CellParams p{};
-          p.nblk = sh.first[0];
-          p.bw = sh.first[1];
-          p.sym = sh.first[2];
-          const std::shared_ptr<BandPlan> P = plan_of(p, cuts_for(steps[{p.nblk, p.bw}], C));
-          levels = std::max(levels, (int)P->lev.size());
+          const BandPlan &P = *made.at(key_of(sh.first, C));
+          levels = std::max(levels, P.lev.size());
           by_level.resize(levels);
-          for (size_t l = 0; l < P->lev.size(); ++l) by_level[l].push_back({&P->lev[l], sh.second});
+          for (size_t l = 0; l < P.lev.size(); ++l) by_level[l].push_back({&P.lev[l], sh.second});
           int f = 0, w = 0;
-          for (size_t q = 0; q < P->fwd.size(); ++q) {
-            f = std::max(f, P->fwd[q].nop);
-            w = std::max(w, P->bwd[q].nop);
+          for (size_t q = 0; q < P.fwd.size(); ++q) {
+            f = std::max(f, P.fwd[q].nop);
+            w = std::max(w, P.bwd[q].nop);
           }
-          split |= P->top.nop > 0;
-          double top = t_op * (P->top.nop + P->top_bwd.nop), apart = t_op * (P->root.nop + P->root_bwd.nop);
-          for (size_t q = 1; q < P->sep_fwd.size(); ++q)
-            apart += 15.0 + t_op * (P->sep_fwd[q][0].nop + 2.0 * P->sep_bwd[q][0].nop);
-          if (P->root.nloc > 0) top = std::min(top, apart);
+          split |= P.top.nop > 0;
+          double top = t_op * (P.top.nop + P.top_bwd.nop), apart = t_op * (P.root.nop + P.root_bwd.nop);
+          for (size_t q = 1; q < P.sep_fwd.size(); ++q)
+            apart += 15.0 + t_op * (P.sep_fwd[q][0].nop + 2.0 * P.sep_bwd[q][0].nop);
+          if (P.root.nloc > 0) top = std::min(top, apart);
           sweep = std::max(sweep, t_op * (f + 2.0 * w) + top);
         }
         double t = sweep + (split ? 30.0 : 0.0);
-        for (int l = 0; l < levels && t < best; ++l) {
+        for (size_t l = 0; l < levels && t < limit; ++l) {
           double tl = 0.0;
           LuPlan::choose_deal(by_level[l], 1, f64, slots, &tl);  // the cuts do not depend on fused_step
           t += tl;
         }
-        if (t < best) {
-          best = t;
-          best_c = C;
+        return t;
+      };
+      double best = 1e300;
+      int best_c = INT_MAX;
+      if (!cand.empty()) {
+        // the most cuts first; of the others only those whose launches alone (a
+        // level holds a pivot at least) take less
+        make_plans({cand[0]});
+        best = estimate(best_c = cand[0], 1e300);
+        std::vector<int> left;
+        for (size_t i = 1; i < cand.size(); ++i) {
+          int levels = 0;
+          for (auto &sh : shapes) {
+            const auto &st = steps[{sh.first[0], sh.first[1]}];
+            levels = std::max(levels, st[cuts_for(st, cand[i])]);
+          }
+          if (levels * (1.5 + LuPlan::inv_time(0, f64)) < best) left.push_back(cand[i]);
+        }
+        make_plans(left);
+        std::vector<double> t(left.size(), 1e300);
+        if (left.size() * shapes.size() > 512) {
+          parallel_cells((int)left.size(), [&](int i) { t[i] = estimate(left[i], 1e300); });
+        }
+        for (size_t i = 0; i < left.size(); ++i) {
+          if (t[i] == 1e300) t[i] = estimate(left[i], best);
+          if (t[i] < best) {
+            best = t[i];
+            best_c = left[i];
+          }
         }
       }
       for (int c = 0; c < b.ncell; ++c)
