@@ -670,6 +670,65 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_band_sweep(const CellParams *
                 rowb);
 }
 
+// sum over a cell's boundary vertices of g . v
+__device__ __forceinline__ double boundary_gdot(const CellParams &p, const BndView &bv, const double *v, double *red) {
+  double a = 0.0;
+  for (int b = p.bnd_off + threadIdx.x; b < p.bnd_off + p.n_bnd; b += SWEEP_THREADS) {
+    if (bv.frame[b].x < 0) continue;
+    const double2 g = bv.g[b], d = reinterpret_cast<const double2 *>(v)[bv.node[b]];
+    a += g.x * d.x + g.y * d.y;
+  }
+  return block_sum<SWEEP_THREADS>(a, red);
+}
+// A cell with smw: its step inc - z t as direction nd (P0: the cell's
+// directions), orthogonal (its K times) to the ones before it, and delta along
+// it to the least residual; false: no direction.  A function of its own with
+// its arguments in memory: inline it took the sweeps' registers (905-element
+// cell, load step: 8 us).
+__device__ __attribute__((noinline)) bool refine_direction(const RefineArgs *args, const CellParams *cp, double *P0, int nd,
+                                                           double t, double *red) {
+  const RefineArgs &ra = *args;
+  const CellParams &p = *cp;
+  const int n0 = p.node_off, n2 = 2 * p.n_nodes;
+  double *P = P0 + 2LL * nd * n2, *Q = P + n2;
+  for (int i = threadIdx.x; i < n2; i += SWEEP_THREADS) {
+    const double d = ra.inc[2 * n0 + i];
+    P[i] = t != 0.0 ? d - ra.z[2 * n0 + i] * t : d;
+  }
+  __syncthreads();
+  const double gd = boundary_gdot(p, ra.bv, P - 2 * n0, red);
+  for (int i = threadIdx.x; i < p.n_nodes; i += SWEEP_THREADS) {
+    const double2 q = product_node(n0 + i, ra.el_tri, ra.adj_start, ra.adj, ra.Ke64, P - 2 * n0, p, ra.bv, gd);
+    Q[2 * i] = q.x;
+    Q[2 * i + 1] = q.y;
+  }
+  __syncthreads();
+  auto dot = [&](const double *a, const double *b) {
+    double v = 0.0;
+    for (int i = threadIdx.x; i < n2; i += SWEEP_THREADS) v += a[i] * b[i];
+    return block_sum<SWEEP_THREADS>(v, red);
+  };
+#pragma unroll 1
+  for (int k = 0; k < 2 * nd; ++k) {  // twice: one pass leaves what cancellation made
+    const double *Pk = P0 + 2LL * (k % nd) * n2, *Qk = Pk + n2;
+    const double a = dot(Qk, Q);
+    for (int i = threadIdx.x; i < n2; i += SWEEP_THREADS) {
+      P[i] -= a * Pk[i];
+      Q[i] -= a * Qk[i];
+    }
+  }
+  const double qq = dot(Q, Q), s = 1.0 / sqrt(qq);
+  if (!(qq > 0.0 && s > 0.0)) return false;  // nothing new, or not finite
+  const double a = s * s * dot(Q, ra.r + 2 * n0);
+  for (int i = threadIdx.x; i < n2; i += SWEEP_THREADS) {
+    ra.delta[2 * n0 + i] += a * P[i];
+    P[i] *= s;
+    Q[i] *= s;
+  }
+  __syncthreads();
+  return true;
+}
+
 // The whole refinement of one cell: sweep, FP64 residual, norm and control,
 // again until lin_rtol is met.  Small cells: a sweep streams few blocks, so
 // five launches per refinement sweep (also of the sweeps that have nothing
@@ -696,7 +755,9 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_band_sweep(const CellParams *
 // condition 2e3 to 4e5 three to six in all to 1e-8, where sweeps by the rank
 // one formula alone stood at 0.03 to 0.8 of the residual after four.
 constexpr double REFINE_POOR = 1.0 / 16.0, REFINE_FLOOR = 1e-13;  // FLOOR: rounding of the FP64 residual
-template <class T>
+// SMW: a batch with cells with smw (without them the kernel holds neither path
+// of theirs: 1.5 % of the 905-element FP64 step).
+template <class T, bool SMW>
 __global__ __launch_bounds__(SWEEP_THREADS) void k_band_refine(const CellParams *cp, CellState *cs,
                                                                const RefineWG *wgs, const SweepOp *ops,
                                                                const SweepLoc *locs, const int *accs, const T *K,
@@ -712,37 +773,22 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_band_refine(const CellParams 
   if (cs[c].ir_done) return;
   const CellParams &p = cp[c];
   const int n0 = p.node_off, n1 = n0 + p.n_nodes;
-  // sum over the boundary vertices of g . v
-  auto gdot = [&](const double *v) {
-    double a = 0.0;
-    for (int b = p.bnd_off + threadIdx.x; b < p.bnd_off + p.n_bnd; b += SWEEP_THREADS) {
-      if (ra.bv.frame[b].x < 0) continue;
-      const double2 g = ra.bv.g[b], d = reinterpret_cast<const double2 *>(v)[ra.bv.node[b]];
-      a += g.x * d.x + g.y * d.y;
-    }
-    return block_sum<SWEEP_THREADS>(a, red);
-  };
+  auto gdot = [&](const double *v) { return boundary_gdot(p, ra.bv, v, red); };
   auto g_of = [&](int i) {
     const int b = ra.bv.bidx[i];
     return b >= 0 && ra.bv.frame[b].x >= 0 ? ra.bv.g[b] : make_double2(0.0, 0.0);
   };
-  double den = 1.0;
-  if (p.smw) {
+  const bool smw = SMW && p.smw;
+  if (smw) {  // the first sweep below: z = B^-1 k g
     for (int i = n0 + threadIdx.x; i < n1; i += SWEEP_THREADS) {
       const double2 g = g_of(i);
       ra.inc[2 * i] = p.k_area * g.x;
       ra.inc[2 * i + 1] = p.k_area * g.y;
     }
     __syncthreads();
-    SweepVec<T> v = sv;
-    v.rhs = ra.inc;
-    v.delta = ra.z;
-    v.from_y = 0;
-    sweep_part<T>(p, wg.whole, ops, locs, accs, K, Dinv, kinv, v, 0, y, rowb);
-    __syncthreads();
-    den = 1.0 + gdot(ra.z);
   }
-  bool rank1 = fabs(den) > 0.0 && fabs(den) < 1e300;
+  double den = 1.0;
+  bool rank1 = true;
   if (ra.it0 == 0 && !ra.fwd_done) {
     for (int i = 2 * n0 + threadIdx.x; i < 2 * n1; i += SWEEP_THREADS) ra.r[i] = -ra.G[i];
     __syncthreads();
@@ -759,58 +805,17 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_band_refine(const CellParams 
     return block_sum<SWEEP_THREADS>(rr, red);
   };
   auto step = [&](int i, double t) { return t != 0.0 ? ra.inc[i] - ra.z[i] * t : ra.inc[i]; };
-  // cells with smw: the step as direction nd, orthogonal (its K times) to the
-  // ones before it, and delta along it to the least residual; false: no direction
-  int nd = -1;  // -1: plain refinement
-  auto direction = [&](double t) {
-    const int n2 = 2 * p.n_nodes;
-    double *P0 = ra.dirs + wg.dirs;
-    double *P = P0 + 2LL * nd * n2, *Q = P + n2;
-    for (int i = threadIdx.x; i < n2; i += SWEEP_THREADS) P[i] = step(2 * n0 + i, t);
-    __syncthreads();
-    const double gd = gdot(P - 2 * n0);
-    for (int i = threadIdx.x; i < p.n_nodes; i += SWEEP_THREADS) {
-      const double2 q =
-          product_node(n0 + i, ra.el_tri, ra.adj_start, ra.adj, ra.Ke64, P - 2 * n0, p, ra.bv, gd);
-      Q[2 * i] = q.x;
-      Q[2 * i + 1] = q.y;
-    }
-    __syncthreads();
-    auto dot = [&](const double *a, const double *b) {
-      double v = 0.0;
-      for (int i = threadIdx.x; i < n2; i += SWEEP_THREADS) v += a[i] * b[i];
-      return block_sum<SWEEP_THREADS>(v, red);
-    };
-#pragma unroll 1
-    for (int k = 0; k < 2 * nd; ++k) {  // twice: one pass leaves what cancellation made
-      const double *Pk = P0 + 2LL * (k % nd) * n2, *Qk = Pk + n2;
-      const double a = dot(Qk, Q);
-      for (int i = threadIdx.x; i < n2; i += SWEEP_THREADS) {
-        P[i] -= a * Pk[i];
-        Q[i] -= a * Qk[i];
-      }
-    }
-    const double qq = dot(Q, Q), s = 1.0 / sqrt(qq);
-    if (!(qq > 0.0 && s > 0.0)) return false;  // nothing new, or not finite
-    const double a = s * s * dot(Q, ra.r + 2 * n0);
-    for (int i = threadIdx.x; i < n2; i += SWEEP_THREADS) {
-      ra.delta[2 * n0 + i] += a * P[i];
-      P[i] *= s;
-      Q[i] *= s;
-    }
-    __syncthreads();
-    nd = nd + 1 < REFINE_DIRS ? nd + 1 : 0;
-    return true;
-  };
+  int nd = -1;  // cells with smw: directions so far (refine_direction); -1: plain refinement
   const double bnorm = cs[c].bnorm;
   double last = bnorm, y1 = 0.0;  // y1: the first guess of g . d
   int most = ra.max_refine;
-  for (int it = ra.it0; it < most; ++it) {
+  for (int it = smw ? ra.it0 - 1 : ra.it0; it < most; ++it) {
+    const bool zsweep = smw && it < ra.it0;
     SweepVec<T> v = sv;
-    v.rhs = ra.r;
+    v.rhs = zsweep ? ra.inc : ra.r;
     v.from_y = it == 0 && ra.fwd_done ? 1 : 0;
-    v.delta = p.smw ? ra.inc : ra.delta;
-    if (nd >= 0) {
+    v.delta = zsweep ? ra.z : smw ? ra.inc : ra.delta;
+    if (smw && nd >= 0) {
       double s = 0.0;
       for (int i = 2 * n0 + threadIdx.x; i < 2 * n1; i += SWEEP_THREADS) s += ra.z[i] * ra.r[i];
       s = rank1 ? block_sum<SWEEP_THREADS>(s, red) / den : 0.0;
@@ -823,45 +828,51 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_band_refine(const CellParams 
       __syncthreads();
       v.rhs = ra.inc;
     }
-    sweep_part<T>(p, v.from_y ? wg.bwd : wg.whole, ops, locs, accs, K, Dinv, kinv, v, p.smw ? 0 : it > 0, y, rowb);
+    sweep_part<T>(p, v.from_y ? wg.bwd : wg.whole, ops, locs, accs, K, Dinv, kinv, v, smw ? 0 : it > 0, y, rowb);
     __syncthreads();
-    const double t = p.smw && rank1 ? (gdot(ra.inc) - y1) / den : 0.0;
-    bool stop = false;
-    double rr;
-    if (nd < 0) {
-      if (p.smw) {
+    if (zsweep) {
+      den = 1.0 + gdot(ra.z);
+      rank1 = fabs(den) > 0.0 && fabs(den) < 1e300;
+      continue;
+    }
+    const double t = smw && rank1 ? (gdot(ra.inc) - y1) / den : 0.0;
+    bool stop = false, undone = false;
+    if (smw && nd >= 0) {
+      stop = !refine_direction(ra.mem, &p, ra.dirs + wg.dirs, nd, t, red);
+      if (!stop) nd = nd + 1 < REFINE_DIRS ? nd + 1 : 0;
+      if (stop && rank1) rank1 = stop = false;  // without the rank one: B alone, one direction more
+    } else if (smw) {
+      for (int i = 2 * n0 + threadIdx.x; i < 2 * n1; i += SWEEP_THREADS) {
+        const double d = step(i, t);
+        ra.delta[i] = it > 0 ? ra.delta[i] + d : d;
+      }
+      __syncthreads();
+    }
+    double nrm;
+#pragma unroll 1
+    for (;;) {
+      nrm = sqrt(residual());
+      if (!smw || nd >= 0 || undone) break;
+      const bool poor = !(nrm <= ra.lin_rtol * bnorm) && !(nrm <= REFINE_FLOOR * bnorm) &&
+                        (!(nrm <= REFINE_POOR * last) || it + 1 == ra.max_refine);
+      if (poor) most = ra.max_refine + REFINE_MORE;
+      if (poor && !(nrm <= last)) {  // worse than before the sweep: without it
         for (int i = 2 * n0 + threadIdx.x; i < 2 * n1; i += SWEEP_THREADS) {
-          const double d = step(i, t);
-          ra.delta[i] = it > 0 ? ra.delta[i] + d : d;
+          const double b = it > 0 ? ra.delta[i] - step(i, t) : 0.0;
+          ra.delta[i] = fabs(b) < 1e300 ? b : 0.0;
         }
         __syncthreads();
-      }
-      rr = residual();
-      const double nrm = sqrt(rr);
-      if (p.smw && !(nrm <= ra.lin_rtol * bnorm) && !(nrm <= REFINE_FLOOR * bnorm) &&
-          (!(nrm <= REFINE_POOR * last) || it + 1 == ra.max_refine)) {
-        if (!(nrm <= last)) {  // worse than before the sweep: without it
-          for (int i = 2 * n0 + threadIdx.x; i < 2 * n1; i += SWEEP_THREADS) {
-            const double b = it > 0 ? ra.delta[i] - step(i, t) : 0.0;
-            ra.delta[i] = fabs(b) < 1e300 ? b : 0.0;
-          }
-          __syncthreads();
-          rr = residual();
-        }
-        nd = 0;
-        most = ra.max_refine + REFINE_MORE;
+        undone = true;
+        continue;
       }
       last = nrm;
-    } else {
-      stop = !direction(t);
-      if (stop && rank1) {  // without the rank one: B alone, one direction more
-        rank1 = stop = false;
-      }
-      rr = residual();
+      if (poor) nd = 0;
+      break;
     }
+    if (undone) nd = 0;
     if (threadIdx.x == 0) {
       CellState &s = cs[c];
-      norm_finish(s, 1, sqrt(rr), ra.lin_rtol);
+      norm_finish(s, 1, nrm, ra.lin_rtol);
       done = s.ir_done;
     }
     __syncthreads();
@@ -874,8 +885,9 @@ void launch_band_refine(hipStream_t s, const CellParams *cp, CellState *cs, cons
                         const SweepOp *ops, const SweepLoc *locs, const int *accs, const T *K, const T *Dinv,
                         const int *kinv, const SweepVec<T> &sv, const RefineArgs &ra) {
   if (nwg <= 0) return;
-  hipLaunchKernelGGL(k_band_refine<T>, dim3(nwg), dim3(SWEEP_THREADS), (size_t)max_loc * NB * sizeof(T), s, cp, cs,
-                     wgs, ops, locs, accs, K, Dinv, kinv, sv, ra);
+  const auto k = ra.dirs ? &k_band_refine<T, true> : &k_band_refine<T, false>;
+  hipLaunchKernelGGL(k, dim3(nwg), dim3(SWEEP_THREADS), (size_t)max_loc * NB * sizeof(T), s, cp, cs, wgs, ops, locs,
+                     accs, K, Dinv, kinv, sv, ra);
 }
 template <class T>
 void launch_band_sweep(hipStream_t s, const CellParams *cp, const CellState *cs, const SweepWG *wgs, int nwg,
@@ -889,8 +901,10 @@ void launch_band_sweep(hipStream_t s, const CellParams *cp, const CellState *cs,
 hipError_t band_prepare_attributes(size_t max_lds) {
   const int dyn = (int)lu_solve_max_dynamic(max_lds);
   const int ref = (int)refine_max_dynamic(max_lds);
-  const std::pair<const void *, int> fns[] = {{reinterpret_cast<const void *>(&k_band_refine<float>), ref},
-                                              {reinterpret_cast<const void *>(&k_band_refine<double>), ref},
+  const std::pair<const void *, int> fns[] = {{reinterpret_cast<const void *>(&k_band_refine<float, false>), ref},
+                                              {reinterpret_cast<const void *>(&k_band_refine<float, true>), ref},
+                                              {reinterpret_cast<const void *>(&k_band_refine<double, false>), ref},
+                                              {reinterpret_cast<const void *>(&k_band_refine<double, true>), ref},
                                               {reinterpret_cast<const void *>(&k_band_sweep<float>), dyn},
                                               {reinterpret_cast<const void *>(&k_band_sweep<double>), dyn},
                                               {reinterpret_cast<const void *>(&k_lu_step_f64), step_lds<double>()}};

@@ -743,6 +743,7 @@ struct Batch {
   // (tail) those of which it runs the sweeps after the second, which few need
   RefineWG *rwg = nullptr;
   double *dirs = nullptr;
+  RefineArgs *rargs = nullptr;
   int nrefine = 0, ntail = 0, refine_loc = 0;
   std::vector<int> refine_at;  // per cell: its place in rwg, or -1
   bool tail = false;
@@ -765,7 +766,7 @@ struct Batch {
 
   void release() {
     void *ptrs[] = {X, x, fau, ea, cC, el_tri, el_cell, el_spr, sp_bary, sp_anchor, sp_state, sp_cell, sp_elem,
-                    sp_local, cp, cs, node_cell, adj_start, adj, Ge, g_start, g_col, g_bpos, g_cstart, g_ke, g_node, Ke64, G, r, delta, Rea, MM, K, Dinv, ysol, sync, ipiv, cells, celem, rwg, dirs,
+                    sp_local, cp, cs, node_cell, adj_start, adj, Ge, g_start, g_col, g_bpos, g_cstart, g_ke, g_node, Ke64, G, r, delta, Rea, MM, K, Dinv, ysol, sync, ipiv, cells, celem, rwg, dirs, rargs,
                     replica, transitions, plan.d_prefix, row_ptr, bcol, diag_pos, el_bpos, csr_cells, chunks, Kb,
                     cgvec, cg, partials, norm_part, norm_cnt, kpos, kinv, yfwd, ysw, slots, rank, refs, fops, sops, slocs, saccs, swg, plan.d_items, plan.d_ranges, plan.d_solve, rp, dp, bt_bidx, bt_node, bt_cst, crange, bt_cand, bt_frame, bt_g, bt_J, bt_area,
                     bt_gd, bt_fext};
@@ -981,6 +982,24 @@ View make_view(const wcfe_ctx *ctx, const Batch &b) {
   v.tab_px = ctx->tab_px; v.tab_py = ctx->tab_py; v.tab_k = ctx->tab_k;
   v.kappa = ctx->opt.kappa;
   return v;
+}
+
+BndView bnd_view(const wcfe_ctx *ctx, const Batch &b) {
+  BndView bv;
+  bv.bidx = b.bt_bidx; bv.node = b.bt_node; bv.cst = b.bt_cst; bv.cand = b.bt_cand;
+  bv.frame = b.bt_frame; bv.g = b.bt_g; bv.J = b.bt_J; bv.area = b.bt_area; bv.gd = b.bt_gd;
+  bv.replica = b.replica;
+  bv.fext = b.bt_fext;
+  bv.dt = ctx->opt.dt;
+  bv.key_lo = ctx->opt.seed_lo;
+  bv.key_hi = ctx->opt.seed_hi;
+  return bv;
+}
+
+// The arrays of k_band_refine (it0 and mem are the launch's).
+RefineArgs refine_args(const wcfe_ctx *ctx, const Batch &b) {
+  return RefineArgs{b.el_tri, b.adj_start, b.adj, b.Ke64, b.G, b.r, b.delta, b.rp, b.dp, b.dirs, bnd_view(ctx, b),
+                    ctx->opt.lin_rtol, 0, std::max(1, ctx->opt.max_refine), b.plan.fused ? 1 : 0, nullptr};
 }
 
 // Lay out cells in HBM.  Elements are stored colour-major (colour k of every
@@ -1361,7 +1380,10 @@ void upload_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
     for (int c : spread) one_wg(c);
   b.ntail = (int)rwg.size() - b.nrefine;
   b.rwg = dupload(rwg);
-  if (dirs > 0) b.dirs = dalloc<double>(dirs);
+  if (dirs > 0) {
+    b.dirs = dalloc<double>(dirs);
+    b.rargs = dupload(std::vector<RefineArgs>{refine_args(ctx, b)});
+  }
   // separators by depth if that is the shorter: per cell the longest part of
   // each depth instead of the sum of all, for two launches more per depth and
   // refinement sweep and one in the first solve (one cell of 20000 elements,
@@ -1980,18 +2002,6 @@ template <class T> CgVectors<T> cg_vectors(const Batch &b) {
                       base + 4 * n2, base + 5 * n2, base + 6 * n2, (long long)std::max(b.nchunk, 1)};
 }
 
-BndView bnd_view(const wcfe_ctx *ctx, const Batch &b) {
-  BndView bv;
-  bv.bidx = b.bt_bidx; bv.node = b.bt_node; bv.cst = b.bt_cst; bv.cand = b.bt_cand;
-  bv.frame = b.bt_frame; bv.g = b.bt_g; bv.J = b.bt_J; bv.area = b.bt_area; bv.gd = b.bt_gd;
-  bv.replica = b.replica;
-  bv.fext = b.bt_fext;
-  bv.dt = ctx->opt.dt;
-  bv.key_lo = ctx->opt.seed_lo;
-  bv.key_hi = ctx->opt.seed_hi;
-  return bv;
-}
-
 // Element assembly colour by colour; in FULL and RESIDUAL mode followed by
 // the node terms (boundary and body forces) of the cells that have them.
 template <class T> void enqueue_assemble(wcfe_ctx *ctx, Batch &b, const Scope &sc, int mode) {
@@ -2253,10 +2263,11 @@ template <class T> void enqueue_solve_refine(wcfe_ctx *ctx, Batch &b, const Scop
   const int max_refine = std::max(1, ctx->opt.max_refine);
   auto refine = [&](int first, int n, int it0) {
     PhaseScope ph(ctx, WCFE_PH_SOLVE);
+    RefineArgs ra = refine_args(ctx, b);
+    ra.it0 = it0;
+    ra.mem = b.rargs;
     launch_band_refine<T>(s, b.cp, b.cs, b.rwg + first, n, b.refine_loc, b.sops, b.slocs, b.saccs, K,
-                          static_cast<const T *>(b.Dinv), b.kinv, sweep_vec<T>(b, b.plan.fused),
-                          RefineArgs{b.el_tri, b.adj_start, b.adj, b.Ke64, b.G, b.r, b.delta, b.rp, b.dp, b.dirs,
-                                     bnd_view(ctx, b), ctx->opt.lin_rtol, it0, max_refine, b.plan.fused ? 1 : 0});
+                          static_cast<const T *>(b.Dinv), b.kinv, sweep_vec<T>(b, b.plan.fused), ra);
   };
   refine(w0, nref, 0);
   if (!spread) return;

@@ -227,6 +227,7 @@ struct RefineArgs {
   BndView bv;
   double lin_rtol;
   int it0, max_refine, fwd_done;
+  const RefineArgs *mem;  // the same pointers in device memory, for the path that seldom runs (cells with smw)
 };
 size_t refine_max_dynamic(size_t max_lds);
 template <class T>
