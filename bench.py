@@ -323,7 +323,7 @@ def run_workload(W, configs, name, cells, tables, steps, warmup, common, precisi
     st = ctx.newton_step(stats=True, check=False)
     prof = ctx.profile_step()
     sched = ctx.schedule()
-    sched["two_chain_cells"] = sum(ctx.cell_layout(i)["chain_top"] > 0 for i in range(len(cells)))
+    sched["cut_cells"] = sum(ctx.cell_layout(i)["leaves"] > 1 for i in range(len(cells)))
     ctx.close()
     n_tri = sum(len(c["tris"]) for c in cells)
     fp64 = precision == W.PREC_FP64
@@ -358,7 +358,7 @@ def main():
     ap.add_argument("--fused-step", type=int, choices=[0, 1, 2, 3, 4, 5], default=None,
                     help="band-LU block-step mode (library default when omitted)")
     ap.add_argument("--twist", type=int, choices=[0, 1, 2], default=None,
-                    help="two-chain band LU: 0 off, 1 automatic (default), 2 always")
+                    help="cuts of the band LU: 0 none, 1 automatic (default), 2 one per longer cell")
     ap.add_argument("--pcg-lanes", type=int, choices=[4, 8, 16], default=None,
                     help="block-CSR PCG: lanes per block row in the SpMV (default 8)")
     ap.add_argument("--copy-probe", type=int, default=0, metavar="MIB",
@@ -416,7 +416,7 @@ def main():
     prof = ctx.profile_step()
     sched = ctx.schedule()
     layouts = [ctx.cell_layout(i) for i in range(len(cells))]
-    sched["two_chain_cells"] = sum(L["chain_top"] > 0 for L in layouts)
+    sched["cut_cells"] = sum(L["leaves"] > 1 for L in layouts)
     ctx.close()
     log("check step:", st)
     log("phases:", {k: round(v["ms"], 3) for k, v in prof.items()})

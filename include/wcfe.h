@@ -260,8 +260,8 @@ int wcfe_synchronize(wcfe_ctx *ctx);
  * (pcg_lanes 4, 8, 16).  Every trial starts from the state the cells were
  * added with, and so does the batch afterwards: call it after wcfe_finalize
  * and before any Newton step.  chosen (optional, 6 entries): lu_depth,
- * lu_groups, dense_max_dof, fused_step, the number of cut cells
- * (wcfe_get_cell_layout) and
+ * lu_groups, dense_max_dof, fused_step, the number of cells for which
+ * wcfe_get_cell_layout reports chains (wcfe_get_cell_cuts: which are cut) and
  * pcg_lanes in effect; ms_best (optional): ms per step. */
 #define WCFE_TUNE_SOLVER 1
 #define WCFE_TUNE_LU 2
@@ -347,11 +347,17 @@ int wcfe_get_cell_sizes(wcfe_ctx *ctx, int32_t cell, int32_t *n_nodes, int32_t *
  * WCFE_SOLVER_CSR), 64-row blocks of its dense system, their block bandwidth
  * in the band numbering (nblk - 1: full matrix), symmetric factorization, and
  * for a cut cell (wcfe_options.twist) longer than the batch's shortest chain
- * of halved cells the blocks of its two halves around a separator in the
- * middle (0, 0: uncut, or cut although a shorter cell; deeper cuts are not
- * reported). */
+ * of halved cells the blocks of the two chains that measure is taken from: m
+ * top down and n bottom up around a window of bw blocks, n <= m - bw (0, 0:
+ * uncut, or cut although a shorter cell).  The cuts themselves lie elsewhere
+ * and may be many: wcfe_get_cell_cuts. */
 int wcfe_get_cell_layout(wcfe_ctx *ctx, int32_t cell, int32_t *solver, int32_t *nblk, int32_t *bw, int32_t *sym,
                          int32_t *chain_top, int32_t *chain_bottom);
+/* The cuts of a dense cell's band in the plan that runs: leaves, the
+ * independent parts that are eliminated at the same time (1: uncut; 0: no plan,
+ * a sparse cell or a full matrix on separate launches), and levels, its
+ * dependent block steps, the separators' included (nblk when uncut). */
+int wcfe_get_cell_cuts(wcfe_ctx *ctx, int32_t cell, int32_t *leaves, int32_t *levels);
 int wcfe_get_cell_info(wcfe_ctx *ctx, int32_t cell, double *time, int32_t *step, int32_t *newton_iter,
                        int32_t *n_colors, int32_t *ndof);
 /* FP64 residual G(x) = R_int(x) - F_spring(x) at the current positions (2N). */

@@ -37,7 +37,7 @@ EXPORTS = [
     "wcfe_copy_probe", "wcfe_autotune", "wcfe_set_ul_state", "wcfe_replace_cell", "wcfe_checkpoint_save",
     "wcfe_checkpoint_load", "wcfe_area_tot", "wcfe_bending_force_2d", "wcfe_area_constraint_force",
     "wcfe_force_ap", "wcfe_get_schedule", "wcfe_num_cells", "wcfe_get_cell_sizes",
-    "wcfe_eval_exp", "wcfe_get_cell_layout", "wcfe_force_fa_noalloc", "wcfe_remesh_cell",
+    "wcfe_eval_exp", "wcfe_get_cell_layout", "wcfe_get_cell_cuts", "wcfe_force_fa_noalloc", "wcfe_remesh_cell",
 ]
 TUNE_SOLVER, TUNE_LU, TUNE_PCG = 1, 2, 4
 # reference constants of the boundary and body forces (UL_growth_explicit.cpp)
@@ -415,12 +415,16 @@ class Context:
     def cell_layout(self, cell):
         """solver (SOLVER_DENSE / SOLVER_CSR), nblk (64-row blocks), bw (block
         bandwidth in the band numbering), sym (symmetric factorization),
-        chain_top / chain_bottom (two-chain band LU: blocks of each chain; 0:
-        one chain)."""
+        leaves (independent parts the band is cut into; 1: uncut, 0: no band
+        plan) and levels (its dependent block steps); chain_top / chain_bottom:
+        the two chains that the choice of cells measures a halved cell by, not
+        the cuts in use (0: uncut, or cut although a shorter cell)."""
         v = [C.c_int32(0) for _ in range(6)]
         self._check(self._L.wcfe_get_cell_layout(self._h, cell, *[C.byref(x) for x in v]))
+        leaves, levels = C.c_int32(0), C.c_int32(0)
+        self._check(self._L.wcfe_get_cell_cuts(self._h, cell, C.byref(leaves), C.byref(levels)))
         return dict(solver=v[0].value, nblk=v[1].value, bw=v[2].value, sym=v[3].value, chain_top=v[4].value,
-                    chain_bottom=v[5].value)
+                    chain_bottom=v[5].value, leaves=leaves.value, levels=levels.value)
 
     def residual(self, cell):
         G = np.zeros(2 * self.cells[cell]["n_nodes"])

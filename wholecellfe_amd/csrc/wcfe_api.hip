@@ -719,7 +719,7 @@ struct Batch {
   // separators (all of it, or backward only), the leaves backward; a batch
   // without separators runs its whole sweeps in one launch
   std::vector<std::shared_ptr<BandPlan>> plans;
-  std::vector<int> chain_top, chain_bottom;  // reported layout (wcfe_get_cell_layout)
+  std::vector<int> chain_top, chain_bottom;  // the measure of halved cells (wcfe_get_cell_layout)
   int nslot = 0;
   int *rank = nullptr;
   BlockRef *refs = nullptr;
@@ -1069,8 +1069,9 @@ void plan_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
     }
     return best;
   };
-  // the reported two-chain layout: cells longer than the shortest batch of
-  // cells cut once
+  // what a halved cell is measured by: two chains of m and nb blocks that meet
+  // in a window of bw (the cut of band_plan.hpp is the more even one); twist 2
+  // cuts the cells longer than the shortest batch of such
   int chain2 = 0;
   auto halves = [](const CellParams &p, int &m, int &nb) {
     if (p.csr || p.bw < 1 || p.bw >= p.nblk - 1 || p.nblk - 2 * p.bw < 2) return false;
@@ -3298,6 +3299,16 @@ int wcfe_get_cell_layout(wcfe_ctx *ctx, int32_t cell, int32_t *solver, int32_t *
     if (sym) *sym = p.sym;
     if (chain_top) *chain_top = ctx->b.chain_top[cell];
     if (chain_bottom) *chain_bottom = ctx->b.chain_bottom[cell];
+  });
+}
+
+int wcfe_get_cell_cuts(wcfe_ctx *ctx, int32_t cell, int32_t *leaves, int32_t *levels) {
+  if (!ctx) return WCFE_ERR_ARG;
+  return guarded(ctx, [&] {
+    check_cell(ctx, cell);
+    const std::shared_ptr<BandPlan> &P = ctx->b.plans[cell];
+    if (leaves) *leaves = P ? P->leaves : 0;
+    if (levels) *levels = P ? (int)P->lev.size() : 0;
   });
 }
 
