@@ -240,8 +240,9 @@ int wcfe_checkpoint_load(wcfe_ctx *ctx, const char *path);
  * PCG checks convergence on the host every few iterations; such batches are
  * not captured in a graph).  With stats, the step's errors are returned:
  * WCFE_ERR_DEGENERATE, WCFE_ERR_ZERO_PIVOT, and WCFE_ERR_NOT_CONVERGED when a
- * cell's linear solve missed lin_rtol within max_refine sweeps (stats are
- * filled in every case; n_failed counts those cells). */
+ * cell's linear solve missed lin_rtol within max_refine sweeps (cells with the
+ * area term: up to 8 more, where sweeps stall; stats are filled in every case;
+ * n_failed counts those cells). */
 int wcfe_newton_step(wcfe_ctx *ctx, wcfe_step_stats *stats);
 /* Newton iterations until every cell has committed one load step. */
 int wcfe_load_step(wcfe_ctx *ctx, int32_t *iterations, wcfe_step_stats *stats);
@@ -252,10 +253,10 @@ int wcfe_synchronize(wcfe_ctx *ctx);
  * threshold (dense_max_dof, cells with solver AUTO; candidates that would not
  * fit in free device memory are skipped); WCFE_TUNE_LU: delayed-update depth
  * (1, 2, 4, 6) x concurrent cell groups (1, 2, 4), at depth 1 with and without
- * the fused block step, with split panel items (fused_step 5) and (mixed
- * precision, one group) the whole factorization in one launch (fused_step
- * 4); then, with fused block steps,
- * uncut cells against one cut per longer cell (twist 0 / 2); WCFE_TUNE_PCG
+ * the fused block step, with an item per column block (fused_step 5) and
+ * (mixed precision, one group) the whole factorization in one launch
+ * (fused_step 4); then, with fused block steps, uncut cells, the automatic
+ * cuts and one cut per longer cell (twist 0 / 1 / 2); WCFE_TUNE_PCG
  * (batches with block-CSR cells): lanes per block row of the PCG's SpMV
  * (pcg_lanes 4, 8, 16).  Every trial starts from the state the cells were
  * added with, and so does the batch afterwards: call it after wcfe_finalize

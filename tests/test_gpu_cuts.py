@@ -32,3 +32,17 @@ def test_reported_cuts(prec):
     assert alone["chain_top"] > 0
     sparse = layouts([ds[0]], precision=prec, dense_max_dof=0)[0]
     assert sparse["solver"] == W.SOLVER_CSR and sparse["leaves"] == 0 and sparse["levels"] == 0
+
+
+# one cell of 5400 elements whose band starts uncut: cut it takes about half
+# the time, in either precision
+@pytest.mark.parametrize("prec", [W.PREC_MIXED, W.PREC_FP64])
+def test_autotune_tries_the_cuts(prec):
+    d = cells.cst_cell(K=30, n_spr=300, seed=1, time=1.0)
+    with W.Context(t0=1.0, precision=prec, twist=0, lu_depth=1, lu_groups=1) as c:
+        cells.add_to_context(c, d)
+        c.finalize()
+        assert c.cell_layout(0)["leaves"] == 1
+        ch = c.autotune(W.TUNE_LU, steps=2)
+        print(ch, c.cell_layout(0), flush=True)
+        assert ch["fused_step"] > 0 and c.cell_layout(0)["leaves"] > 2

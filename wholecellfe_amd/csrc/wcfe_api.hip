@@ -2876,11 +2876,10 @@ int wcfe_autotune(wcfe_ctx *ctx, int32_t flags, int32_t steps, int32_t *chosen, 
       for (int d : depths)
         for (int g : groups)
           for (int f : {5, 4, 1, 0}) {
-            // the per-launch choice (1) covers the L-item, split panel and
-            // panel forms; 5 takes split panel items wherever 1 takes panel
-            // items; 4 (one workgroup per cell) with one group in FP32
+            // 1 prices the dealings of each launch, 5 is one of them; 4 (one
+            // workgroup per cell) with one group in FP32
             if (d > 1 && f != 1) continue;
-            if ((f == 4 && (g != 1 || !mixed(ctx))) || (f == 5 && !mixed(ctx))) continue;
+            if (f == 4 && (g != 1 || !mixed(ctx))) continue;
             ctx->opt = base;
             ctx->opt.lu_depth = d;
             ctx->opt.lu_groups = g;
@@ -2893,16 +2892,19 @@ int wcfe_autotune(wcfe_ctx *ctx, int32_t flags, int32_t steps, int32_t *chosen, 
             }
           }
     }
-    // 3. with fused block steps in FP32: one chain per cell against two-chain
-    //    cells for every cell longer than the batch needs (the automatic
-    //    rule splits only when the block steps are latency bound)
-    if ((flags & WCFE_TUNE_LU) && mixed(ctx) && best.fused_step >= 1 &&
-        (best.lu_depth == 1 || (best.lu_depth == 0 && ctx->b.lu_depth == 1))) {
+    // 3. fused block steps on narrow bands: uncut, the automatic cuts, one cut
+    //    per longer cell (also where another schedule of uncut bands was faster)
+    if ((flags & WCFE_TUNE_LU) && ctx->b.solve_wg) {
       const wcfe_options base = best;
-      for (int tw : {0, 2}) {
-        if (tw == base.twist) continue;
+      const bool fused = base.fused_step >= 1 && base.lu_depth <= 1;
+      for (int tw : {0, 1, 2}) {
+        if (fused ? tw == base.twist : tw == 0) continue;
         ctx->opt = base;
         ctx->opt.twist = tw;
+        if (!fused) {
+          ctx->opt.fused_step = 1;
+          ctx->opt.lu_depth = 1;
+        }
         const double ms = trial();
         if (ms < 1e300) tried.push_back({ms, ctx->opt});
         if (ms < best_ms) {
