@@ -1025,7 +1025,8 @@ template <class F> void parallel_cells(int ncell, F f) {
 // Workgroups of a block step that make headway at once: two FP32 ones fit a
 // compute unit but each then takes about twice as long (a launch of 322 items
 // over 256 compute units 24 us, of 850 about 60; alone an item takes 12), and
-// one FP64.
+// one FP64 (0.75: us per step at 0.5 / 0.75 / 1.0: 64 cells of 1000 elements
+// 386 / 375 / 379, 32 of 2000 618 / 601 / 655, 8 of 2000 435 / 423 / 436).
 double step_slots(const wcfe_ctx *ctx, int elem_size) { return (elem_size == 4 ? 1.0 : 0.75) * ctx->n_cu; }
 
 // time of one block product of a sweep's stream
@@ -1222,12 +1223,13 @@ void plan_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
 // ends the step (k_cell_finish).
 // REFINE_OPS: the block products of the longest whole sweep up to which the
 // whole refinement in one workgroup is the faster (us per Newton step, whole
-// / spread over launches: 12 products 92 / 107, 43 FP64 206 / 222, but about
-// 240: 32 cells 629 / 541, 256 cells 1641 / 1450, where the launches' other
-// workgroups work on the same cell).
-// FINISH_BATCH: likewise elements of the batch (85 elements 92 / 97, 905
-// 206 / 211, 32 UL cells 541 / 584, but 375000: 1450 / 1412, 1.07 million
-// 4555 / 4520).
+// / spread over launches: 12 products 92 / 107, 55 176 / 179, 64 cells 246 /
+// 272; 124, 64 cells: 484 / 469, FP64 659 / 653; 182, one cell: 301 / 263, FP64
+// 331 / 313, 16 cells 363 / 342, FP64 422 / 432; about 240, 256 cells 1641 /
+// 1450, where the launches' other workgroups work on the same cell).
+// FINISH_BATCH: likewise elements of a batch of cells up to FINISH_ELEMS (120
+// cells of 500 elements 212 / 227, 200 277 / 285; 60 of 2000 553 / 557, and
+// 375000 elements 1450 / 1412, 1.07 million 4555 / 4520).
 constexpr int REFINE_OPS = 96, FINISH_BATCH = 65536;
 void choose_refine(const wcfe_ctx *ctx, Batch &b, int elem_size) {
   b.finish = b.T <= FINISH_BATCH;

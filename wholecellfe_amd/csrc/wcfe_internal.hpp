@@ -118,7 +118,12 @@ void launch_node_terms(hipStream_t s, bool full, const View &v, const BndView &b
                        T *K, T *Kb, const int *row_ptr, const int *bcol, const int *diag_pos, double *G);
 // the end of a Newton step with one workgroup per cell: x += delta, the FP64
 // residual and its norm, the Newton test and the commit of a converged cell
-constexpr int FINISH_ELEMS = 12000;  // most elements of a cell (larger ones run the batch-wide kernels)
+// most elements of a cell: larger ones keep one workgroup longer than the
+// batch-wide launches take (us per Newton step, one workgroup per cell /
+// launches: one cell of 1000 elements 188 / 192, 1300 216 / 218, 1700 278 / 277,
+// 2700 328 / 317, 11500 727 / 646; 12 UL cells of 1300 295 / 308, of 3000
+// 497 / 492; FP64 alike)
+constexpr int FINISH_ELEMS = 1700;
 struct FinishArgs {
   double2 *X, *x, *fau;
   double *ea, *cC, *Ge, *G, *Rea, *MM, *sp_state, *sp_anchor;
