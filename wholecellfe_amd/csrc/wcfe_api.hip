@@ -913,7 +913,9 @@ void release_batch(wcfe_ctx *ctx) {
 }
 
 void free_old_K(wcfe_ctx *ctx) {
-  if (ctx->old_K) (void)hipFree(ctx->old_K);
+  if (!ctx->old_K) return;
+  (void)hipFree(ctx->old_K);
+  (void)hipDeviceSynchronize();  // as in release_batch
   ctx->old_K = nullptr;
   ctx->old_K_bytes = 0;
 }
