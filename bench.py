@@ -170,19 +170,20 @@ def measured_traffic(kernel, workload, pivoting):
 
 
 def lu_roofline(prof, fused, fp64=False, traffic=None):
-    """The band LU's dominant kernel.  fused (one launch per block step,
-    k_lu_step): achieved = useful 64^3 block products (trailing updates, L
+    """The band LU's dominant kernel.  fused (one launch per level of the
+    plans, k_lu_step_f32 / _f64): achieved = useful 64^3 block products (trailing updates, L
     block solves and the diagonal inverse, whose Gauss-Jordan elimination is
     64^3 multiply-adds) x 2 64^3 flop / summed launch time (HIP events at the
-    kernel's own start and end); the inverses that L items form again are not
+    kernel's own start and end); the inverses that items form again are not
     counted.  Otherwise (k_lu_gemm): trailing-update products x 2 64^3 flop."""
     g = prof["lu_gemm"]
     tile_flops = 2.0 * 64 ** 3
     flops = g["work"] * tile_flops
     achieved = flops / (g["ms"] * 1e-3) if g["ms"] > 0 else 0.0
     peak = MFMA_FP64_PEAK if fp64 else MFMA_FP32_PEAK
-    kernel = ("k_lu_step<%s> (fused band-LU block step: trailing update, Gauss-Jordan inverse of the diagonal block, "
-              "L block solves)" if fused else "k_lu_gemm<%s> (LU trailing update)") % ("double" if fp64 else "float")
+    kernel = ("k_lu_step_%s (fused band-LU block step: trailing update, Gauss-Jordan inverse of the diagonal block, "
+              "L block solves)" % ("f64" if fp64 else "f32") if fused else
+              "k_lu_gemm<%s> (LU trailing update)" % ("double" if fp64 else "float"))
     return {"kernel": kernel, "bound": "mfma", "achieved": achieved / 1e12, "peak": peak / 1e12, "unit": "TFLOP/s",
             "frac": achieved / peak, "traffic": traffic, "launches_per_step": g["launches"],
             "block_products_per_step": g["work"], "flops_per_block_product": tile_flops,
@@ -423,7 +424,7 @@ def main():
     log("LU schedule:", sched)
     dense = [c for c, L in zip(cells, layouts) if L["solver"] != 2]
     if prof["lu_gemm"]["launches"] > 0:
-        traffic = measured_traffic("k_lu_step" if sched["fused_step"] else "k_lu_gemm", a.workload, a.pivoting) \
+        traffic = measured_traffic("k_lu_step_f32" if sched["fused_step"] else "k_lu_gemm", a.workload, a.pivoting) \
             if a.workload == "batched256" and a.cells == 256 else None
         roofline = lu_roofline(prof, bool(sched["fused_step"]), traffic=traffic)
     else:

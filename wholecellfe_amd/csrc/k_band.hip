@@ -171,10 +171,10 @@ __device__ __forceinline__ long long blk_off(int bi, int bj, long long ld) {
 // Gauss-Jordan steps, each a chain of 16 pivots): every INV item inverts
 // block s from the same inputs, so no workgroup waits for another and only
 // the STORE item's inverse is kept; diagonal blocks of K stay unfactored,
-// nothing reads them afterwards.  Per launch the items are dealt out in one
-// of three forms (one INV item per column block; one for the pivot and its
-// whole column; the first column block with the pivot's), the same products
-// in the same order.
+// nothing reads them afterwards.  How many column
+// blocks an INV item takes and how many updated blocks another is chosen per
+// launch by estimated time (LuPlan::choose_deal); the same products in the same
+// order for every choice.
 // ---------------------------------------------------------------------------
 
 // forward substitution of the first solve (right-hand side -G in the band
