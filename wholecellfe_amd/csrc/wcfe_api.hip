@@ -61,6 +61,29 @@ template <class T> T *dupload(const std::vector<T> &h) {
   return d;
 }
 
+// Read-only tables in one device allocation and one copy (each of its own
+// takes a layout about 8 us).
+struct Tables {
+  template <class T> void add(T *&to, const std::vector<T> &v) {
+    const size_t off = (h.size() + 255) & ~(size_t)255;
+    h.resize(off + v.size() * sizeof(T));
+    if (!v.empty()) memcpy(h.data() + off, v.data(), v.size() * sizeof(T));
+    at.push_back({&to, off});
+  }
+  unsigned char *upload() {
+    unsigned char *d = dupload(h);
+    for (const auto &a : at) {
+      void *q = d + a.second;
+      memcpy(a.first, &q, sizeof q);
+    }
+    return d;
+  }
+
+ private:
+  std::vector<unsigned char> h;
+  std::vector<std::pair<void *, size_t>> at;  // the pointer to set, its table's offset
+};
+
 struct HostCell {
   int n_nodes = 0, n_tris = 0, law = 0, node_springs = 0, spring_law = 0, table_id = 0, kinetics = 0, n_spr = 0;
   int solver = 0;
@@ -505,7 +528,8 @@ struct LuPlan {
   // fuse 4: the whole factorization in one launch (k_lu_cell), every cell's
   // items in level order in one workgroup, longest cells first
   void build_fused(const std::vector<CellParams> &cp, const std::vector<const BandPlan *> &plans,
-                   const std::vector<int2> &base, int groups, int fuse, int f64, double slots, bool per_cell) {
+                   const std::vector<int2> &base, int groups, int fuse, int f64, double slots, bool per_cell,
+                   Tables &tables) {
     pivoting = 0;
     depth = 1;
     fused = true;
@@ -557,8 +581,8 @@ struct LuPlan {
       for (int q = g; q < n; q += G) mine.push_back(order[q]);
       grp.push_back(stages(mine));
     }
-    d_items = dupload(buf);
-    d_ranges = dupload(ranges);
+    tables.add(d_items, buf);
+    tables.add(d_ranges, ranges);
   }
 
   // host: the work lists stay there, for the caller to upload and own
@@ -721,6 +745,7 @@ struct Batch {
   std::vector<std::shared_ptr<BandPlan>> plans;
   std::vector<int> chain_top, chain_bottom;  // the measure of halved cells (wcfe_get_cell_layout)
   int nslot = 0;
+  unsigned char *tables = nullptr;  // holds rank, refs, fops, sops, slocs, saccs, swg, rwg and the fused schedule
   int *rank = nullptr;
   BlockRef *refs = nullptr;
   FwdOp *fops = nullptr;
@@ -766,9 +791,9 @@ struct Batch {
 
   void release() {
     void *ptrs[] = {X, x, fau, ea, cC, el_tri, el_cell, el_spr, sp_bary, sp_anchor, sp_state, sp_cell, sp_elem,
-                    sp_local, cp, cs, node_cell, adj_start, adj, Ge, g_start, g_col, g_bpos, g_cstart, g_ke, g_node, Ke64, G, r, delta, Rea, MM, K, Dinv, ysol, sync, ipiv, cells, celem, rwg, dirs, rargs,
+                    sp_local, cp, cs, node_cell, adj_start, adj, Ge, g_start, g_col, g_bpos, g_cstart, g_ke, g_node, Ke64, G, r, delta, Rea, MM, K, Dinv, ysol, sync, ipiv, cells, celem, dirs, rargs, tables,
                     replica, transitions, plan.d_prefix, row_ptr, bcol, diag_pos, el_bpos, csr_cells, chunks, Kb,
-                    cgvec, cg, partials, norm_part, norm_cnt, kpos, kinv, yfwd, ysw, slots, rank, refs, fops, sops, slocs, saccs, swg, plan.d_items, plan.d_ranges, plan.d_solve, rp, dp, bt_bidx, bt_node, bt_cst, crange, bt_cand, bt_frame, bt_g, bt_J, bt_area,
+                    cgvec, cg, partials, norm_part, norm_cnt, kpos, kinv, yfwd, ysw, slots, plan.d_solve, rp, dp, bt_bidx, bt_node, bt_cst, crange, bt_cand, bt_frame, bt_g, bt_J, bt_area,
                     bt_gd, bt_fext};
     for (void *p : ptrs)
       if (p) (void)hipFree(p);
@@ -1258,7 +1283,8 @@ void upload_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
     const std::shared_ptr<BandPlan> &P = b.plans[&p - b.cp_h.data()];
     for (int i = 0; i < p.nblk; ++i) rank.push_back(P ? P->rank[i] : i);
   }
-  b.rank = dupload(rank);
+  Tables tables;
+  tables.add(b.rank, rank);
   choose_refine(ctx, b, elem_size);
   HIPCHECK(hipMemcpy(b.cp, b.cp_h.data(), sizeof(CellParams) * b.ncell, hipMemcpyHostToDevice));
   const bool planned = std::any_of(b.plans.begin(), b.plans.end(), [](const std::shared_ptr<BandPlan> &p) { return !!p; });
@@ -1293,11 +1319,11 @@ void upload_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
     }
     base[c] = make_int2(it->second.ref, it->second.fop);
   }
-  b.refs = dupload(refs);
-  b.fops = dupload(fops);
+  tables.add(b.refs, refs);
+  tables.add(b.fops, fops);
   if (fused)
     b.plan.build_fused(b.cp_h, plans, base, b.lu_groups, ctx->opt.fused_step, elem_size == 8,
-                       step_slots(ctx, elem_size), !ctx->opt.batched);
+                       step_slots(ctx, elem_size), !ctx->opt.batched, tables);
   if (!fused || !b.solve_wg) {
     LuPlan lists;
     lists.build(b.cp_h, ctx->opt.pivoting, b.lu_groups, b.lu_depth);
@@ -1310,10 +1336,13 @@ void upload_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
       b.plan.d_solve = lists.d_prefix;
     }
   }
-  if (!b.solve_wg) return;
-  b.sops = dupload(ops);
-  b.slocs = dupload(locs);
-  b.saccs = dupload(accs);
+  if (!b.solve_wg) {
+    b.tables = tables.upload();
+    return;
+  }
+  tables.add(b.sops, ops);
+  tables.add(b.slocs, locs);
+  tables.add(b.saccs, accs);
   std::vector<SweepWG> wg;
   auto lists_of = [&](const std::vector<int> &cells) {
     Batch::SweepLists S;
@@ -1384,7 +1413,7 @@ void upload_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
   if (b.tail)
     for (int c : spread) one_wg(c);
   b.ntail = (int)rwg.size() - b.nrefine;
-  b.rwg = dupload(rwg);
+  tables.add(b.rwg, rwg);
   if (dirs > 0) {
     b.dirs = dalloc<double>(dirs);
     b.rargs = dupload(std::vector<RefineArgs>{refine_args(ctx, b)});
@@ -1415,7 +1444,8 @@ void upload_bands(wcfe_ctx *ctx, Batch &b, int elem_size) {
   b.sweeps_cell.clear();
   if (!ctx->opt.batched)
     for (int c = 0; c < b.ncell; ++c) b.sweeps_cell.push_back(lists_of({c}));
-  b.swg = dupload(wg);
+  tables.add(b.swg, wg);
+  b.tables = tables.upload();
 }
 
 void build_batch(wcfe_ctx *ctx, Batch &b, const std::vector<HostCell> &hc, int elem_size) {
