@@ -83,3 +83,16 @@ def test_band_part_singular(K, k_area, which, prec):
     assert sv[-1] < 1e-10 * sv[0]
     dx, st = step(d, prec, 4)
     check(d, dx, st)
+
+
+# max_refine holds where the sweeps converge: one sweep of an ordinary cell
+@pytest.mark.parametrize("prec", [W.PREC_MIXED, W.PREC_FP64])
+def test_one_sweep_stays_one(prec):
+    print("case one sweep", prec, flush=True)
+    d = area_cell(6, W.K_AREA_REF)
+    with W.Context(precision=prec, t0=d["time"], dt=d["dt"], lin_rtol=1e-14 if prec else 1e-12, max_refine=1) as c:
+        c.add_cell(X=d["X"], x=d["x"], tris=d["tris"], law=d["law"], mu=d["mu"], thick=d["thick"], ea=d["ea"],
+                   node_springs=1, cC=d["cC"], fau=d["fau0"], rho_max=d["rho_max"], spring_law=0, k_lin=d["k_lin"],
+                   k_bend=d["k_bend"], k_area=d["k_area"], area_0=d["area_0"], drag=d["drag"])
+        c.finalize()
+        assert c.newton_step(check=False)["max_refine_used"] == 1

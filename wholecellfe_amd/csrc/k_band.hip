@@ -744,7 +744,8 @@ __device__ __attribute__((noinline)) bool refine_direction(const RefineArgs *arg
 // B can be singular where K is not (the area off area_0 by a pressure that the
 // cell's stiffness balances); then y and z are large, almost cancel, and the
 // sweeps stall.  From the first sweep that leaves more than REFINE_POOR of the
-// residual, or if max_refine end above lin_rtol, the solve is mixed block
+// residual, or a last one (of max_refine) that leaves more than roundoff
+// explains (1e-2, FP64 1e-4), the solve is mixed block
 // elimination (Govaerts and Pryce 1990; its solve with the transpose taken as
 // z / k, which the mostly symmetric B allows): a first guess of the rank one's
 // part leaves the right-hand side before B^-1 is applied.  The updates then are
@@ -806,7 +807,7 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_band_refine(const CellParams 
   };
   auto step = [&](int i, double t) { return t != 0.0 ? ra.inc[i] - ra.z[i] * t : ra.inc[i]; };
   int nd = -1;  // cells with smw: directions so far (refine_direction); -1: plain refinement
-  const double bnorm = cs[c].bnorm;
+  const double bnorm = cs[c].bnorm, slow = sizeof(T) == 4 ? 1e-2 : 1e-4;
   double last = bnorm, y1 = 0.0;  // y1: the first guess of g . d
   int most = ra.max_refine;
   for (int it = smw ? ra.it0 - 1 : ra.it0; it < most; ++it) {
@@ -854,7 +855,7 @@ __global__ __launch_bounds__(SWEEP_THREADS) void k_band_refine(const CellParams 
       nrm = sqrt(residual());
       if (!smw || nd >= 0 || undone) break;
       const bool poor = !(nrm <= ra.lin_rtol * bnorm) && !(nrm <= REFINE_FLOOR * bnorm) &&
-                        (!(nrm <= REFINE_POOR * last) || it + 1 == ra.max_refine);
+                        (!(nrm <= REFINE_POOR * last) || (it + 1 == ra.max_refine && !(nrm <= slow * last)));
       if (poor) most = ra.max_refine + REFINE_MORE;
       if (poor && !(nrm <= last)) {  // worse than before the sweep: without it
         for (int i = 2 * n0 + threadIdx.x; i < 2 * n1; i += SWEEP_THREADS) {
