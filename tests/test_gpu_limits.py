@@ -21,6 +21,15 @@ def free_bytes():
     return free.value
 
 
+def most_free(seconds=0.5):
+    """The runtime gives memory back some time after the call that frees it."""
+    end, most = time.monotonic() + seconds, 0
+    while time.monotonic() < end:
+        most = max(most, free_bytes())
+        time.sleep(0.01)
+    return most
+
+
 # a checkpoint holds at most 2047 cells, and the LU's work lists 11 bits of them
 def test_batches_above_2047_cells_are_refused():
     X, T, _ = mesh.disk_rings(1, 10.0)
@@ -50,7 +59,7 @@ def test_large_dense_solve_takes_what_it_needs():
     need = 8 * (n * n + 6016 * 6016 + 128 * 6016)
     with W.Context(precision=W.PREC_FP64) as c:
         solve(c, 200, 1)  # code and streams are loaded
-        before, least, stop = free_bytes(), [1 << 62], threading.Event()
+        before, least, stop = most_free(), [1 << 62], threading.Event()
 
         def watch():
             while not stop.is_set():
@@ -88,15 +97,6 @@ def test_two_threads_in_one_context():
         for t in ts:
             t.join()
     assert not bad
-
-
-def most_free(seconds=0.5):
-    """The runtime gives memory back some time after the call that frees it."""
-    end, most = time.monotonic() + seconds, 0
-    while time.monotonic() < end:
-        most = max(most, free_bytes())
-        time.sleep(0.01)
-    return most
 
 
 # two concurrent cell groups: the captured step runs on streams of its own
